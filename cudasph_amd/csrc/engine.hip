@@ -493,10 +493,7 @@ void Engine<T>::solve() {
   {
     TimerScope ts(timers_, "solve_range", s_);
     WalkParams wp = walk_params();
-    if (solve_cache_ > 0 || (solve_cache_ < 0 && solve_cache_pays(nd_))) {
-      if (solve_rec_.n < (size_t)kSolveCacheK * nd_) solve_rec_.alloc((size_t)kSolveCacheK * nd_);
-      wp.solve_cache = solve_rec_.p;
-    }
+    wp.solve_cache = solve_cache_ != 0;
     launch_solve_range<T>(pos_, n_ngb_, hash_, tree_, nd_, wp, s_);
   }
   if (adj_mode_ == kAdjRecord) {

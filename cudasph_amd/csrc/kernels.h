@@ -16,23 +16,22 @@ struct WalkParams {
   // also skips a child whose subtree box lies beyond the range.  The same
   // neighbours in the same order; fewer nodes visited (the walk length)
   const F4* boxes = nullptr;
-  // h-solve candidate cache, or null: kSolveCacheK records of V4<T> per
-  // lane, record k of lane t at k * n_dev + t (launch_solve_range)
-  void* solve_cache = nullptr;
+  // the h-solve keeps the distances of its first walk and filters them at its
+  // later ranges (0: it walks at every range); the same bits either way
+  int solve_cache = 1;
 };
-constexpr int kSolveCacheK = 128;
 
 struct EosConst;  // sph_math.h
 
-// ---- sph_passes.hip ----
+// ---- walks.hip ----
 template <class T>
 void launch_solve_range(V4<T>* pos, int* n_ngb, const KV* hash, const V4<T>* tree, int n_dev,
                         const WalkParams& wp, hipStream_t s);
-bool solve_cache_pays(int n_dev);
 template <class T>
 void launch_find_ngb(const V4<T>* pos, const V4<T>* tree, KV* hash, const int* offset, const int* cap_count,
                      int* count_out, int* list, int* flags, int n_dev, const WalkParams& wp, int clamp,
                      hipStream_t s);
+// ---- sph_passes.hip ----
 // plain and FP64 forms
 template <class T>
 void launch_density(const V4<T>* pos, const V4<T>* vel, V4<T>* hydro, V4<T>* dots, const KV* hash,

@@ -218,8 +218,9 @@ long   sph_engine_get(void* e, const char* name, void* host, long max_bytes);
  * at 65 536 particles, leaving the SPH passes beside it room on every CU;
  * the sums' grouping follows it; also the FP64 form's forward gravity;
  * read-only grav_parts_auto: the count the default takes at this size).
- * solve_cache (the h-solve's candidate cache: 1 on, 0 off, -1, the default:
- * on below 65 536 particles; the same bits either way).
+ * solve_cache (below 2^19 particles the h-solve keeps the distances of its
+ * first walk for its later ranges: 1 and -1, the default, on, 0 off; the same
+ * bits either way).
  * Plain-form Plummer gravity, the same bits either way: grav_sums (1: each
  * particle's four sums in four wavefronts, 2: in two, 0: in one lane; -1,
  * the default: four wavefronts up to 16 384 particles, two up to 65 536).
