@@ -40,15 +40,52 @@ __device__ __forceinline__ void dr_sub(DR& x, float y) {
 }
 __device__ __forceinline__ void dr_add(DR& x, float y) { dr_sub(x, -y); }
 
+// A dreal sum with its last step's low word still to be formed: hi, and
+// lo = t2 - (hi - t1).  sub is dr_sub.  The fast ones are dr_sub where
+// |hi| >= |y|: the rounding error of hi - y is then exact in two operations
+// (Dekker's fast two-sum) instead of five, so they return dr_sub's bits with
+// 7 operations instead of 10.
+struct Chain {
+  float hi = 0.f, t1 = 0.f, t2 = 0.f;
+  __device__ __forceinline__ void sub(float y) {
+    DR v{hi, t2 - (hi - t1)};
+    const float d1 = v.hi - y;
+    const float e = d1 - v.hi;
+    const float d2 = ((-y - e) + (v.hi - (d1 - e))) + v.lo;
+    hi = d1 + d2;
+    t1 = d1;
+    t2 = d2;
+  }
+  __device__ __forceinline__ void sub_fast(float y) {
+    const float lo = t2 - (hi - t1), d1 = hi - y;
+    t2 = ((hi - d1) - y) + lo;
+    hi = d1 + t2;
+    t1 = d1;
+  }
+  // ... for a wavefront that has only this chain to issue: a step depends on
+  // the one before through 5 operations, and the two that form the previous
+  // low word go between them (left to itself the compiler puts all 7 in a row)
+  __device__ __forceinline__ void sub_fast_alone(float y) {
+    float n1, q, d;
+    asm("v_sub_f32 %[n1], %[hi], %[y]\n\t"     // n1 = hi - y
+        "v_sub_f32 %[q], %[hi], %[t1]\n\t"
+        "v_sub_f32 %[d], %[hi], %[n1]\n\t"
+        "v_sub_f32 %[q], %[t2], %[q]\n\t"      // q = the low word
+        "v_sub_f32 %[d], %[d], %[y]\n\t"       // d = the rounding error
+        "v_add_f32 %[t2], %[d], %[q]\n\t"
+        "v_add_f32 %[hi], %[n1], %[t2]"
+        : [n1] "=&v"(n1), [q] "=&v"(q), [d] "=&v"(d), [hi] "+&v"(hi), [t2] "+&v"(t2)
+        : [t1] "v"(t1), [y] "v"(y));
+    t1 = n1;
+  }
+};
+// the four sums of one particle
+struct Chains4 {
+  Chain a0, a1, a2, a3;
+};
+
 template <class T, int ACC>
 struct GAcc;
-template <>
-struct GAcc<float, 0> {                      // per-pair dreal
-  DR v{0.f, 0.f};
-  __device__ __forceinline__ void sub(float y) { dr_sub(v, y); }
-  __device__ __forceinline__ void tile_end() {}
-  __device__ __forceinline__ float get() const { return v.hi; }
-};
 template <>
 struct GAcc<float, 1> {                      // blocked compensation
   DR v{0.f, 0.f};
@@ -90,19 +127,30 @@ __device__ __forceinline__ double inv_sqrt(double x) {
   return y * (1.5 - 0.5 * x * y * y);
 }
 
+// sum C of an accumulator set
+template <int C, class T, int ACC>
+__device__ __forceinline__ GAcc<T, ACC>& acc(GAcc<T, ACC> (&a)[4]) { return a[C]; }
+template <int C, class S>
+__device__ __forceinline__ auto& acc(S& a) {
+  if constexpr (C == 0) return a.a0;
+  else if constexpr (C == 1) return a.a1;
+  else if constexpr (C == 2) return a.a2;
+  else return a.a3;
+}
+
 // spline-softened pair (sph_grav_kernel.cu:14-111); pj = (x,y,z,m),
 // vi.w / vj.w = range^2
 template <class T, bool EXACT, class A>
-__device__ __forceinline__ void pair_spline(A* a, T rx, T ry, T rz, T ri2, T mj, T rj2) {
+__device__ __forceinline__ void pair_spline(A&& a, T rx, T ry, T rz, T ri2, T mj, T rj2) {
   const T d2 = rx * rx + ry * ry + rz * rz;
   const T inv = inv_sqrt<EXACT>(d2);
   const T inv3 = inv * inv * inv;
   T s3 = mj * inv3;
   if (d2 >= ri2 && d2 >= rj2) {
-    a[0].sub(rx * s3);
-    a[1].sub(ry * s3);
-    a[2].sub(rz * s3);
-    a[3].sub(mj * inv);
+    acc<0>(a).sub(rx * s3);
+    acc<1>(a).sub(ry * s3);
+    acc<2>(a).sub(rz * s3);
+    acc<3>(a).sub(mj * inv);
     return;
   }
   s3 = T(0.5f) * s3;
@@ -118,15 +166,15 @@ __device__ __forceinline__ void pair_spline(A* a, T rx, T ry, T rz, T ri2, T mj,
     }
     gacc = T(0.5 * (double)mj * (double)gacc / (double)(ri2 * h));
     gpot = -gpot;
-    a[0].sub(rx * gacc);
-    a[1].sub(ry * gacc);
-    a[2].sub(rz * gacc);
-    a[3].sub(mj * gpot / h);
+    acc<0>(a).sub(rx * gacc);
+    acc<1>(a).sub(ry * gacc);
+    acc<2>(a).sub(rz * gacc);
+    acc<3>(a).sub(mj * gpot / h);
   } else {
-    a[0].sub(rx * s3);
-    a[1].sub(ry * s3);
-    a[2].sub(rz * s3);
-    a[3].sub(mj * inv);
+    acc<0>(a).sub(rx * s3);
+    acc<1>(a).sub(ry * s3);
+    acc<2>(a).sub(rz * s3);
+    acc<3>(a).sub(mj * inv);
   }
   if (d2 < rj2) {
     const T u2 = d2 / rj2, h = dsqrt(rj2), u = dsqrt(u2), u3 = u2 * u;
@@ -134,27 +182,27 @@ __device__ __forceinline__ void pair_spline(A* a, T rx, T ry, T rz, T ri2, T mj,
     if (u < T(0.5)) gacc = T(32.0 / 3.0) + u2 * (T(32) * u - T(38.4));
     else gacc = T(64.0 / 3.0) - T(48) * u + T(38.4) * u2 - T(32.0 / 3.0) * u3 - T(1.0 / 15.0) / u3;
     gacc = T(0.5 * (double)mj * (double)gacc / (double)(rj2 * h));
-    a[0].sub(rx * gacc);
-    a[1].sub(ry * gacc);
-    a[2].sub(rz * gacc);
+    acc<0>(a).sub(rx * gacc);
+    acc<1>(a).sub(ry * gacc);
+    acc<2>(a).sub(rz * gacc);
   } else {
-    a[0].sub(rx * s3);
-    a[1].sub(ry * s3);
-    a[2].sub(rz * s3);
+    acc<0>(a).sub(rx * s3);
+    acc<1>(a).sub(ry * s3);
+    acc<2>(a).sub(rz * s3);
   }
 }
 
 // Plummer pair: a -= m r (r^2+eps^2)^-3/2, phi -= m (r^2+eps^2)^-1/2
 template <class T, bool EXACT, class A>
-__device__ __forceinline__ void pair_plummer(A* a, T rx, T ry, T rz, T mj, T eps2) {
+__device__ __forceinline__ void pair_plummer(A&& a, T rx, T ry, T rz, T mj, T eps2) {
   const T d2 = rx * rx + ry * ry + rz * rz + eps2;
   const T inv = inv_sqrt<EXACT>(d2);
   const T inv3 = inv * inv * inv;
   const T s3 = mj * inv3;
-  a[0].sub(rx * s3);
-  a[1].sub(ry * s3);
-  a[2].sub(rz * s3);
-  a[3].sub(mj * inv);
+  acc<0>(a).sub(rx * s3);
+  acc<1>(a).sub(ry * s3);
+  acc<2>(a).sub(rz * s3);
+  acc<3>(a).sub(mj * inv);
 }
 
 constexpr int kGravBlock = 256;
@@ -181,8 +229,8 @@ __device__ __forceinline__ int stage_tile(R* __restrict__ s, const R* __restrict
   return cnt;
 }
 
-// reference-layout kernel (plain and FP64 forms): gpos = (x,y,z,m),
-// gvel.w = range^2
+// reference-layout kernel of the FP64 form (spline softening, and Plummer's
+// reference arithmetic): gpos = (x,y,z,m), gvel.w = range^2
 template <class T, int SOFT, int ACC, bool EXACT>
 __global__ __launch_bounds__(kGravBlock) void k_gravity(const V4<T>* __restrict__ gpos,
                                                         const V4<T>* __restrict__ gvel, V4<T>* __restrict__ out,
@@ -208,60 +256,240 @@ __global__ __launch_bounds__(kGravBlock) void k_gravity(const V4<T>* __restrict_
     };
     // j in ascending order (the reference's summation order).  The loop is
     // left rolled: unrolling it measured slower for these longer pair bodies
-    // (dreal accumulation, FP64)
     for (int j = 0; j < cnt; ++j) body(j);
   }
   if (i < n_i) out[i] = {a[0].get(), a[1].get(), a[2].get(), a[3].get()};
 }
 
-// Plain form, Plummer softening (the presets' softening).  A particle's four
-// per-pair dreal sums (ax, ay, az, potential) are serial chains from record
-// to record, and the issue is in order, so both kernels below are
-// software-pipelined: the terms of the next G records are computed in the
-// same block as the chain over the current G, which gives the issue
-// independent work between the chain's dependent steps.  The terms enter the
-// chains in ascending j and each term is pair_plummer's expression, so the
-// sums are pair_plummer's bits.
-template <int C, bool EXACT>
-__device__ __forceinline__ float plummer_term(const F4& pj, const F4& pi, float eps2) {
+// ---------------------------------------------------------------------------
+// Plain form: the reference's per-pair dreal sums.  A particle's four sums
+// (ax, ay, az, potential) are serial chains from record to record, in
+// ascending j, and each term is pair_plummer's (pair_spline's) expression, so
+// the results are the reference's bits.
+//
+// FP32 VALU issue bounds it: 17 operations and an rsq for a pair's terms, and
+// 4 two-sums of 10 operations; with few particles the latency of the chains
+// (a dependent operation takes about 9 cycles in a lone wavefront, and a SIMD
+// issues at its full rate only from 4 wavefronts on).
+//
+// k_gravity_chains (up to kChainsMaxN particles): a block takes 64 particles.
+// Its first four wavefronts keep one sum each; the other four compute the
+// terms, each of a quarter of a batch of records, and hand them over through
+// LDS, double buffered, with one barrier per batch.  So a pair's distance
+// and rsq are computed once, and every SIMD has an independent stream of
+// terms beside its dependent chain.
+//  * A chain takes its terms 8 at a time.  The fast two-sum is right where the
+//    sum is at least as large as the term; for 8 terms that holds if |sum| >= 9
+//    times the largest (7 of them lower |sum| by 7 times that at most).  Sums
+//    over many records exceed their next terms by far: 87 % of the groups take
+//    it at 16 384 particles, 98 % at 131 072.  The wavefront decides by one ballot,
+//    and a group that fails takes dr_sub.
+//  * Terms past the last record are zero: a two-sum with zero changes nothing.
+//  * Spline softening: a record beyond both ranges has the Newtonian term.
+//    One inside them has a term for each range; 4 records of which some lane
+//    has one inside carry the second terms (zero for the others) in a buffer
+//    of their own.
+// Measured alone, one lane per particle (four wavefronts with a sum each up to
+// 16 384, two with two each up to 65 536) -> this kernel, ms: Plummer 1 000
+// particles 0.057 -> 0.044, 16 384: 0.88 -> 0.51, 32 768: 2.48 -> 1.42, 65 536:
+// 5.9 -> 4.6, 100 003: 11.4 -> 11.3, 131 072: 15.0 -> 16.1; spline 16 384: 3.9 ->
+// 0.82, 65 536: 13.9 -> 6.8, 100 003: 20.9 -> 17.0.  Plain Plummer step, beside
+// the SPH passes, one lane / this kernel: 65 536: 7.6 / 5.3, 81 920: 10.1 / 8.6,
+// 90 112: 11.0 / 10.2, 100 003: 12.1 / 12.5, 131 072: 15.7 / 16.3.  (32 records per batch: 16 384 particles 0.49, but 1 045
+// against 914 ms at 2^20, where fewer blocks fit; two sums per wavefront:
+// 16 384: 0.79, 65 536: 5.3.)
+constexpr int kChainParticles = 64;   // particles per block
+
+// the terms of one pair: y[0..2], y[3] and, with the spline softening, the
+// second acceleration terms z[0..2]
+struct PairTerms {
+  float y[4], z[3];
+};
+// pair_spline's accumulator that takes its terms apart: the first sub of a
+// component is its first term
+struct TermSink {
+  float first = 0.f, second = 0.f;
+  bool have = false;
+  __device__ __forceinline__ void sub(float y) {
+    if (have) second = y;
+    else first = y;
+    have = true;
+  }
+};
+struct TermSinks {
+  TermSink a0, a1, a2, a3;
+};
+
+template <int SOFT, bool EXACT>
+__device__ __forceinline__ bool pair_terms(PairTerms& t, const F4& pj, float rj2, const F4& pi, float ri2,
+                                           float eps2) {
   const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
-  const float d2 = rx * rx + ry * ry + rz * rz + eps2;
+  float d2 = rx * rx + ry * ry + rz * rz;
+  if constexpr (SOFT == 1) d2 = d2 + eps2;
   const float inv = inv_sqrt<EXACT>(d2);
-  if constexpr (C == 3) {
-    return pj.w * inv;
-  } else {
-    const float s3 = pj.w * (inv * inv * inv);
-    return (C == 0 ? rx : C == 1 ? ry : rz) * s3;
-  }
+  const float s3 = pj.w * (inv * inv * inv);
+  t.y[0] = rx * s3;
+  t.y[1] = ry * s3;
+  t.y[2] = rz * s3;
+  t.y[3] = pj.w * inv;
+  return SOFT == 0 && !(d2 >= ri2 && d2 >= rj2);
+}
+template <bool EXACT>
+__device__ __forceinline__ void pair_terms_near(PairTerms& t, const F4& pj, float rj2, const F4& pi, float ri2) {
+  TermSinks k;
+  pair_spline<float, EXACT>(k, pi.x - pj.x, pi.y - pj.y, pi.z - pj.z, ri2, pj.w, rj2);
+  t.y[0] = k.a0.first;
+  t.y[1] = k.a1.first;
+  t.y[2] = k.a2.first;
+  t.y[3] = k.a3.first;
+  t.z[0] = k.a0.second;
+  t.z[1] = k.a1.second;
+  t.z[2] = k.a2.second;
 }
 
-template <int G, class Term, class Chain>
-__device__ __forceinline__ void pipelined(int cnt, Term term, Chain chain) {
-  using Y = decltype(term(0));
-  int j = 0;
-  if (cnt >= G) {
-    Y y[G];
+__device__ __forceinline__ float max_abs8(const float* y) {
+  const float m = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fabsf(y[2]));
+  const float n = fmaxf(fmaxf(fabsf(y[3]), fabsf(y[4])), fabsf(y[5]));
+  return fmaxf(fmaxf(m, n), fmaxf(fabsf(y[6]), fabsf(y[7])));
+}
+// 4 records (wavefront-uniform: scalar loads)
+template <int SOFT>
+struct Quad {
+  F4 p[4];
+  float r2[4];
+  __device__ __forceinline__ void load(const F4* __restrict__ gpos, const F4* __restrict__ gvel, int j0, int n_j) {
 #pragma unroll
-    for (int k = 0; k < G; ++k) y[k] = term(k);
-    for (j = G; j + G <= cnt; j += G) {
-      Y yn[G];
-#pragma unroll
-      for (int k = 0; k < G; ++k) yn[k] = term(j + k);
-#pragma unroll
-      for (int k = 0; k < G; ++k) chain(y[k]);
-#pragma unroll
-      for (int k = 0; k < G; ++k) y[k] = yn[k];
+    for (int k = 0; k < 4; ++k) {
+      const int j = min(j0 + k, n_j - 1);
+      p[k] = gpos[j];
+      r2[k] = SOFT == 0 ? gvel[j].w : 0.f;
     }
-#pragma unroll
-    for (int k = 0; k < G; ++k) chain(y[k]);   // records j - G .. j - 1
   }
-  for (; j < cnt; ++j) chain(term(j));
+};
+
+// the terms of a quad at records j0 .. j0 + 3 for the lane's particle; returns
+// whether some lane needs the second terms
+template <int SOFT, bool EXACT>
+__device__ __forceinline__ bool quad_terms(PairTerms (&t)[4], const Quad<SOFT>& r, int j0, int n_j, const F4& pi,
+                                           float ri2, float eps2) {
+  bool near = false;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) near |= pair_terms<SOFT, EXACT>(t[k], r.p[k], r.r2[k], pi, ri2, eps2);
+  bool any = false;
+  if constexpr (SOFT == 0) {
+    any = __any(near);
+    if (any) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) pair_terms_near<EXACT>(t[k], r.p[k], r.r2[k], pi, ri2);
+    }
+  }
+  if (j0 + 4 > n_j) {   // past the last record
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j0 + k >= n_j) {
+        t[k].y[0] = t[k].y[1] = t[k].y[2] = t[k].y[3] = 0.f;
+        t[k].z[0] = t[k].z[1] = t[k].z[2] = 0.f;
+      }
+  }
+  return any;
 }
 
-// One lane per particle, its four chains side by side, one record ahead
-// (measured against the same loop without the pipelining: 8.66 -> 7.38 ms at
-// N = 65 536, 71.5 -> 66.9 ms at 262 144, 1037 -> 1012 ms at 2^20; two
-// records ahead gained less).
+constexpr int kChainBlock = 512;
+template <int SOFT, bool EXACT>
+__global__ __launch_bounds__(kChainBlock) void k_gravity_chains(const F4* __restrict__ gpos,
+                                                             const F4* __restrict__ gvel, F4* __restrict__ out,
+                                                             int n_i, int n_j, float eps2) {
+  constexpr int B = 16, Q = B / 4;   // records and quads per batch, one quad per wavefront of terms
+  __shared__ float4 s_y[2][4][Q][64];
+  __shared__ float4 s_z[SOFT == 0 ? 2 : 1][SOFT == 0 ? 3 : 1][SOFT == 0 ? Q : 1][SOFT == 0 ? 64 : 1];
+  __shared__ int s_near[2][Q];
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = blockIdx.x * kChainParticles + lane;
+  const int ii = i < n_i ? i : n_i - 1;
+  const int batches = (n_j + B - 1) / B;
+  if (w >= 4) {   // terms
+    const F4 pi = gpos[ii];
+    const float ri2 = SOFT == 0 ? gvel[ii].w : 0.f;
+    const int quad = w - 4;
+    Quad<SOFT> r;
+    r.load(gpos, gvel, quad * 4, n_j);
+    for (int b = 0; b < batches; ++b) {
+      Quad<SOFT> next;   // (past the last batch: the last record once more, unused)
+      next.load(gpos, gvel, (b + 1) * B + quad * 4, n_j);
+      PairTerms t[4];
+      const bool any = quad_terms<SOFT, EXACT>(t, r, b * B + quad * 4, n_j, pi, ri2, eps2);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        s_y[b & 1][c][quad][lane] = make_float4(t[0].y[c], t[1].y[c], t[2].y[c], t[3].y[c]);
+      if constexpr (SOFT == 0) {
+        if (any) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            s_z[b & 1][c][quad][lane] = make_float4(t[0].z[c], t[1].z[c], t[2].z[c], t[3].z[c]);
+        }
+        if (lane == 0) s_near[b & 1][quad] = any;
+      }
+      r = next;
+      __syncthreads();
+    }
+  } else {   // chains: batch b while the next one's terms are computed
+    Chain a;
+    for (int b = 0; b < batches; ++b) {
+      __syncthreads();
+      float y[B];
+#pragma unroll
+      for (int k = 0; k < Q; ++k) {
+        const float4 v = s_y[b & 1][w][k][lane];
+        y[4 * k] = v.x, y[4 * k + 1] = v.y, y[4 * k + 2] = v.z, y[4 * k + 3] = v.w;
+      }
+      unsigned second = 0;   // quads with second terms (the potential has none)
+      if (SOFT == 0 && w < 3) {
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+          second |= (unsigned)__builtin_amdgcn_readfirstlane(s_near[b & 1][k]) << k;
+      }
+      float m = max_abs8(y);
+      bool fast = __all(fabsf(a.hi) >= 9.f * m);
+#pragma unroll
+      for (int g = 0; g < B; g += 8) {
+        const float mn = g + 8 < B ? max_abs8(y + g + 8) : 0.f;
+        if (SOFT == 0 && ((second >> (g / 4)) & 3u)) {
+#pragma unroll
+          for (int h = g / 4; h < g / 4 + 2; ++h) {
+            const float4 e = (second >> h) & 1u ? s_z[b & 1][w % 3][h][lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+            a.sub(y[4 * h]);
+            a.sub(e.x);
+            a.sub(y[4 * h + 1]);
+            a.sub(e.y);
+            a.sub(y[4 * h + 2]);
+            a.sub(e.z);
+            a.sub(y[4 * h + 3]);
+            a.sub(e.w);
+          }
+          fast = __all(fabsf(a.hi) >= 9.f * mn);
+        } else {
+          // the next 8 are judged by the sum before these 8, which lower it
+          // by 8 times their largest at most: the verdict is there in time
+          const bool next = __all(fabsf(a.hi) >= 9.5f * (m + mn));
+          if (fast) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) a.sub_fast_alone(y[g + k]);
+          } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) a.sub(y[g + k]);
+          }
+          fast = next;
+        }
+        m = mn;
+      }
+    }
+    if (i < n_i) reinterpret_cast<float*>(out + i)[w] = a.hi;
+  }
+}
+
+// Many particles: a lane keeps all four chains of its particle, 256 particles
+// per block, the records in LDS tiles, software-pipelined (the next record's
+// terms are computed in the same block as the current one's chain steps).
 template <bool EXACT>
 __global__ __launch_bounds__(kGravBlock) void k_gravity_lane(const F4* __restrict__ gpos, F4* __restrict__ out,
                                                              int n_i, int n_j, float eps2) {
@@ -271,103 +499,135 @@ __global__ __launch_bounds__(kGravBlock) void k_gravity_lane(const F4* __restric
   DR a0{0.f, 0.f}, a1{0.f, 0.f}, a2{0.f, 0.f}, a3{0.f, 0.f};
   for (int t0 = 0; t0 < n_j; t0 += kJTile) {
     const int cnt = stage_tile(s_pos, gpos, t0, n_j);
-    pipelined<1>(
-        cnt,
-        [&](int j) {
-          const F4 pj = s_pos[j];
-          return F4{plummer_term<0, EXACT>(pj, pi, eps2), plummer_term<1, EXACT>(pj, pi, eps2),
-                    plummer_term<2, EXACT>(pj, pi, eps2), plummer_term<3, EXACT>(pj, pi, eps2)};
-        },
-        [&](const F4& y) {
-          dr_sub(a0, y.x);
-          dr_sub(a1, y.y);
-          dr_sub(a2, y.z);
-          dr_sub(a3, y.w);
-        });
+    auto terms = [&](int j) {
+      PairTerms t;
+      pair_terms<1, EXACT>(t, s_pos[j], 0.f, pi, 0.f, eps2);
+      return F4{t.y[0], t.y[1], t.y[2], t.y[3]};
+    };
+    auto chain = [&](const F4& y) {
+      dr_sub(a0, y.x);
+      dr_sub(a1, y.y);
+      dr_sub(a2, y.z);
+      dr_sub(a3, y.w);
+    };
+    F4 y = terms(0);
+    for (int j = 1; j < cnt; ++j) {
+      const F4 yn = terms(j);
+      chain(y);
+      y = yn;
+    }
+    chain(y);
   }
   if (i < n_i) out[i] = {a0.hi, a1.hi, a2.hi, a3.hi};
 }
 
-// Few particles: one wavefront per sum.  A block takes 64 particles and its
-// wavefront c keeps sum c of each, repeating the pair's distance and rsq and
-// running one two-sum per pair instead of four (~23 VALU + rsq per pair and
-// lane against ~58 + rsq), on four times as many wavefronts: at N = 16 384
-// the one-lane kernel has a wavefront for 256 of the GPU's 1024 SIMDs, this
-// one fills all of them, 8 records ahead (16 384: 2.19 -> 0.89 ms).
-constexpr int kSumParticles = kGravBlock / 4;   // particles per block of k_gravity_sums
+// The same with the shortened two-sum, the records judged 16 at a time by a
+// bound of their terms that needs only the group's place: M / d^2 for an
+// acceleration and M / d for the potential, M the group's largest mass and d
+// its distance (from a record of the group, less the group's radius about it).
+// A group that fails, or one that comes within the spline's ranges, takes its
+// records one by one.  Measured, Plummer, this kernel against k_gravity_lane:
+// 131 072 particles 18.9 / 15.0 ms, 262 144: 64.3 / 58.9 (2 and 4 wavefronts per
+// SIMD, where the longer block issues worse), 2^20: 848 / 946.  Spline, against
+// the one-record loop it replaces: 100 003: 15.5 / 20.9, 131 072: 19.4 / 26.9,
+// 262 144: 65.6 / 85.2.
+constexpr int kLaneGroup = 16;
+struct LaneGroup {
+  float x, y, z, radius;
+  float m, r2;   // 17.5 times the largest |mass|; the largest range^2
+};
 
-template <int C, bool EXACT>
-__device__ __forceinline__ void plummer_sum(DR& acc, const F4* __restrict__ s_pos, int cnt, const F4& pi,
-                                            float eps2) {
-  pipelined<8>(
-      cnt, [&](int j) { return plummer_term<C, EXACT>(s_pos[j], pi, eps2); }, [&](float y) { dr_sub(acc, y); });
-}
-
-template <bool EXACT>
-__global__ __launch_bounds__(kGravBlock) void k_gravity_sums(const F4* __restrict__ gpos, F4* __restrict__ out,
-                                                             int n_i, int n_j, float eps2) {
-  __shared__ F4 s_pos[kJTile];
-  const int c = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);   // the wavefront's sum
-  const int i = blockIdx.x * kSumParticles + (threadIdx.x & 63);
-  const F4 pi = gpos[i < n_i ? i : n_i - 1];
-  DR acc{0.f, 0.f};
+template <int SOFT, bool EXACT>
+__global__ __launch_bounds__(kGravBlock) void k_gravity_lane_fast(const F4* __restrict__ gpos,
+                                                                  const F4* __restrict__ gvel, F4* __restrict__ out,
+                                                                  int n_i, int n_j, float eps2) {
+  __shared__ F4 s_pos[kJTile + 1];   // (the last one is read ahead, unused)
+  __shared__ float s_r2[SOFT == 0 ? kJTile : 1];
+  __shared__ LaneGroup s_group[kJTile / kLaneGroup];
+  const int i = blockIdx.x * kGravBlock + threadIdx.x;
+  const int ii = i < n_i ? i : n_i - 1;
+  const F4 pi = gpos[ii];
+  const float ri2 = SOFT == 0 ? gvel[ii].w : 0.f;
+  Chains4 a;
   for (int t0 = 0; t0 < n_j; t0 += kJTile) {
-    const int cnt = stage_tile(s_pos, gpos, t0, n_j);
-    switch (c) {
-      case 0: plummer_sum<0, EXACT>(acc, s_pos, cnt, pi, eps2); break;
-      case 1: plummer_sum<1, EXACT>(acc, s_pos, cnt, pi, eps2); break;
-      case 2: plummer_sum<2, EXACT>(acc, s_pos, cnt, pi, eps2); break;
-      default: plummer_sum<3, EXACT>(acc, s_pos, cnt, pi, eps2); break;
+    const int cnt = min(kJTile, n_j - t0);
+    __syncthreads();
+    for (int q = threadIdx.x; q < kJTile; q += kGravBlock) {
+      const int j = min(t0 + q, n_j - 1);   // (past the end: the last record again, outside every whole group)
+      const F4 p = gpos[j];
+      s_pos[q] = p;
+      float r2 = 0.f;
+      if constexpr (SOFT == 0) {
+        r2 = gvel[j].w;
+        s_r2[q] = r2;
+      }
+      const float cx = __shfl(p.x, kLaneGroup / 2, kLaneGroup), cy = __shfl(p.y, kLaneGroup / 2, kLaneGroup),
+                  cz = __shfl(p.z, kLaneGroup / 2, kLaneGroup);
+      const float dx = p.x - cx, dy = p.y - cy, dz = p.z - cz;
+      float d2 = dx * dx + dy * dy + dz * dz, m = fabsf(p.w);
+      for (int o = 1; o < kLaneGroup; o <<= 1) {
+        d2 = fmaxf(d2, __shfl_xor(d2, o));
+        m = fmaxf(m, __shfl_xor(m, o));
+        if constexpr (SOFT == 0) r2 = fmaxf(r2, __shfl_xor(r2, o));
+      }
+      if (q % kLaneGroup == 0)
+        s_group[q / kLaneGroup] = {cx, cy, cz, 1.00001f * __builtin_sqrtf(d2), 17.5f * m, r2};
     }
+    __syncthreads();
+    auto terms = [&](int j) {
+      PairTerms t;
+      pair_terms<SOFT, EXACT>(t, s_pos[j], 0.f, pi, ri2, eps2);
+      return F4{t.y[0], t.y[1], t.y[2], t.y[3]};
+    };
+    auto one = [&](int j) {
+      const F4 pj = s_pos[j];
+      const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
+      if constexpr (SOFT == 0) pair_spline<float, EXACT>(a, rx, ry, rz, ri2, pj.w, s_r2[j]);
+      else pair_plummer<float, EXACT>(a, rx, ry, rz, pj.w, eps2);
+    };
+    auto chain = [&](const F4& y) {
+      a.a0.sub(y.x);
+      a.a1.sub(y.y);
+      a.a2.sub(y.z);
+      a.a3.sub(y.w);
+    };
+    int g = 0;
+    F4 y = terms(0);
+    for (; (g + 1) * kLaneGroup <= cnt; ++g) {
+      const LaneGroup b = s_group[g];
+      const float dx = pi.x - b.x, dy = pi.y - b.y, dz = pi.z - b.z;
+      const float d = fmaxf(__builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz) - b.radius, 0.f);
+      const float d2 = SOFT == 1 ? d * d + eps2 : d * d;
+      const int j0 = g * kLaneGroup;
+      if (SOFT == 0 && !__all(0.99999f * d2 >= fmaxf(ri2, b.r2))) {
+        for (int k = 0; k < kLaneGroup; ++k) one(j0 + k);
+        y = terms(j0 + kLaneGroup);
+        continue;
+      }
+      const float inv = __builtin_amdgcn_rsqf(d2), pot = b.m * inv, acc = pot * inv;
+      const bool fast = fminf(fminf(fabsf(a.a0.hi), fabsf(a.a1.hi)), fabsf(a.a2.hi)) >= acc && fabsf(a.a3.hi) >= pot;
+      if (__all(fast)) {
+#pragma unroll 2
+        for (int k = 1; k <= kLaneGroup; ++k) {
+          const F4 n = terms(j0 + k);
+          a.a0.sub_fast(y.x);
+          a.a1.sub_fast(y.y);
+          a.a2.sub_fast(y.z);
+          a.a3.sub_fast(y.w);
+          y = n;
+        }
+      } else {
+#pragma unroll 1
+        for (int k = 1; k <= kLaneGroup; ++k) {
+          const F4 n = terms(j0 + k);
+          chain(y);
+          y = n;
+        }
+      }
+    }
+    for (int j = g * kLaneGroup; j < cnt; ++j) one(j);
   }
-  if (i < n_i) reinterpret_cast<float*>(out + i)[c] = acc.hi;
-}
-
-// Between the two: two wavefronts per 64 particles, one keeping ax and ay,
-// the other az and the potential, each repeating the pair's distance and
-// rsq once for its two two-sums, 4 records ahead.  Measured alone (ms per
-// launch, one lane / four wavefronts / two wavefronts): 16 384 particles
-// 1.85 / 0.89 / 1.23; 20 480: 2.31 / 1.56 / 1.53; 32 768: 3.71 / 2.54 / 2.46;
-// 49 152: 5.56 / 5.16 / 4.42; 65 536: 7.43 / 8.9 / 5.9.  In the plain step,
-// beside the SPH passes (whose walks take the higher issue priority), ms per
-// step: 16 384: 2.05 / 1.33 / 1.45; 32 768: 4.10 / 3.84 / 3.38; 49 152:
-// 5.72 / - / 5.26; 65 536: 7.62 / - / 6.72; 81 920: 10.47 / - / 13.2.
-template <int C0, int C1, bool EXACT>
-__device__ __forceinline__ void plummer_two(DR& a0, DR& a1, const F4* __restrict__ s_pos, int cnt, const F4& pi,
-                                            float eps2) {
-  pipelined<4>(
-      cnt,
-      [&](int j) {
-        const F4 pj = s_pos[j];
-        return float2{plummer_term<C0, EXACT>(pj, pi, eps2), plummer_term<C1, EXACT>(pj, pi, eps2)};
-      },
-      [&](const float2& y) {
-        dr_sub(a0, y.x);
-        dr_sub(a1, y.y);
-      });
-}
-
-constexpr int kTwoParticles = kGravBlock / 2;   // particles per block of k_gravity_two
-
-template <bool EXACT>
-__global__ __launch_bounds__(kGravBlock) void k_gravity_two(const F4* __restrict__ gpos, F4* __restrict__ out,
-                                                            int n_i, int n_j, float eps2) {
-  __shared__ F4 s_pos[kJTile];
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int half = w & 1;   // 0: ax, ay; 1: az, potential
-  const int i = blockIdx.x * kTwoParticles + (w >> 1) * 64 + (threadIdx.x & 63);
-  const F4 pi = gpos[i < n_i ? i : n_i - 1];
-  DR a0{0.f, 0.f}, a1{0.f, 0.f};
-  for (int t0 = 0; t0 < n_j; t0 += kJTile) {
-    const int cnt = stage_tile(s_pos, gpos, t0, n_j);
-    if (half == 0) plummer_two<0, 1, EXACT>(a0, a1, s_pos, cnt, pi, eps2);
-    else plummer_two<2, 3, EXACT>(a0, a1, s_pos, cnt, pi, eps2);
-  }
-  if (i < n_i) {
-    float* o = reinterpret_cast<float*>(out + i) + 2 * half;
-    o[0] = a0.hi;
-    o[1] = a1.hi;
-  }
+  if (i < n_i) out[i] = {a.a0.hi, a.a1.hi, a.a2.hi, a.a3.hi};
 }
 
 // ---------------------------------------------------------------------------
@@ -1173,9 +1433,9 @@ void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_
   }
 }
 
-int gravity_sums_mode(int n_i, int sums) {
-  if (sums >= 0) return sums;
-  return n_i <= kFourSumsMaxN ? 1 : (n_i <= kTwoSumsMaxN ? 2 : 0);
+bool gravity_by_chains(int n_i, int soft, int sums) {
+  if (sums >= 0) return sums != 0;
+  return n_i <= (soft == 1 ? kChainsMaxN : kChainsMaxNSpline);
 }
 
 template <class T>
@@ -1184,24 +1444,24 @@ void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, i
   const dim3 grid(ceil_div(n_i, kGravBlock)), block(kGravBlock);
   const T eps2 = eps * eps;
   if constexpr (sizeof(T) == 4) {
-    if (soft == 1) {
-      const int mode = gravity_sums_mode(n_i, sums);
-      if (mode == 2) {
-        const dim3 grid2(ceil_div(n_i, kTwoParticles));
-        if (exact) hipLaunchKernelGGL(k_gravity_two<true>, grid2, block, 0, s, gpos, out, n_i, n_j, eps2);
-        else hipLaunchKernelGGL(k_gravity_two<false>, grid2, block, 0, s, gpos, out, n_i, n_j, eps2);
-      } else if (mode == 1) {
-        const dim3 grid4(ceil_div(n_i, kSumParticles));
-        if (exact) hipLaunchKernelGGL(k_gravity_sums<true>, grid4, block, 0, s, gpos, out, n_i, n_j, eps2);
-        else hipLaunchKernelGGL(k_gravity_sums<false>, grid4, block, 0, s, gpos, out, n_i, n_j, eps2);
-      } else {
-        if (exact) hipLaunchKernelGGL(k_gravity_lane<true>, grid, block, 0, s, gpos, out, n_i, n_j, eps2);
-        else hipLaunchKernelGGL(k_gravity_lane<false>, grid, block, 0, s, gpos, out, n_i, n_j, eps2);
-      }
-    } else {
-      if (exact) hipLaunchKernelGGL((k_gravity<float, 0, 0, true>), grid, block, 0, s, gpos, gvel, out, n_i, n_j, eps2);
-      else hipLaunchKernelGGL((k_gravity<float, 0, 0, false>), grid, block, 0, s, gpos, gvel, out, n_i, n_j, eps2);
-    }
+    const bool chains = gravity_by_chains(n_i, soft, sums);
+    const auto pick = [&](auto soft_c, auto exact_c) {
+      constexpr int S = decltype(soft_c)::value;
+      constexpr bool E = decltype(exact_c)::value;
+      if (chains)
+        hipLaunchKernelGGL((k_gravity_chains<S, E>), dim3(ceil_div(n_i, kChainParticles)), dim3(kChainBlock), 0, s,
+                           gpos, gvel, out, n_i, n_j, eps2);
+      else if (S == 0 || n_i >= kFastLaneMinN)
+        hipLaunchKernelGGL((k_gravity_lane_fast<S, E>), grid, block, 0, s, gpos, gvel, out, n_i, n_j, eps2);
+      else
+        hipLaunchKernelGGL(k_gravity_lane<E>, grid, block, 0, s, gpos, out, n_i, n_j, eps2);
+    };
+    using Spline = std::integral_constant<int, 0>;
+    using Plummer = std::integral_constant<int, 1>;
+    if (soft == 1 && exact) pick(Plummer{}, std::true_type{});
+    else if (soft == 1) pick(Plummer{}, std::false_type{});
+    else if (exact) pick(Spline{}, std::true_type{});
+    else pick(Spline{}, std::false_type{});
   } else {
     if (soft == 0) hipLaunchKernelGGL((k_gravity<double, 0, 2, true>), grid, block, 0, s, gpos, gvel, out, n_i, n_j, eps2);
     else hipLaunchKernelGGL((k_gravity<double, 1, 2, true>), grid, block, 0, s, gpos, gvel, out, n_i, n_j, eps2);

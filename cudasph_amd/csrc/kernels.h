@@ -53,13 +53,14 @@ void launch_hydro(const V4<T>* pos, const V4<T>* vel, const V4<T>* hydro, const 
                   int n_dev, T alpha, T beta, hipStream_t s);
 
 // ---- gravity.hip ----
-// sums: for the FP32 Plummer kernel, 1 keeps each particle's four sums in
-// four wavefronts (k_gravity_sums), 2 in two (k_gravity_two), 0 in one lane
-// (k_gravity_lane), -1 (auto) four up to kFourSumsMaxN particles, two up to
-// kTwoSumsMaxN, one lane above; the same bits either way
-constexpr int kFourSumsMaxN = 16384;
-constexpr int kTwoSumsMaxN = 65536;
-int gravity_sums_mode(int n_i, int sums);
+// sums (FP32): 0 keeps a particle's four sums in one lane (k_gravity_lane), 1
+// and 2 one per wavefront (k_gravity_chains), -1 (auto) the latter up to
+// kChainsMaxN particles (kChainsMaxNSpline with the spline softening); the
+// same bits either way.  kFastLaneMinN: see k_gravity_lane.
+constexpr int kChainsMaxN = 94208;
+constexpr int kChainsMaxNSpline = 81920;
+constexpr int kFastLaneMinN = 1 << 19;
+bool gravity_by_chains(int n_i, int soft, int sums);
 template <class T>
 void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, int n_j, int soft, T eps,
                     int exact, hipStream_t s, int sums = -1);
