@@ -157,15 +157,13 @@ void write_state_from(EngineBase* e, FILE* f, int n, int nd) {
   }
 }
 
-// Scratch of sph_radix_sort_noalloc: the digit-count and offset tables and
-// the scan partials of launch_radix_sort for up to SPH_NOALLOC_SORT_MAX
-// records (4096 records per tile, 256 digits; radix_scratch_ints).  Each GPU
-// the library runs on holds its own copy until the process ends.  Host code
-// never uses this name as an address: sort_scratch_ptr() looks the device
-// address up once per device.
+// Scratch of sph_radix_sort_noalloc: the digit counts and tile tables of
+// launch_radix_sort for up to SPH_NOALLOC_SORT_MAX records (4096 records per
+// tile, 256 digits; radix_scratch_ints).  Each GPU the library runs on holds
+// its own copy until the process ends.  Host code never uses this name as an
+// address: sort_scratch_ptr() looks the device address up once per device.
 constexpr long kNoAllocSortMax = SPH_NOALLOC_SORT_MAX;
-constexpr long kNoAllocTable = 256L * ((kNoAllocSortMax + 4095) / 4096);
-constexpr long kNoAllocScratchInts = 2 * kNoAllocTable + 2 + (kNoAllocTable + 2047) / 2048 + 1;
+constexpr long kNoAllocScratchInts = radix_header_ints + 2 * 256L * ((kNoAllocSortMax + 4095) / 4096);
 static __device__ __align__(256) int g_sort_scratch[kNoAllocScratchInts];
 
 constexpr int kMaxDevices = 64;

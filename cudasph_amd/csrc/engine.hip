@@ -116,7 +116,7 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
   tr_end_.alloc(nd_ + 1);
   flags_.alloc(4);
   scan_tmp_.alloc(scan_scratch_ints(std::max<long>(cap_, nd_ + 1)) + 16);
-  sort_tmp_.alloc(radix_scratch_ints(cap_) + 16);
+  sort_tmp_.alloc(3 * radix_scratch_ints(nd_));   // three axes' sorts side by side
   dt_cur_.alloc(1);
   dt_next_.alloc(1);
   partials_.alloc(reduce_partials(nd_) + 64);
@@ -422,13 +422,8 @@ void Engine<T>::tree_fetch() {
     const long need = tree_work_ints(n_);
     if ((long)tree_work_.n < need) tree_work_.alloc(need);
     TimerScope ts(timers_, "tree_build", s_);
-    int* ties = nullptr;
-    if (tree_gpu_ == 2) {
-      CS_HIP(hipMemsetAsync(ties_, 0, sizeof(int), s_));
-      ties = ties_.p;
-    }
-    launch_tree_build<T>(pos_, n_, nd_, tree_, hash_, i_order_, tree_work_, pairs_, pairs_alt_, sort_tmp_, scan_tmp_,
-                         s_, ties);
+    launch_tree_build<T>(pos_, n_, nd_, tree_, hash_, i_order_, tree_work_, pairs_, pairs_alt_, sort_tmp_, s_,
+                         tree_gpu_ == 2 ? ties_.p : nullptr);
     boxes_stale_ = true;
     if (tree_gpu_ == 2) {
       CS_HIP(hipMemcpyAsync(h_pos_.p, pos_, (size_t)nd_ * sizeof(V4<T>), hipMemcpyDeviceToHost, s_));

@@ -94,19 +94,21 @@ void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F
 // scan_scratch_ints(n) ints.
 long scan_scratch_ints(long n);
 void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scratch, hipStream_t s);
-// two such scans (mode 0) in one launch sequence: the second's input and
-// output `stride` ints after the first's; scratch 2 scan_scratch_ints(n)
-void launch_exclusive_scan_pair(const int* in, int* out, long n, long stride, int* scratch, hipStream_t s);
 // stable LSD radix sort of KV records by key bits [0, bits); the result is
 // left in `data` (alt is scratch of the same length).  scratch holds
 // radix_scratch_ints(n) ints.
 long radix_scratch_ints(long n);
 void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s);
-// `batch` independent sorts of n records in one sequence of launches: sort b
-// on data + b * data_stride (alt likewise) with scratch + b *
-// radix_scratch_ints(n)
-void launch_radix_sort_batch(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s, int batch,
-                             long data_stride);
+constexpr long radix_header_ints = 8 * 257 + 8;
+// ints of a sort's scratch to be zero before launch_axis_sorts
+long radix_clear_ints(long n);
+// for each axis a the ids 0 .. n-1 in ascending order of (pos[id]'s coordinate
+// a, id), in lists + a * list_stride.  kv and alt hold 3 n records; scratch
+// 3 radix_scratch_ints(n) ints, the first radix_clear_ints(n) of each third
+// zero
+template <class T>
+void launch_axis_sorts(const V4<T>* pos, int n, KV* kv, KV* alt, int* lists, long list_stride, int* scratch,
+                       hipStream_t s);
 // the reaction lists: for each of the n particles j, the list slots k
 // naming j in ascending k, as pairs {key = owner i, value = k} in
 // pairs[start[j], end[j]) (end[j] = start[j + 1]; start holds n + 1 ints).
@@ -135,16 +137,15 @@ void launch_ph_keys(const V4<T>* pos, int n, int bits, uint32_t* key_hi, uint32_
 // device: tree[0..n_dev+1] and hash[0..n_dev) as the host builder writes them
 // (heap_order 1: hash in the nodes' heap order, 0: identity).  work holds
 // tree_work_ints(n) ints; kv and kv_alt 3 n records each; sort_scratch
-// 3 radix_scratch_ints(n) and scan_scratch 2 scan_scratch_ints(n) ints.
+// 3 radix_scratch_ints(n) ints.
 long tree_work_ints(long n);
-// ties (may be null): set to 1 when some node's particle shares its split
+// ties (may be null): cleared, and set to 1 when some node's particle shares its split
 // coordinate with another particle of its subtree -- the one case in which
 // the reference's quicksort may have picked the other particle as the node;
 // otherwise the tree is the reference's, bit for bit.
 template <class T>
 void launch_tree_build(const V4<T>* pos, int n, int n_dev, V4<T>* tree, KV* hash, int heap_order, int* work,
-                       KV* kv, KV* kv_alt, int* sort_scratch, int* scan_scratch, hipStream_t s,
-                       int* ties = nullptr);
+                       KV* kv, KV* kv_alt, int* sort_scratch, hipStream_t s, int* ties = nullptr);
 // Subtree bounding boxes of a kd-tree over n_nodes particles: box[2k] (low
 // corner) and box[2k+1] (high corner) of node k's subtree, for k up to
 // n_nodes+1; FP32, rounded outward.  Two launches: one block per subtree

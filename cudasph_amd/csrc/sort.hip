@@ -1,15 +1,6 @@
 // Device-wide primitives: exclusive scan, stable LSD radix sort of
 // (key,value) records, the counting-sort transpose that turns the i-side
 // neighbour lists into j-side reaction lists, and Peano-Hilbert keys.
-//
-// The radix sort replaces the reference's RadixSort (radixsort.cu:50-77).
-// Each pass (8 key bits) is three launches: per-tile digit histograms,
-// an exclusive scan of the digit-major histogram table, and a stable
-// scatter.  The scatter ranks a tile in 16 striped rounds of 256 records; in
-// each round a wavefront finds the lanes holding the same digit with eight
-// ballots (one per digit bit), takes its rank from a popcount, and adds the
-// counts of the lower wavefronts from LDS.  Equal keys keep their input
-// order, which the reaction pass relies on.
 #include <algorithm>
 
 #include "kernels.h"
@@ -43,14 +34,9 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_tmp, int& tota
   return incl - v;
 }
 
-// Batched scans (blockIdx.y = batch b): array b's input and output start
-// `stride` ints after array b-1's, its tile partials `pstride` ints after
-// b-1's.
 __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int* __restrict__ in, long n, int mode,
-                                                             int* __restrict__ partial, long stride, long pstride) {
+                                                             int* __restrict__ partial) {
   __shared__ int s_tmp[kScanBlock];
-  in += blockIdx.y * stride;
-  partial += blockIdx.y * pstride;
   const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
   int sum = 0;
   for (int k = 0; k < kScanItems; ++k) sum += scan_load(in, base + k, n, mode);
@@ -60,9 +46,8 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int* __restric
 }
 
 // one block scans the tile partials in chunks of 256, carrying the sum
-__global__ __launch_bounds__(kScanBlock) void k_scan_partials(int* __restrict__ partial, int n_part, long pstride) {
+__global__ __launch_bounds__(kScanBlock) void k_scan_partials(int* __restrict__ partial, int n_part) {
   __shared__ int s_tmp[kScanBlock];
-  partial += blockIdx.y * pstride;
   int carry = 0;
   for (int c0 = 0; c0 < n_part; c0 += kScanBlock) {
     const int idx = c0 + threadIdx.x;
@@ -77,11 +62,8 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_partials(int* __restrict__ 
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_down(const int* __restrict__ in, long n, int mode,
                                                            const int* __restrict__ partial, int* __restrict__ out,
-                                                           int n_part, long stride, long pstride) {
+                                                           int n_part) {
   __shared__ int s_tmp[kScanBlock];
-  in += blockIdx.y * stride;
-  partial += blockIdx.y * pstride;
-  out += blockIdx.y * stride;
   const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
   int v[kScanItems];
   int sum = 0;
@@ -100,144 +82,305 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(const int* __restrict_
 
 long scan_scratch_ints(long n) { return (n + kScanTile - 1) / kScanTile + 1; }
 
-// `batch` scans at once: in and out of scan b at b * stride ints past the
-// first's, its scratch at b * pstride
-static void exclusive_scan_batch(const int* in, int* out, long n, int mode, int* scratch, hipStream_t s,
-                                 int batch, long stride, long pstride) {
+void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scratch, hipStream_t s) {
   const int n_part = (int)((n + kScanTile - 1) / kScanTile);
   if (n_part == 0) {
-    for (int b = 0; b < batch; ++b) CS_HIP(hipMemsetAsync(out + b * stride, 0, sizeof(int), s));
+    CS_HIP(hipMemsetAsync(out, 0, sizeof(int), s));
     return;
   }
-  hipLaunchKernelGGL(k_scan_reduce, dim3(n_part, batch), dim3(kScanBlock), 0, s, in, n, mode, scratch, stride,
-                     pstride);
+  hipLaunchKernelGGL(k_scan_reduce, dim3(n_part), dim3(kScanBlock), 0, s, in, n, mode, scratch);
   CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_scan_partials, dim3(1, batch), dim3(kScanBlock), 0, s, scratch, n_part, pstride);
+  hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kScanBlock), 0, s, scratch, n_part);
   CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_scan_down, dim3(n_part, batch), dim3(kScanBlock), 0, s, in, n, mode, scratch, out, n_part,
-                     stride, pstride);
+  hipLaunchKernelGGL(k_scan_down, dim3(n_part), dim3(kScanBlock), 0, s, in, n, mode, scratch, out, n_part);
   CS_CHECK_LAUNCH();
-}
-
-void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scratch, hipStream_t s) {
-  exclusive_scan_batch(in, out, n, mode, scratch, s, 1, 0, 0);
-}
-
-void launch_exclusive_scan_pair(const int* in, int* out, long n, long stride, int* scratch, hipStream_t s) {
-  exclusive_scan_batch(in, out, n, 0, scratch, s, 2, stride, scan_scratch_ints(n));
 }
 
 // ---------------------------------------------------------------------------
-// radix sort
-constexpr int kRadixBlock = 256;
-constexpr int kRadixRounds = 16;
-constexpr int kRadixTile = kRadixBlock * kRadixRounds;   // 4096 records per block
+// Radix sort (replaces the reference's RadixSort, radixsort.cu:50-77): stable,
+// least significant digit first, 8 bits a pass, one launch and one reading
+// and writing of the records per pass.
+//
+// The digit counts of all passes are taken in one reading of the keys (they
+// do not depend on the order).  In a pass a block sorts a tile of 4096
+// records by its digit: each wavefront ranks its 256 records by matching
+// digits with ballots, the block's digit counts come from the wavefronts'
+// in order, and the tile goes out through LDS in runs of equal digits.
+// Where a tile's run of digit d starts is the count of smaller digits plus
+// that of d in earlier tiles.  For the latter the tiles publish their digit
+// counts in a table and look back over it (decoupled look-back, Merrill and
+// Garland): an entry says whether it holds the tile's own count or already
+// the sum over all tiles up to it, and a tile adds earlier ones' counts until
+// it meets a sum.  Tiles take their number from a counter as they start, so a
+// tile waits only for ones that are running, and those publish before they
+// wait.  A pass uses one of two tables and clears its part of the other for
+// the next.
+//
+// Bound: the records in and out (16 B a pass and record) for many records,
+// the chain of launches for few.  1 000 003 records, 4 passes: 137 us with a
+// histogram, a scan of 3 launches and a scatter per pass -> 51 us.
+constexpr int kRadixBlock = 1024;
+constexpr int kRadixItems = 4;
+constexpr int kRadixTile = kRadixBlock * kRadixItems;   // records per block
+constexpr int kRadixMaxPasses = 8;
+constexpr unsigned kCountFlag = 1u << 30, kSumFlag = 2u << 30, kCountMask = kCountFlag - 1;
+// polls of a table entry before a tile gives up (seconds; an earlier tile
+// that never publishes can only mean that another sort uses the same scratch)
+constexpr int kRadixMaxPolls = 1 << 22;
 
-__global__ __launch_bounds__(kRadixBlock) void k_radix_hist(const KV* __restrict__ in, long n, int shift,
-                                                             int* __restrict__ counts, int n_blocks,
-                                                             long data_stride, long scratch_stride) {
-  __shared__ int s_hist[256];
-  in += blockIdx.y * data_stride;
-  counts += blockIdx.y * scratch_stride;
-  s_hist[threadIdx.x] = 0;
-  __syncthreads();
-  const long base = (long)blockIdx.x * kRadixTile;
-  for (int r = 0; r < kRadixRounds; ++r) {
-    const long p = base + r * kRadixBlock + threadIdx.x;
-    if (p < n) atomicAdd(&s_hist[(in[p].key >> shift) & 255], 1);
-  }
-  __syncthreads();
-  counts[(long)threadIdx.x * n_blocks + blockIdx.x] = s_hist[threadIdx.x];
+// scratch of one sort: digit counts of each pass, the tile counter of each
+// pass, two tables of 256 entries per tile
+__host__ __device__ __forceinline__ long radix_tiles(long n) { return (n + kRadixTile - 1) / kRadixTile; }
+long radix_scratch_ints(long n) { return radix_header_ints + 2 * 256 * radix_tiles(n); }
+static_assert(radix_header_ints >= kRadixMaxPasses * 257, "counts and counters");
+
+// zero the header and the first table
+__global__ __launch_bounds__(kBlock) void k_radix_clear(int* __restrict__ scratch, long count, long stride) {
+  const long t = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (t < count) scratch[blockIdx.y * stride + t] = 0;
+}
+long radix_clear_ints(long n) { return radix_header_ints + 256 * radix_tiles(n); }
+
+// adds the digit counts of 4 keys' worth of passes for one record
+__device__ __forceinline__ void count_digits(int (*s_hist)[256], uint32_t key, int first, int passes) {
+  for (int p = 0; p < passes; ++p) atomicAdd(&s_hist[first + p][(key >> (8 * p)) & 255], 1);
 }
 
-__global__ __launch_bounds__(kRadixBlock) void k_radix_scatter(const KV* __restrict__ in, KV* __restrict__ out,
-                                                                long n, int shift,
-                                                                const int* __restrict__ offsets, int n_blocks,
-                                                                long data_stride, long scratch_stride) {
-  __shared__ int s_base[256];
-  in += blockIdx.y * data_stride;
-  out += blockIdx.y * data_stride;
-  offsets += blockIdx.y * scratch_stride;
-  __shared__ int s_wave[4][256];
+__global__ __launch_bounds__(kRadixBlock) void k_radix_count(const KV* __restrict__ in, long n, int passes,
+                                                              int* __restrict__ scratch) {
+  __shared__ int s_hist[4][256];
+  (&s_hist[0][0])[threadIdx.x] = 0;
+  __syncthreads();
+  for (int r = 0; r < kRadixItems; ++r) {
+    const long p = (long)blockIdx.x * kRadixTile + r * kRadixBlock + threadIdx.x;
+    if (p < n) count_digits(s_hist, in[p].key, 0, passes);
+  }
+  __syncthreads();
+  const int c = (&s_hist[0][0])[threadIdx.x];
+  if (c && (int)threadIdx.x < passes * 256) atomicAdd(&scratch[threadIdx.x], c);
+}
+
+// rekey(record) may replace a record's key as it is read; out_ids, if given,
+// receives the values alone
+template <class Rekey>
+__device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __restrict__ out, int* __restrict__ out_ids,
+                                           long n, int shift, int pass, int* __restrict__ scratch, Rekey&& rekey) {
+  __shared__ int s_cnt[kRadixBlock / 64][256];   // per wavefront and digit: count, then first place
+  __shared__ KV s_rec[kRadixTile];
+  __shared__ int s_local[256], s_out[256];       // a digit's first place in the tile; its run's place in `out`, less that
+  __shared__ int s_tot[2][4];
+  __shared__ int s_tile;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  s_base[tid] = offsets[(long)tid * n_blocks + blockIdx.x];
-  const long base = (long)blockIdx.x * kRadixTile;
-  for (int r = 0; r < kRadixRounds; ++r) {
-    s_wave[0][tid] = 0;
-    s_wave[1][tid] = 0;
-    s_wave[2][tid] = 0;
-    s_wave[3][tid] = 0;
-    __syncthreads();
-    const long p = base + r * kRadixBlock + tid;
-    const bool valid = p < n;
-    KV rec{0u, 0u};
-    int d = 0;
-    if (valid) {
-      rec = in[p];
-      d = (int)((rec.key >> shift) & 255);
-    }
+  const long tiles = radix_tiles(n);
+  int* hist = scratch + pass * 256;
+  int* counter = scratch + kRadixMaxPasses * 256 + pass;
+  unsigned* table = reinterpret_cast<unsigned*>(scratch + radix_header_ints) + (pass & 1) * 256 * tiles;
+  unsigned* other = reinterpret_cast<unsigned*>(scratch + radix_header_ints) + ((pass & 1) ^ 1) * 256 * tiles;
+  if (tid == 0) s_tile = atomicAdd(counter, 1);
+  for (int q = tid; q < kRadixBlock / 64 * 256; q += kRadixBlock) (&s_cnt[0][0])[q] = 0;
+  __syncthreads();
+  const long tile = s_tile, base = tile * kRadixTile;
+  if (tile >= tiles) return;   // (a counter shared with another sort)
+  const int cnt = (int)(n - base < kRadixTile ? n - base : kRadixTile);
+  KV rec[kRadixItems];
+  int rank[kRadixItems];
+#pragma unroll
+  for (int r = 0; r < kRadixItems; ++r) {
+    const int q = wave * 64 * kRadixItems + r * 64 + lane;
+    rec[r] = q < cnt ? rekey(in[base + q]) : KV{0u, 0u};
+  }
+#pragma unroll
+  for (int r = 0; r < kRadixItems; ++r) {
+    const bool valid = wave * 64 * kRadixItems + r * 64 + lane < cnt;
+    const int d = (int)((rec[r].key >> shift) & 255);
     unsigned long long same = __ballot(valid);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      const int bit = (d >> b) & 1;
+      const bool bit = (d >> b) & 1;
       const unsigned long long m = __ballot(valid && bit);
       same &= bit ? m : ~m;
     }
-    const int rank = __popcll(same & ((1ull << lane) - 1ull));
-    if (valid && rank == 0) s_wave[wave][d] = __popcll(same);
-    __syncthreads();
-    if (valid) {
-      int before = 0;
-      for (int w = 0; w < wave; ++w) before += s_wave[w][d];
-      out[s_base[d] + before + rank] = rec;
+    const int below = __popcll(same & ((1ull << lane) - 1ull));
+    const int before = s_cnt[wave][d];
+    rank[r] = before + below;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && below == 0) s_cnt[wave][d] = before + __popcll(same);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  __syncthreads();
+  int total = 0, excl = 0, smaller = 0;
+  if (tid < 256) {   // digit tid
+    for (int w = 0; w < kRadixBlock / 64; ++w) {
+      const int c = s_cnt[w][tid];
+      s_cnt[w][tid] = total;
+      total += c;
     }
-    __syncthreads();
-    s_base[tid] += s_wave[0][tid] + s_wave[1][tid] + s_wave[2][tid] + s_wave[3][tid];
-    __syncthreads();
+    __hip_atomic_store(&table[tile * 256 + tid], (tile == 0 ? kSumFlag : kCountFlag) | (unsigned)total,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    other[tile * 256 + tid] = 0;
+    // exclusive sums over the digits: of the tile's counts, of all records'
+    int x = total, y = hist[tid];
+    const int y0 = y;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int ux = __shfl_up(x, o), uy = __shfl_up(y, o);
+      if (lane >= o) {
+        x += ux;
+        y += uy;
+      }
+    }
+    if (lane == 63) {
+      s_tot[0][wave] = x;
+      s_tot[1][wave] = y;
+    }
+    excl = x - total;
+    smaller = y - y0;
+  }
+  __syncthreads();
+  if (tid < 256) {
+    for (int w = 0; w < wave; ++w) {
+      excl += s_tot[0][w];
+      smaller += s_tot[1][w];
+    }
+    s_local[tid] = excl;
+    unsigned earlier = 0;
+    int polls = 0;
+    for (long t = tile - 1; t >= 0;) {
+      constexpr int kAhead = 4;   // entries read together
+      unsigned v[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        v[k] = t - k >= 0 ? __hip_atomic_load(&table[(t - k) * 256 + tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                          : kSumFlag;
+      bool done = false;
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        if (done || v[k] < kCountFlag) break;   // not published: read again from here
+        earlier += v[k] & kCountMask;
+        done = v[k] >= kSumFlag;
+        --t;
+      }
+      if (done || ++polls > kRadixMaxPolls) break;
+    }
+    if (tile > 0)
+      __hip_atomic_store(&table[tile * 256 + tid], kSumFlag | (earlier + (unsigned)total), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    s_out[tid] = smaller + (int)earlier - excl;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRadixItems; ++r) {
+    const int d = (int)((rec[r].key >> shift) & 255);
+    if (wave * 64 * kRadixItems + r * 64 + lane < cnt) s_rec[s_local[d] + s_cnt[wave][d] + rank[r]] = rec[r];
+  }
+  __syncthreads();
+  for (int q = tid; q < cnt; q += kRadixBlock) {
+    const KV e = s_rec[q];
+    const long to = (long)s_out[(e.key >> shift) & 255] + q;
+    if (to < 0 || to >= n) continue;   // (only where the table was not this sort's alone)
+    if (out_ids) out_ids[to] = (int)e.value;
+    else out[to] = e;
   }
 }
 
-long radix_scratch_ints(long n) {
-  const long nb = (n + kRadixTile - 1) / kRadixTile;
-  const long table = 256 * nb;
-  return 2 * table + 2 + scan_scratch_ints(table);
-}
-
-void launch_radix_sort_batch(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s, int batch,
-                             long data_stride) {
-  if (n <= 1 || bits <= 0 || batch <= 0) return;
-  const int nb = (int)((n + kRadixTile - 1) / kRadixTile);
-  const long table = 256L * nb;
-  const long sstride = radix_scratch_ints(n);   // each sort's scratch
-  int* counts = scratch;
-  int* offsets = scratch + table;
-  int* scan_tmp = scratch + 2 * table + 2;
-  KV* src = data;
-  KV* dst = alt;
-  int passes = 0;
-  for (int shift = 0; shift < bits; shift += 8, ++passes) {
-    hipLaunchKernelGGL(k_radix_hist, dim3(nb, batch), dim3(kRadixBlock), 0, s, src, n, shift, counts, nb,
-                       data_stride, sstride);
-    CS_CHECK_LAUNCH();
-    // the scan's input, output and partials sit at the same offsets in
-    // every sort's scratch
-    exclusive_scan_batch(counts, offsets, table, 0, scan_tmp, s, batch, sstride, sstride);
-    hipLaunchKernelGGL(k_radix_scatter, dim3(nb, batch), dim3(kRadixBlock), 0, s, src, dst, n, shift, offsets, nb,
-                       data_stride, sstride);
-    CS_CHECK_LAUNCH();
-    KV* t = src;
-    src = dst;
-    dst = t;
-  }
-  if (passes & 1)
-    for (int b = 0; b < batch; ++b)
-      CS_HIP(hipMemcpyAsync(data + b * data_stride, alt + b * data_stride, n * sizeof(KV), hipMemcpyDeviceToDevice,
-                            s));
+__global__ __launch_bounds__(kRadixBlock) void k_radix_pass(const KV* __restrict__ in, KV* __restrict__ out, long n,
+                                                             int shift, int pass, int* __restrict__ scratch) {
+  radix_pass(in, out, nullptr, n, shift, pass, scratch, [](const KV& e) { return e; });
 }
 
 void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s) {
-  launch_radix_sort_batch(data, alt, n, bits, scratch, s, 1, 0);
+  if (n <= 1 || bits <= 0) return;
+  const int passes = std::min(4, (bits + 7) / 8), nb = (int)radix_tiles(n);
+  const long clear = radix_clear_ints(n);
+  hipLaunchKernelGGL(k_radix_clear, dim3(ceil_div(clear, kBlock)), dim3(kBlock), 0, s, scratch, clear, 0l);
+  CS_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_radix_count, dim3(nb), dim3(kRadixBlock), 0, s, data, n, passes, scratch);
+  CS_CHECK_LAUNCH();
+  KV* src = data;
+  KV* dst = alt;
+  for (int p = 0; p < passes; ++p) {
+    hipLaunchKernelGGL(k_radix_pass, dim3(nb), dim3(kRadixBlock), 0, s, src, dst, n, 8 * p, p, scratch);
+    CS_CHECK_LAUNCH();
+    std::swap(src, dst);
+  }
+  if (passes & 1) CS_HIP(hipMemcpyAsync(data, alt, n * sizeof(KV), hipMemcpyDeviceToDevice, s));
 }
+
+// The three axes' presorts of the tree build (blockIdx.y = axis): ids in
+// ascending order of (coordinate image, id).
+//
+// order-preserving unsigned images of a coordinate (IEEE: flip all bits of a
+// negative value, the sign bit of a positive one)
+__device__ __forceinline__ uint32_t ordered_bits(float x) {
+  const uint32_t u = __float_as_uint(x);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ uint64_t ordered_bits(double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  return (u & 0x8000000000000000ull) ? ~u : (u | 0x8000000000000000ull);
+}
+template <class T>
+__device__ __forceinline__ T coordinate(const V4<T>& p, int axis) {
+  return axis == 0 ? p.x : (axis == 1 ? p.y : p.z);
+}
+
+// records {low key word, id} and the digit counts of every pass
+template <class T>
+__global__ __launch_bounds__(kRadixBlock) void k_axis_keys(const V4<T>* __restrict__ pos, KV* __restrict__ kv, int n,
+                                                            int* __restrict__ scratch, long stride) {
+  constexpr int P = (int)sizeof(T);   // passes
+  __shared__ int s_hist[P][256];
+  const int axis = blockIdx.y;
+  for (int q = threadIdx.x; q < P * 256; q += kRadixBlock) (&s_hist[0][0])[q] = 0;
+  __syncthreads();
+  for (int r = 0; r < kRadixItems; ++r) {
+    const int i = blockIdx.x * kRadixTile + r * kRadixBlock + threadIdx.x;
+    if (i >= n) continue;
+    const auto b = ordered_bits(coordinate(pos[i], axis));
+    kv[(size_t)axis * n + i] = {(uint32_t)b, (uint32_t)i};
+    count_digits(s_hist, (uint32_t)b, 0, 4);
+    if constexpr (P == 8) count_digits(s_hist, (uint32_t)(b >> 32), 4, 4);
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < P * 256; q += kRadixBlock) {
+    const int c = (&s_hist[0][0])[q];
+    if (c) atomicAdd(&scratch[axis * stride + q], c);
+  }
+}
+
+// pass p; the pass that starts the high key words (FP64) takes them from the
+// coordinates; the last one writes the ids to the axis's list
+template <class T>
+__global__ __launch_bounds__(kRadixBlock) void k_axis_pass(const KV* __restrict__ in, KV* __restrict__ out,
+                                                            int* __restrict__ lists, long list_stride, int n, int pass,
+                                                            int* __restrict__ scratch, long stride,
+                                                            const V4<T>* __restrict__ pos) {
+  __builtin_amdgcn_s_setprio(3);   // a chain of short passes; beside gravity it would wait for issue
+  const int axis = blockIdx.y;
+  radix_pass(in + (size_t)axis * n, out + (size_t)axis * n,
+             pass == (int)sizeof(T) - 1 ? lists + axis * list_stride : nullptr, n, 8 * (pass & 3), pass,
+             scratch + axis * stride, [&](const KV& e) {
+               if (sizeof(T) == 8 && pass == 4)
+                 return KV{(uint32_t)((uint64_t)ordered_bits(coordinate(pos[e.value], axis)) >> (sizeof(T) * 4)),
+                           e.value};
+               return e;
+             });
+}
+
+template <class T>
+void launch_axis_sorts(const V4<T>* pos, int n, KV* kv, KV* alt, int* lists, long list_stride, int* scratch,
+                       hipStream_t s) {
+  const int nb = (int)radix_tiles(n);
+  const long stride = radix_scratch_ints(n);
+  hipLaunchKernelGGL(k_axis_keys<T>, dim3(nb, 3), dim3(kRadixBlock), 0, s, pos, kv, n, scratch, stride);
+  CS_CHECK_LAUNCH();
+  for (int p = 0; p < (int)sizeof(T); ++p) {
+    hipLaunchKernelGGL(k_axis_pass<T>, dim3(nb, 3), dim3(kRadixBlock), 0, s, (p & 1) ? alt : kv, (p & 1) ? kv : alt,
+                       lists, list_stride, n, p, scratch, stride, pos);
+    CS_CHECK_LAUNCH();
+  }
+}
+template void launch_axis_sorts<float>(const F4*, int, KV*, KV*, int*, long, int*, hipStream_t);
+template void launch_axis_sorts<double>(const D4*, int, KV*, KV*, int*, long, int*, hipStream_t);
 
 // ---------------------------------------------------------------------------
 // reaction transpose: for every j, the list slots k that name j, in

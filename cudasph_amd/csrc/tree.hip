@@ -9,23 +9,29 @@
 // nodes of a level are closed forms of n (subtree_size, subtree_start).
 //
 // The build is level by level, on three lists of particle ids, one per axis,
-// each sorted once by that coordinate (stable LSD radix sort on an
-// order-preserving integer image of the coordinate) and kept grouped by
-// subtree: at level L every particle not yet placed carries the heap index t
-// of the level-L subtree that holds it, and each list holds the unplaced
-// particles subtree by subtree (t ascending), each subtree's run still in
-// its axis's order.  One level:
+// each sorted once by (coordinate, id) (launch_axis_sorts) and kept grouped by
+// subtree: at level L each list holds the particles not yet placed subtree by
+// subtree (t ascending), each subtree's run still in its axis's order.  A
+// place in a list tells its subtree (subtree_at), all in closed form.  One
+// level, two launches:
 //  * the list of the split axis L % 3 holds each subtree's particles in split
 //    order, so the particle at rank size(2t) of the run becomes node t, the
 //    ones before go to subtree 2t and the ones after to 2t+1 -- both runs stay
 //    contiguous and in order, shifted by the closed-form count of nodes placed
 //    before them;
-//  * the other two lists are partitioned stably: a particle going to 2t is
-//    placed after the earlier ones of its run going to 2t (an exclusive scan
-//    of "goes left" flags), one going to 2t+1 after the earlier ones going
-//    right (its rank in the run minus those going left and the one placed).
+//  * the other two lists are partitioned stably.  A particle's side follows
+//    from (its coordinate, its id) against the node's particle's -- the order
+//    of the split axis's list.  k_tree_count finds the sides and counts them
+//    per tile of 1024 places; k_tree_move adds the tiles before, and places each
+//    particle after the earlier ones of its side: those of its own run are the
+//    counted ones less the closed-form total of the runs before.
 // Levels: floor(log2 n) + 1.  Work per level is O(n); nothing is sorted after
 // the first three sorts.
+//
+// Bound: the latency of its dependent launches (few particles) and of their
+// gathers.  Five launches of presorts, two per level and the LDS finish, in
+// place of 22, six per level and the finish; every closed form is a handful of
+// operations (they had been loops over the levels).
 //
 // Ties in a coordinate: the reference's first-element-pivot quicksort decides
 // which of two equal-coordinate particles becomes the node; here the order of
@@ -39,40 +45,53 @@
 namespace cudasph {
 namespace {
 
-// nodes in the subtree of heap node t of the complete tree of n nodes
+// The complete tree of n nodes: levels 0 .. D, all full but the last, which
+// holds heap nodes 2^D .. n.  A node k levels above the last has 2^k places in
+// it, filled from the left.
+__host__ __device__ __forceinline__ int floor_log2(int x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return 31 - __clz(x);
+#else
+  return 31 - __builtin_clz((unsigned)x);
+#endif
+}
+
+// nodes in the subtree of heap node t (0 if t > n)
 __host__ __device__ __forceinline__ int subtree_size(int t, int n) {
-  int size = 0;
-  long long lo = t, hi = t;
-  while (lo <= n) {
-    size += (int)((hi < n ? hi : n) - lo + 1);
-    lo <<= 1;
-    hi = (hi << 1) | 1;
-  }
-  return size;
+  if (t > n) return 0;
+  const int k = floor_log2(n) - floor_log2(t);
+  const int first = t << k, last = n - first + 1;   // (places of the last level: below 2^24)
+  return (1 << k) - 1 + (last < 0 ? 0 : last < (1 << k) ? last : 1 << k);
 }
 
 // among the nodes of levels >= L, laid out subtree by subtree, the offset of
-// the subtree of level-L node t: the nodes below the level-L nodes left of t
+// the subtree of level-L node t (2^L <= t <= 2^(L+1)): the nodes below the
+// level-L nodes left of t
 __host__ __device__ __forceinline__ int subtree_start(int t, int L, int n) {
-  int s = 0;
-  long long a = 1ll << L, b = t;
-  while (a <= n) {
-    s += (int)((b < (long long)n + 1 ? b : (long long)n + 1) - a);
-    a <<= 1;
-    b <<= 1;
-  }
-  return s;
+  const int k = floor_log2(n) - L;
+  if (k < 0) return 0;
+  const int m = t - (1 << L), fill = n + 1 - (1 << (k + L)), slots = m << k;
+  return m * ((1 << k) - 1) + (slots < fill ? slots : fill);
 }
 
-// order-preserving unsigned images of a coordinate (IEEE: flip all bits of a
-// negative value, the sign bit of a positive one)
-__device__ __forceinline__ uint32_t ordered_bits(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+// of those, the ones below left children
+__host__ __device__ __forceinline__ int lefts_before(int t, int L, int n) {
+  const int k = floor_log2(n) - L - 1;   // of the level-(L+1) children
+  if (k < 0) return 0;
+  const int m = t - (1 << L), fill = n + 1 - (1 << (k + 1 + L)), slots = m << (k + 1);
+  const int filled = slots < fill ? slots : fill;
+  const int part = filled & ((2 << k) - 1);
+  return m * ((1 << k) - 1) + ((filled >> (k + 1)) << k) + (part < (1 << k) ? part : 1 << k);
 }
-__device__ __forceinline__ uint64_t ordered_bits(double x) {
-  const uint64_t u = (uint64_t)__double_as_longlong(x);
-  return (u & 0x8000000000000000ull) ? ~u : (u | 0x8000000000000000ull);
+
+// the level-L node whose run holds place idx of the level's layout
+__host__ __device__ __forceinline__ int subtree_at(int idx, int L, int n) {
+  const int k = floor_log2(n) - L;
+  const int fill = n + 1 - (1 << (k + L)), full = fill >> k, part = fill & ((1 << k) - 1);
+  const int large = (2 << k) - 1, small = (1 << k) - 1;   // a subtree's nodes with and without its last level
+  if (idx < full * large) return (1 << L) + idx / large;
+  idx -= full * large;
+  return (1 << L) + full + (idx < small + part ? 0 : 1 + (idx - small - part) / small);
 }
 
 template <class T>
@@ -83,38 +102,18 @@ __device__ __forceinline__ T coord(const V4<T>& p, int axis) {
 __device__ __forceinline__ float node_word(float, int bits) { return __int_as_float(bits); }
 __device__ __forceinline__ double node_word(double, int bits) { return (double)bits; }
 
-// key word `word` (0: low 32 bits, 1: high 32 bits of a double's image) of
-// the coordinate of particle `value` (the value of the record, so a second
-// pass re-keys records already ordered by the first)
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_tree_keys(const V4<T>* __restrict__ pos, KV* __restrict__ kv, int n,
-                                                       int word, int first) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  const int axis = blockIdx.y;   // the three axes' records one after another in kv
-  kv += (size_t)axis * n;
-  if (i >= n) return;
-  const int id = first ? i : (int)kv[i].value;
-  const auto b = ordered_bits(coord(pos[id], axis));
-  kv[i] = {(uint32_t)(word ? (uint64_t)b >> 32 : (uint64_t)b & 0xffffffffu), (uint32_t)id};
-}
-
-// axis blockIdx.y's sorted ids into its list (the lists 2 n ints apart)
-__global__ __launch_bounds__(kBlock) void k_tree_ids(const KV* __restrict__ kv, int* __restrict__ list,
-                                                      int* __restrict__ tag, int n) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  const int axis = blockIdx.y;
-  if (i >= n) return;
-  list[(size_t)axis * 2 * n + i] = (int)kv[(size_t)axis * n + i].value;
-  if (axis == 0) tag[i] = 1;
-}
-
 // fixed slots (sph_accelerations.cpp:21-33, read_state.cpp:85-88): slot 0 and
 // slot n_dev+1 zero, slots n+1..n_dev far sentinels with split 3; the
 // identity hash, or the padding part of the heap-order hash
+// and the zeros that the presorts start from
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_tree_fixed(V4<T>* __restrict__ tree, KV* __restrict__ hash, int n,
-                                                        int n_dev, int heap_order) {
+                                                        int n_dev, int heap_order, int* __restrict__ scratch,
+                                                        int clear, long stride, int* __restrict__ ties) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t < clear)
+    for (int a = 0; a < 3; ++a) scratch[a * stride + t] = 0;
+  if (ties && t == 0) *ties = 0;
   if (t >= n_dev + 2) return;
   if (t == 0 || t == n_dev + 1) tree[t] = {T(0), T(0), T(0), T(0)};
   else if (t > n) tree[t] = {T(1e10), T(1e10), T(1e10), node_word(T(0), -1)};
@@ -124,87 +123,160 @@ __global__ __launch_bounds__(kBlock) void k_tree_fixed(V4<T>* __restrict__ tree,
   }
 }
 
-// level L on the split axis's list (m unplaced particles): place the medians,
-// give every other particle its child subtree, and move it to its run of the
-// next level's layout
+// order of the split axis's list: (coordinate image, id)
+__device__ __forceinline__ bool before(float a, int ia, float b, int ib) {
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  const uint32_t ox = (x & 0x80000000u) ? ~x : (x | 0x80000000u), oy = (y & 0x80000000u) ? ~y : (y | 0x80000000u);
+  return ox < oy || (ox == oy && ia < ib);
+}
+__device__ __forceinline__ bool before(double a, int ia, double b, int ib) {
+  const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b), top = 1ull << 63;
+  const uint64_t ox = (x & top) ? ~x : (x | top), oy = (y & top) ? ~y : (y | top);
+  return ox < oy || (ox == oy && ia < ib);
+}
+
+constexpr int kLevelRounds = 4;
+constexpr int kLevelTile = kBlock * kLevelRounds;   // places per block
+enum { kPlaced = 0, kLeft = 1, kRight = 2 };
+
+// place of round r of this thread in its tile: each wavefront takes 256
+// consecutive places
+__device__ __forceinline__ int level_place(int r) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  return blockIdx.x * kLevelTile + wave * (kLevelTile / 4) + r * 64 + lane;
+}
+
+// level L: the side of every place of the two lists not split (blockIdx.y 0,
+// 1), and each tile's {left, right} counts
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_tree_split(const int* __restrict__ la, int* __restrict__ la_next,
-                                                        int* __restrict__ tag, const V4<T>* __restrict__ pos,
-                                                        V4<T>* __restrict__ tree, KV* __restrict__ hash, int m,
-                                                        int L, int n, int axis, int heap_order,
-                                                        int* __restrict__ ties) {
-  const int idx = blockIdx.x * kBlock + threadIdx.x;
-  if (idx >= m) return;
-  const int id = la[idx];
-  const int t = tag[id];
-  const int p = idx - subtree_start(t, L, n);
-  const int lt = 2 * t <= n ? subtree_size(2 * t, n) : 0;
-  const int placed_before = t - (1 << L);   // level-L nodes left of t
-  if (p < lt) {
-    tag[id] = 2 * t;
-    la_next[idx - placed_before] = id;
-  } else if (p == lt) {
-    const V4<T> q = pos[id];
-    tree[t] = {q.x, q.y, q.z, node_word(T(0), id | (axis << 24))};
-    if (heap_order) hash[t - 1] = {(uint32_t)(t - 1), (uint32_t)id};
-    // a run neighbour with the node's coordinate: which of the two becomes
-    // the node is the presort's choice, not necessarily the reference's
-    if (ties) {
-      const T c = coord(q, axis);
-      if ((p > 0 && coord(pos[la[idx - 1]], axis) == c) ||
-          (p + 1 < subtree_size(t, n) && coord(pos[la[idx + 1]], axis) == c))
-        atomicOr(ties, 1);
+__global__ __launch_bounds__(kBlock) void k_tree_count(const int* __restrict__ la, const int* __restrict__ lb,
+                                                        const int* __restrict__ lc, const V4<T>* __restrict__ pos,
+                                                        uint8_t* __restrict__ side, int2* __restrict__ tile_counts,
+                                                        int m, int L, int n, int axis) {
+  __builtin_amdgcn_s_setprio(3);
+  __shared__ int2 s_wave[kBlock / 64];
+  const int* l = blockIdx.y ? lc : lb;
+  side += (size_t)blockIdx.y * n;
+  int nl = 0, nr = 0;
+#pragma unroll
+  for (int r = 0; r < kLevelRounds; ++r) {
+    const int idx = level_place(r);
+    int f = kPlaced;
+    if (idx < m) {
+      const int id = l[idx];
+      const int t = subtree_at(idx, L, n);
+      const int node = la[subtree_start(t, L, n) + subtree_size(2 * t, n)];   // becomes node t
+      if (id != node)
+        f = before(coord(pos[id], axis), id, coord(pos[node], axis), node) ? kLeft : kRight;
+      side[idx] = (uint8_t)f;
     }
-  } else {
-    tag[id] = 2 * t + 1;
-    la_next[idx - placed_before - 1] = id;
+    nl += __popcll(__ballot(f == kLeft));
+    nr += __popcll(__ballot(f == kRight));
+  }
+  if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = make_int2(nl, nr);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int2 c = s_wave[0];
+    for (int w = 1; w < kBlock / 64; ++w) {
+      c.x += s_wave[w].x;
+      c.y += s_wave[w].y;
+    }
+    tile_counts[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = c;
   }
 }
 
-// the other two lists: "goes left" flags for the scan, and where in each list
-// the run's placed particle sits
-__global__ __launch_bounds__(kBlock) void k_tree_flags(const int* __restrict__ lb, const int* __restrict__ lc,
-                                                        const int* __restrict__ tag, int* __restrict__ fb,
-                                                        int* __restrict__ fc, int* __restrict__ at_b,
-                                                        int* __restrict__ at_c, int m, int L) {
-  const int idx = blockIdx.x * kBlock + threadIdx.x;
-  if (idx >= m) return;
-  const int next_level = 2 << L;   // tags of the next level are >= 2^(L+1); a placed particle kept t < that
-  const int tb = tag[lb[idx]], tc = tag[lc[idx]];
-  fb[idx] = tb >= next_level && !(tb & 1);
-  fc[idx] = tc >= next_level && !(tc & 1);
-  if (tb < next_level) at_b[tb] = idx;
-  if (tc < next_level) at_c[tc] = idx;
-}
-
-__device__ __forceinline__ void regroup_one(const int* __restrict__ l, int* __restrict__ l_next,
-                                            const int* __restrict__ sc, const int* __restrict__ at,
-                                            const int* __restrict__ tag, int idx, int L, int n) {
-  const int id = l[idx];
-  const int nt = tag[id];
-  if (nt < (2 << L)) return;   // placed at this level
-  const int t = nt >> 1;
-  const int s = subtree_start(t, L, n);
-  const int base = s - (t - (1 << L));   // where subtree 2t starts in the next layout
-  const int lefts = sc[idx] - sc[s];
-  if (!(nt & 1)) {
-    l_next[base + lefts] = id;
-  } else {
-    const int lt = subtree_size(2 * t, n);
-    const int rights = (idx - s) - lefts - (at[t] < idx ? 1 : 0);
-    l_next[base + lt + rights] = id;
+// level L: the three lists into the next level's layout (blockIdx.y 0: the
+// split axis's, 1, 2: the others), the nodes placed
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_tree_move(const int* __restrict__ la, const int* __restrict__ lb,
+                                                       const int* __restrict__ lc, int* __restrict__ la_next,
+                                                       int* __restrict__ lb_next, int* __restrict__ lc_next,
+                                                       const uint8_t* __restrict__ side,
+                                                       const int2* __restrict__ tile_counts,
+                                                       const V4<T>* __restrict__ pos, V4<T>* __restrict__ tree,
+                                                       KV* __restrict__ hash, int m, int L, int n, int axis,
+                                                       int heap_order, int* __restrict__ ties) {
+  __builtin_amdgcn_s_setprio(3);
+  if (blockIdx.y == 0) {
+#pragma unroll
+    for (int r = 0; r < kLevelRounds; ++r) {
+      const int idx = level_place(r);
+      if (idx >= m) continue;
+      const int id = la[idx];
+      const int t = subtree_at(idx, L, n);
+      const int p = idx - subtree_start(t, L, n), lt = subtree_size(2 * t, n);
+      const int placed_before = t - (1 << L);   // level-L nodes left of t
+      if (p < lt) {
+        la_next[idx - placed_before] = id;
+      } else if (p > lt) {
+        la_next[idx - placed_before - 1] = id;
+      } else {
+        const V4<T> q = pos[id];
+        tree[t] = {q.x, q.y, q.z, node_word(T(0), id | (axis << 24))};
+        if (heap_order) hash[t - 1] = {(uint32_t)(t - 1), (uint32_t)id};
+        // a run neighbour with the node's coordinate: which of the two becomes
+        // the node is the presort's choice, not necessarily the reference's
+        if (ties) {
+          const T c = coord(q, axis);
+          if ((p > 0 && coord(pos[la[idx - 1]], axis) == c) ||
+              (p + 1 < subtree_size(t, n) && coord(pos[la[idx + 1]], axis) == c))
+            atomicOr(ties, 1);
+        }
+      }
+    }
+    return;
   }
-}
-
-__global__ __launch_bounds__(kBlock) void k_tree_regroup(const int* __restrict__ lb, int* __restrict__ lb_next,
-                                                          const int* __restrict__ sb, const int* __restrict__ at_b,
-                                                          const int* __restrict__ lc, int* __restrict__ lc_next,
-                                                          const int* __restrict__ sc, const int* __restrict__ at_c,
-                                                          const int* __restrict__ tag, int m, int L, int n) {
-  const int idx = blockIdx.x * kBlock + threadIdx.x;
-  if (idx >= m) return;
-  regroup_one(lb, lb_next, sb, at_b, tag, idx, L, n);
-  regroup_one(lc, lc_next, sc, at_c, tag, idx, L, n);
+  const int which = blockIdx.y - 1;
+  const int* l = which ? lc : lb;
+  int* next = which ? lc_next : lb_next;
+  side += (size_t)which * n;
+  tile_counts += (size_t)which * gridDim.x;
+  __shared__ int2 s_before[kBlock / 64], s_wave[kBlock / 64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // the tiles before
+  int2 sum = make_int2(0, 0);
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock) {
+    const int2 c = tile_counts[b];
+    sum.x += c.x;
+    sum.y += c.y;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    sum.x += __shfl_xor(sum.x, o);
+    sum.y += __shfl_xor(sum.y, o);
+  }
+  int f[kLevelRounds], lefts[kLevelRounds], rights[kLevelRounds], nl = 0, nr = 0;
+  const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int r = 0; r < kLevelRounds; ++r) {
+    const int idx = level_place(r);
+    f[r] = idx < m ? side[idx] : (int)kPlaced;
+    const unsigned long long ml = __ballot(f[r] == kLeft), mr = __ballot(f[r] == kRight);
+    lefts[r] = nl + __popcll(ml & below);
+    rights[r] = nr + __popcll(mr & below);
+    nl += __popcll(ml);
+    nr += __popcll(mr);
+  }
+  if (lane == 0) {
+    s_before[wave] = sum;
+    s_wave[wave] = make_int2(nl, nr);
+  }
+  __syncthreads();
+  int bl = 0, br = 0;
+  for (int w = 0; w < kBlock / 64; ++w) {
+    bl += s_before[w].x + (w < wave ? s_wave[w].x : 0);
+    br += s_before[w].y + (w < wave ? s_wave[w].y : 0);
+  }
+#pragma unroll
+  for (int r = 0; r < kLevelRounds; ++r) {
+    if (f[r] == kPlaced) continue;
+    const int idx = level_place(r);
+    const int t = subtree_at(idx, L, n);
+    const int start = subtree_start(t, L, n), run = t - (1 << L);   // placed before this run: one per run
+    const int base = start - run;                                    // where subtree 2t starts in the next layout
+    const int lb0 = lefts_before(t, L, n);
+    if (f[r] == kLeft) next[base + bl + lefts[r] - lb0] = l[idx];
+    else next[base + subtree_size(2 * t, n) + br + rights[r] - (base - lb0)] = l[idx];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -259,6 +331,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_tree_lds(const int* __restrict_
                                                       int L0, int cur0, int cur1, int cur2,
                                                       const V4<T>* __restrict__ pos, V4<T>* __restrict__ tree,
                                                       KV* __restrict__ hash, int heap_order, int* __restrict__ ties) {
+  __builtin_amdgcn_s_setprio(3);
   __shared__ uint16_t s_list[3][2][kLdsMax];   // slots, per axis, double-buffered
   __shared__ int s_tag[kLdsMax];               // the heap node each slot's particle belongs to
   __shared__ uint8_t s_fb[kLdsMax], s_fc[kLdsMax];
@@ -305,7 +378,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_tree_lds(const int* __restrict_
       const int slot = s_list[a][cur[a]][i];
       const int t = s_tag[slot];
       const int p = g - subtree_start(t, L, n);
-      const int lt = 2 * t <= n ? subtree_size(2 * t, n) : 0;
+      const int lt = subtree_size(2 * t, n);
       const int pb = t - (1 << L);
       if (p < lt) {
         s_tag[slot] = 2 * t;
@@ -386,40 +459,27 @@ __global__ __launch_bounds__(kLdsThreads) void k_tree_lds(const int* __restrict_
 
 }  // namespace
 
-long tree_work_ints(long n) { return 13 * n + 8; }
+// three lists and their next-level copies, the sides (bytes) and tile counts
+// of two, the slot names of the LDS finish
+static long level_tiles(long n) { return (n + kLevelTile - 1) / kLevelTile; }
+long tree_work_ints(long n) { return 8 * n + 4 * level_tiles(n) + 16; }
 
 template <class T>
 void launch_tree_build(const V4<T>* pos, int n, int n_dev, V4<T>* tree, KV* hash, int heap_order, int* work,
-                       KV* kv, KV* kv_alt, int* sort_scratch, int* scan_scratch, hipStream_t s, int* ties) {
+                       KV* kv, KV* kv_alt, int* sort_scratch, hipStream_t s, int* ties) {
   if (n <= 0 || n > n_dev) throw std::invalid_argument("tree build: need 0 < n <= n_dev");
-  hipLaunchKernelGGL((k_tree_fixed<T>), dim3(ceil_div(n_dev + 2, kBlock)), dim3(kBlock), 0, s, tree, hash, n, n_dev,
-                     heap_order);
+  const long clear = radix_clear_ints(n);
+  hipLaunchKernelGGL((k_tree_fixed<T>), dim3(ceil_div(std::max<long>(n_dev + 2, clear), kBlock)), dim3(kBlock), 0, s,
+                     tree, hash, n, n_dev, heap_order, sort_scratch, (int)clear, radix_scratch_ints(n), ties);
   CS_CHECK_LAUNCH();
   int* list[3][2];
   for (int a = 0; a < 3; ++a)
     for (int k = 0; k < 2; ++k) list[a][k] = work + (size_t)(2 * a + k) * n;
-  // the scans write m + 1 outputs (the total last), so each holds n + 1;
-  // fc and sc lie n + 1 after fb and sb, so one batched scan does both
-  int* tag = work + 6 * (size_t)n;
-  int* fb = work + 7 * (size_t)n;
-  int* fc = fb + (size_t)n + 1;
-  int* sb = work + 9 * (size_t)n + 2;
-  int* sc = sb + (size_t)n + 1;
-  int* at_b = work + 11 * (size_t)n + 4 - 1;   // indexed by heap node 1..n
-  int* at_c = work + 12 * (size_t)n + 4 - 1;
-  // the three presorted lists, sorted side by side (FP64 coordinates: low
-  // key word, then high)
-  const dim3 g3(ceil_div(n, kBlock), 3);
-  hipLaunchKernelGGL((k_tree_keys<T>), g3, dim3(kBlock), 0, s, pos, kv, n, 0, 1);
-  CS_CHECK_LAUNCH();
-  launch_radix_sort_batch(kv, kv_alt, n, 32, sort_scratch, s, 3, n);
-  if (sizeof(T) == 8) {
-    hipLaunchKernelGGL((k_tree_keys<T>), g3, dim3(kBlock), 0, s, pos, kv, n, 1, 0);
-    CS_CHECK_LAUNCH();
-    launch_radix_sort_batch(kv, kv_alt, n, 32, sort_scratch, s, 3, n);
-  }
-  hipLaunchKernelGGL(k_tree_ids, g3, dim3(kBlock), 0, s, kv, list[0][0], tag, n);
-  CS_CHECK_LAUNCH();
+  int* slot_of = work + 6 * (size_t)n;
+  // (16-byte steps: int2 counts, then the bytes)
+  int2* tile_counts = reinterpret_cast<int2*>(work + ((7 * (size_t)n + 3) & ~(size_t)3));
+  uint8_t* side = reinterpret_cast<uint8_t*>(tile_counts + 2 * level_tiles(n));
+  launch_axis_sorts<T>(pos, n, kv, kv_alt, list[0][0], 2l * n, sort_scratch, s);
   int cur[3] = {0, 0, 0};
   int m = n;
   // level kernels while the level's subtrees hold more than kLdsMax
@@ -427,28 +487,21 @@ void launch_tree_build(const V4<T>* pos, int n, int n_dev, V4<T>* tree, KV* hash
   int L_lds = 0;
   while (subtree_size(1 << L_lds, n) > kLdsMax) ++L_lds;
   for (int L = 0; m > 0 && L < L_lds; ++L) {
-    const int a = L % 3, b = (L + 1) % 3, c = (L + 2) % 3;
-    const dim3 gm(ceil_div(m, kBlock));
-    hipLaunchKernelGGL((k_tree_split<T>), gm, dim3(kBlock), 0, s, list[a][cur[a]], list[a][cur[a] ^ 1], tag, pos,
-                       tree, hash, m, L, n, a, heap_order, ties);
+    const int a = L % 3, b = (L + 1) % 3, c = (L + 2) % 3, tiles = (int)level_tiles(m);
+    hipLaunchKernelGGL((k_tree_count<T>), dim3(tiles, 2), dim3(kBlock), 0, s, list[a][cur[a]], list[b][cur[b]],
+                       list[c][cur[c]], pos, side, tile_counts, m, L, n, a);
     CS_CHECK_LAUNCH();
-    const int placed = (int)std::min<long>(1l << L, (long)n - ((1l << L) - 1));
-    if (m - placed > 0) {
-      hipLaunchKernelGGL(k_tree_flags, gm, dim3(kBlock), 0, s, list[b][cur[b]], list[c][cur[c]], tag, fb, fc, at_b,
-                         at_c, m, L);
-      CS_CHECK_LAUNCH();
-      launch_exclusive_scan_pair(fb, sb, m, (long)n + 1, scan_scratch, s);
-      hipLaunchKernelGGL(k_tree_regroup, gm, dim3(kBlock), 0, s, list[b][cur[b]], list[b][cur[b] ^ 1], sb, at_b,
-                         list[c][cur[c]], list[c][cur[c] ^ 1], sc, at_c, tag, m, L, n);
-      CS_CHECK_LAUNCH();
-    }
+    hipLaunchKernelGGL((k_tree_move<T>), dim3(tiles, 3), dim3(kBlock), 0, s, list[a][cur[a]], list[b][cur[b]],
+                       list[c][cur[c]], list[a][cur[a] ^ 1], list[b][cur[b] ^ 1], list[c][cur[c] ^ 1], side,
+                       tile_counts, pos, tree, hash, m, L, n, a, heap_order, ties);
+    CS_CHECK_LAUNCH();
     for (int k = 0; k < 3; ++k) cur[k] ^= 1;
-    m -= placed;
+    m -= (int)std::min<long>(1l << L, (long)n - ((1l << L) - 1));
   }
   if (m > 0) {
     const int roots = (int)std::min<long>(1l << L_lds, (long)n - (1l << L_lds) + 1);
-    hipLaunchKernelGGL((k_tree_lds<T>), dim3(roots), dim3(kLdsThreads), 0, s, work, tag, n, L_lds, cur[0], cur[1], cur[2],
-                       pos, tree, hash, heap_order, ties);
+    hipLaunchKernelGGL((k_tree_lds<T>), dim3(roots), dim3(kLdsThreads), 0, s, work, slot_of, n, L_lds, cur[0], cur[1],
+                       cur[2], pos, tree, hash, heap_order, ties);
     CS_CHECK_LAUNCH();
   }
 }
@@ -546,10 +599,8 @@ void launch_tree_boxes(const V4<T>* tree, F4* box, int n_nodes, int fix_phantom,
   }
 }
 
-template void launch_tree_build<float>(const F4*, int, int, F4*, KV*, int, int*, KV*, KV*, int*, int*, hipStream_t,
-                                       int*);
-template void launch_tree_build<double>(const D4*, int, int, D4*, KV*, int, int*, KV*, KV*, int*, int*, hipStream_t,
-                                        int*);
+template void launch_tree_build<float>(const F4*, int, int, F4*, KV*, int, int*, KV*, KV*, int*, hipStream_t, int*);
+template void launch_tree_build<double>(const D4*, int, int, D4*, KV*, int, int*, KV*, KV*, int*, hipStream_t, int*);
 template void launch_tree_boxes<float>(const F4*, F4*, int, int, hipStream_t);
 template void launch_tree_boxes<double>(const D4*, F4*, int, int, hipStream_t);
 

@@ -1,0 +1,31 @@
+"""The look-back radix sort (csrc/sort.hip) around its tile of 4096 records
+and with few distinct digits, against numpy's stable sort bit for bit."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 4095, 4096, 4097, 8192, 12289, 300001])
+@pytest.mark.parametrize("bits", [3, 8, 16, 24, 32])
+@pytest.mark.parametrize("kind", ["random", "equal", "descending"])
+def test_sort_around_tiles(cs, n, bits, kind):
+    print(f"sort n={n} bits={bits} {kind}", flush=True)
+    import torch
+    rng = np.random.default_rng(n + bits)
+    top = 1 << bits
+    keys = {"random": rng.integers(0, top, n, dtype=np.uint64), "equal": np.full(n, top - 1, np.uint64),
+            "descending": np.sort(rng.integers(0, top, n, dtype=np.uint64))[::-1]}[kind].astype(np.uint32)
+    kv = np.stack([keys, np.arange(n, dtype=np.uint32)], 1)
+    data = torch.from_numpy(kv.astype(np.int64).astype(np.uint32).view(np.int32).copy()).cuda()
+    alt = torch.zeros_like(data)
+    L = cs.lib()
+    L.sph_radix_sort_noalloc.argtypes = [C.c_void_p, C.c_void_p, C.c_uint, C.c_uint, C.c_void_p]
+    L.sph_radix_sort_noalloc.restype = C.c_int
+    for _ in range(2):   # sorted input the second time
+        assert L.sph_radix_sort_noalloc(data.data_ptr(), alt.data_ptr(), n, bits,
+                                        torch.cuda.current_stream().cuda_stream) == 0
+        got = data.cpu().numpy().view(np.uint32)
+        assert np.array_equal(got, kv[np.argsort(keys, kind="stable")])
