@@ -98,8 +98,8 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
   tree_.alloc(nd_ + 2);
   ties_.alloc(1);
   boxes_.alloc(2 * ((size_t)nd_ + 2));
-  if (!kF32) {   // the larger of the forward and reverse passes' splits
-    const int parts = std::max(gravity64_parts(nd_), gravity64_forward_parts(nd_));
+  if (!kF32) {
+    const int parts = gravity64_parts(nd_);
     if (parts > 1) gpart64_.alloc((size_t)parts * nd_);
   }
   hash_.alloc(nd_);
@@ -269,8 +269,8 @@ double Engine<T>::get_scalar(const std::string& name) {
   if (name == "grav_sums") return grav_sums_;
   if (name == "grav_parts") return grav_parts_;
   if (name == "grav_parts_auto") {   // the j-parts the automatic choice takes at this size
-    if (!kF32) return gravity64_forward_parts(nd_);
-    return mixed() ? gravity_mixed_parts(nd_, grav_far_) : 1;
+    if (!kF32) return gravity64_parts(nd_);
+    return mixed() ? kGravMixedParts : 1;
   }
   if (name == "solve_cache") return solve_cache_;
   if (name == "adj_free_ranges") return adj_free_ranges_;
@@ -698,7 +698,7 @@ void Engine<T>::gravity_kernels(hipStream_t gs) {
   }
   if constexpr (!kF32) {
     if (p_.grav_mode == 1) {
-      const int parts = grav_parts_ ? grav_parts_ : gravity64_forward_parts(nd_);
+      const int parts = grav_parts_ ? grav_parts_ : gravity64_parts(nd_);
       if (parts > 1 && gpart64_.n < (size_t)parts * nd_) gpart64_.alloc((size_t)parts * nd_);
       launch_gravity64_plummer(gpos_, grav_, gpart64_.p, nd_, nd_, (double)p_.grav_eps, gs, parts);
       return;

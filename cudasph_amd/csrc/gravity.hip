@@ -208,7 +208,7 @@ __device__ __forceinline__ void pair_plummer(A&& a, T rx, T ry, T rz, T mj, T ep
 constexpr int kGravBlock = 256;
 constexpr int kTile = 64;        // j per blocked-compensation partial (mixed form)
 constexpr int kJTile = 512;      // j records staged in LDS per block iteration (reference-layout kernels)
-constexpr int kGravParts = 8;    // j-parts of the mixed Plummer kernel, one per XCD (at most)
+constexpr int kGravParts = kGravMixedParts;
 // j records per LDS tile of the mixed Plummer kernel: one 64-record sub-tile
 // per wavefront.  Its 12 KB of LDS lets 8 blocks share a CU (the kernel's 63
 // VGPRs allow 8 waves per SIMD), so the 4096 x 8 blocks at N = 2^20 run in
@@ -937,8 +937,9 @@ __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx,
 // (4 MiB of hi+lo records at N = 2^20), which its L2 holds; without the
 // split every XCD streams the whole j-set and re-fetches it from HBM.  Each
 // block writes its compensated (hi, lo) partial sums; k_gravity_combine adds
-// the parts in order.  (gravity_mixed_parts picks fewer parts where 8 would
-// fill most of the GPU's block slots in one round.)
+// the parts in order.  (Fewer parts leave the SPH passes beside gravity more
+// room but lengthen it: mixed step, 4 / 6 / 8 parts, 65 536 particles 2.30 /
+// 2.31 / 2.04 ms, 50 000: 1.57 / 1.44 / 1.40, 40 000: 1.20 / 1.02 / 1.00.)
 // The far-field instantiation holds the 48 moment words of an expansion in
 // VGPRs next to the pairwise state: left alone the compiler takes 127
 // registers (4 wavefronts per SIMD); capped at 5 wavefronts it fits 96
@@ -1346,12 +1347,13 @@ __global__ __launch_bounds__(kGravBlock) void k_gravity_mixed_spline(const F4* _
 // ---------------------------------------------------------------------------
 // FP64 form, Plummer softening.  The pair body in fused multiply-adds (the
 // FP64 form has no bit contract with the reference's FP32 arithmetic):
-// 3 sub, 3 FMA for s^2 = r^2 + eps^2, v_rsq_f64 and two Newton steps
-// (y <- y (1.5 - (s^2/2) y^2), 3 operations each after s^2/2), 3 for
-// m/s^3, 3 FMA into the acceleration and one into the potential.  With few
-// i-blocks (N below 2^19) the j-range is split into parts, one block per
-// (i-block, part), so that the GPU holds enough wavefronts to hide the FP64
-// latencies; the parts' sums are added in part order (deterministic).
+// 3 sub, 3 FMA for s^2 = r^2 + eps^2, v_rsq_f64 refined by one third-order
+// step (y0 (1 + e (1/2 + 3/8 e)), e = 1 - s^2 y0^2: 5 operations, its remainder
+// 5/16 e^3 below one rounding), 3 for m/s^3, 3 FMA into the acceleration and one
+// into the potential.  With few i-blocks (N below 2^19) the j-range is split
+// into parts, one block per (i-block, part), so that the GPU holds enough
+// wavefronts to hide the FP64 latencies; the parts' sums are added in part
+// order (deterministic).
 constexpr int kG64Tile = kGravBlock;
 __global__ __launch_bounds__(kGravBlock) void k_gravity64_plummer(const D4* __restrict__ gpos, D4* __restrict__ out,
                                                                    int n_i, int n_j, int parts, int chunk,
@@ -1371,10 +1373,9 @@ __global__ __launch_bounds__(kGravBlock) void k_gravity64_plummer(const D4* __re
       const D4 pj = s_pos[j];
       const double rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
       const double d2 = __builtin_fma(rx, rx, __builtin_fma(ry, ry, __builtin_fma(rz, rz, eps2)));
-      const double h = 0.5 * d2;
-      double y = __builtin_amdgcn_rsq(d2);
-      y = y * __builtin_fma(-h, y * y, 1.5);
-      y = y * __builtin_fma(-h, y * y, 1.5);
+      const double y0 = __builtin_amdgcn_rsq(d2);
+      const double e = __builtin_fma(-(d2 * y0), y0, 1.0);
+      const double y = __builtin_fma(__builtin_fma(e, 0.375, 0.5), y0 * e, y0);
       const double my = pj.w * y;
       const double s3 = my * (y * y);
       ax = __builtin_fma(-rx, s3, ax);
@@ -1399,29 +1400,28 @@ __global__ __launch_bounds__(kBlock) void k_gravity64_combine(const D4* __restri
   out[i] = a;
 }
 
+// Parts for the passes of the FP64 form: of 2 .. 8 (1 from 2^19 particles on)
+// the count whose blocks fill the CUs most evenly, the larger of equals.
+// Every block is resident at once and takes the same time, so a pass lasts as
+// long as its fullest CU.  FP64 step, 2 / 4 / 6 / 8 parts, ms: 50 021 particles
+// (196 i-blocks on 256 CUs) 3.00 / 2.77 / 2.30 / 2.47, 65 536: 4.30 / 3.65 / 4.02 / 3.55,
+// 131 072: 14.6 / 13.7 / 13.2 / 13.3.
 int gravity64_parts(int n_i) {
   const int blocks = ceil_div(n_i, kGravBlock);
-  return std::max(1, std::min(8, ceil_div(2048, blocks)));
-}
-
-// The forward pass runs beside the FP64 SPH passes.  With no more i-blocks
-// than CUs it takes parts for two blocks per CU, leaving the passes the rest
-// of each CU; otherwise the reverse pass's split.  Measured, FP64 step /
-// gravity alone: 65 536 particles, 8 parts 5.51 / 3.54 ms, 3 parts 5.04 /
-// 3.67, 2 parts 4.71 / 3.81; 262 144 particles, 2 parts 50.6 / 50.9 ms,
-// 1 part 70.2 / 54.1 (there the passes beside a half-empty grid slow it).
-int gravity64_forward_parts(int n_i) {
+  if (blocks >= 2048) return 1;
   int dev = 0, cus = 0;
   CS_HIP(hipGetDevice(&dev));
   CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int blocks = ceil_div(n_i, kGravBlock);
-  if (blocks > cus) return gravity64_parts(n_i);
-  return std::max(1, std::min(8, ceil_div(2 * cus, blocks)));
+  int best = 8;
+  for (int p = 7; p >= 2 && (long)p * blocks >= 4l * cus; --p)   // fewer: too few wavefronts per SIMD
+    // fullest CU's blocks per unit of work: ceil(p blocks / cus) / p
+    if ((long)ceil_div((long)p * blocks, cus) * best < (long)ceil_div((long)best * blocks, cus) * p) best = p;
+  return best;
 }
 
 void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_j, double eps, hipStream_t s,
                               int parts) {
-  if (parts <= 0) parts = gravity64_forward_parts(n_i);
+  if (parts <= 0) parts = gravity64_parts(n_i);
   if (parts > 8) throw std::invalid_argument("gravity: at most 8 j-parts");
   const int chunk = ceil_div(ceil_div(n_j, parts), kG64Tile) * kG64Tile;
   hipLaunchKernelGGL(k_gravity64_plummer, dim3(ceil_div(n_i, kGravBlock) * parts), dim3(kGravBlock), 0, s, gpos,
@@ -1469,27 +1469,6 @@ void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, i
   CS_CHECK_LAUNCH();
 }
 
-// j-parts of the pairwise mixed kernel: 8, one per XCD, unless the 8-part
-// grid would take more than half of the GPU's block slots (8 blocks of
-// 63-register wavefronts per CU) in a single round.  Such a grid holds the
-// CUs until gravity ends and the latency-bound SPH passes queued beside it
-// find no slot; with fewer parts gravity keeps about half of each SIMD's 8
-// wavefront slots, which still fill its VALU, and the passes run in the rest
-// (their walks at the higher issue priority).  Mixed step at 65 536
-// particles (256 i-blocks): 8 parts 3.21 ms, 4 parts 2.19, 3 parts 2.39
-// (gravity alone 2.03 / 2.07 / 2.22 ms).  Grids of several rounds keep 8
-// (262 144 particles: 8 parts 22.6 ms/step, 2 parts 25.0, 1 part 28.0).  The
-// far-field kernel keeps 8.
-int gravity_mixed_parts(int n_i, int far) {
-  if (far) return kGravParts;
-  int dev = 0, cus = 0;
-  CS_HIP(hipGetDevice(&dev));
-  CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const long slots = 8l * cus, blocks = (long)ceil_div(n_i, kGravBlock);
-  if (blocks * kGravParts <= slots / 2 || blocks * kGravParts > slots) return kGravParts;
-  return (int)std::max(1l, slots / 2 / blocks);
-}
-
 void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F4* part, float* mass_range,
                           float* moments, float far_ratio, float far_grade, int n_i, int n_j, int n_real,
                           int soft, float eps, int split_only, hipStream_t s, int parts) {
@@ -1504,7 +1483,7 @@ void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F
     hipLaunchKernelGGL(k_mass_range_final, dim3(1), dim3(kBlock), 0, s, mass_range + 2, nb, mass_range);
     CS_CHECK_LAUNCH();
     const bool far = (split_only & 16) && moments;
-    if (parts <= 0 || far) parts = gravity_mixed_parts(n_i, far);
+    if (parts <= 0 || far) parts = kGravParts;
     if (parts > kGravParts) throw std::invalid_argument("gravity: at most 8 j-parts");
     const int chunk = ceil_div(ceil_div(n_j, parts), kTile) * kTile;
     F4* part_hi = part;

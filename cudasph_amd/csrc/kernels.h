@@ -65,12 +65,9 @@ template <class T>
 void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, int n_j, int soft, T eps,
                     int exact, hipStream_t s, int sums = -1);
 // FP64 form, Plummer softening (fused pair body; the j-range split into
-// `parts` parts, 0 for gravity64_forward_parts(n_i), `part` then holding
-// parts * n_i records when parts > 1).  gravity64_parts(n_i) is the
-// reverse pass's split: enough parts to fill the GPU when the i-blocks alone
-// would not.
+// `parts` parts, 0 for gravity64_parts(n_i), `part` then holding parts * n_i
+// records when parts > 1).  gravity64_parts: also the reverse pass's split.
 int gravity64_parts(int n_i);
-int gravity64_forward_parts(int n_i);
 void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_j, double eps, hipStream_t s,
                               int parts = 0);
 // part: scratch of 2 * 8 * n_i records (per-j-part partial sums, Plummer only);
@@ -82,8 +79,8 @@ void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_
 // field, split_only bit 4, taken where every lane of a wavefront is
 // far_ratio radii away, the ratio at a level of C records scaled by
 // (C / 16384)^far_grade; may be null otherwise)
-// parts: the number of j-parts (1..8), 0 for gravity_mixed_parts(n_i, far)
-int gravity_mixed_parts(int n_i, int far);
+// parts: the number of j-parts, 1 .. kGravMixedParts; 0 for the most
+constexpr int kGravMixedParts = 8;   // one per XCD
 void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F4* part, float* mass_range,
                           float* moments, float far_ratio, float far_grade, int n_i, int n_j, int n_real,
                           int soft, float eps, int split_only, hipStream_t s, int parts = 0);
