@@ -230,14 +230,14 @@ __global__ __launch_bounds__(kBlock) void k_adj_hydro(const D4v* __restrict__ po
 // j-side sums: for each j, the slots whose neighbour is j, in ascending slot
 // order (the forward's sorted pairs); ncomp = 10 after hydro, 6 after density
 __global__ __launch_bounds__(kBlock) void k_adj_gather(const KV* __restrict__ pairs, const int* __restrict__ start,
-                                                        const int* __restrict__ end, const double* __restrict__ pb,
+                                                        const double* __restrict__ pb,
                                                         D4v* __restrict__ xs, D4v* __restrict__ vs,
                                                         D4v* __restrict__ hb1, D4v* __restrict__ hb2, int n,
                                                         int ncomp) {
   const int j = blockIdx.x * kBlock + threadIdx.x;
   if (j >= n) return;
   double s[kPair] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int p = start[j]; p < end[j]; ++p) {
+  for (int p = start[j], p1 = start[j + 1]; p < p1; ++p) {
     const double* r = pb + (size_t)pairs[p].value * kPair;
     for (int c = 0; c < kPair; ++c)
       if (c < ncomp) s[c] += r[c];
@@ -673,13 +673,12 @@ __global__ __launch_bounds__(kBlock) void k_adj_range_hydro(const D4v* __restric
 // rbar[j] += the j-side parts of the slots naming j (ascending slot order)
 __global__ __launch_bounds__(kBlock) void k_adj_range_gather(const KV* __restrict__ pairs,
                                                              const int* __restrict__ start,
-                                                             const int* __restrict__ end,
                                                              const double* __restrict__ pb,
                                                              double* __restrict__ rbar, int n) {
   const int j = blockIdx.x * kBlock + threadIdx.x;
   if (j >= n) return;
   double s = 0.0;
-  for (int p = start[j]; p < end[j]; ++p) s += pb[(size_t)pairs[p].value * kPair];
+  for (int p = start[j], p1 = start[j + 1]; p < p1; ++p) s += pb[(size_t)pairs[p].value * kPair];
   rbar[j] += s;
 }
 
@@ -838,8 +837,7 @@ void Engine<T>::adj_capture(EvalSlot& e) {
   grow(e.dots, nd);
   grow(e.off, nd + 1);
   grow(e.cnt, nd);
-  grow(e.tr_start, nd);
-  grow(e.tr_end, nd);
+  grow(e.tr_start, nd + 1);
   grow(e.list, std::max<size_t>(tot, 1));
   grow(e.pairs, std::max<size_t>(tot, 1));
   d2d(e.pos.p, pos_.p, nd, s_);
@@ -848,8 +846,7 @@ void Engine<T>::adj_capture(EvalSlot& e) {
   d2d(e.dots.p, dots_.p, nd, s_);
   d2d(e.off.p, ngb_offset_.p, nd + 1, s_);
   d2d(e.cnt.p, ngb_count_.p, nd, s_);
-  d2d(e.tr_start.p, tr_start_.p, nd, s_);
-  d2d(e.tr_end.p, tr_end_.p, nd, s_);
+  d2d(e.tr_start.p, tr_start_.p, nd + 1, s_);
   d2d(e.list.p, list_.p, tot, s_);
   d2d(e.pairs.p, pairs_.p, tot, s_);
   e.tot = ngb_tot_;
@@ -864,8 +861,7 @@ void Engine<T>::adj_restore(const EvalSlot& e) {
   d2d(dots_.p, e.dots.p, nd, s_);
   d2d(ngb_offset_.p, e.off.p, nd + 1, s_);
   d2d(ngb_count_.p, e.cnt.p, nd, s_);
-  d2d(tr_start_.p, e.tr_start.p, nd, s_);
-  d2d(tr_end_.p, e.tr_end.p, nd, s_);
+  d2d(tr_start_.p, e.tr_start.p, nd + 1, s_);
   d2d(list_.p, e.list.p, tot, s_);
   d2d(pairs_.p, e.pairs.p, tot, s_);
   ngb_tot_ = e.tot;
@@ -919,7 +915,7 @@ void Engine<T>::adj_forces_backward(bool seed_rho) {
                        ngb_offset_.p, ngb_count_.p, list_.p, xs_.p, vs_.p, hb1_.p, hb2_.p, pairbuf_.p, n_,
                        (double)p_.av_alpha, (double)p_.av_beta);
     CS_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_adj_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, tr_end_.p, pairbuf_.p,
+    hipLaunchKernelGGL(k_adj_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, pairbuf_.p,
                        xs_.p, vs_.p, hb1_.p, hb2_.p, n_, kPair);
     CS_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_adj_eos, grid(n_), dim3(kBlock), 0, s_, hydro_.p, hb1_.p, n_, eos_const(),
@@ -928,7 +924,7 @@ void Engine<T>::adj_forces_backward(bool seed_rho) {
     hipLaunchKernelGGL(k_adj_density, grid(n_), dim3(kBlock), 0, s_, pos_.p, vel_.p, hydro_.p, dots_.p, hb1_.p,
                        hb2_.p, ngb_offset_.p, ngb_count_.p, list_.p, xs_.p, vs_.p, pairbuf_.p, n_);
     CS_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_adj_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, tr_end_.p, pairbuf_.p,
+    hipLaunchKernelGGL(k_adj_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, pairbuf_.p,
                        xs_.p, vs_.p, hb1_.p, hb2_.p, n_, 6);
     CS_CHECK_LAUNCH();
     if (adj_implicit_h_) {   // the ranges' dependence on the positions (the h-solve)
@@ -937,13 +933,13 @@ void Engine<T>::adj_forces_backward(bool seed_rho) {
                          ngb_offset_.p, ngb_count_.p, list_.p, adj_rbar_.p, pairbuf_.p, n_, (double)p_.av_alpha,
                          (double)p_.av_beta);
       CS_CHECK_LAUNCH();
-      hipLaunchKernelGGL(k_adj_range_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, tr_end_.p,
+      hipLaunchKernelGGL(k_adj_range_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p,
                          pairbuf_.p, adj_rbar_.p, n_);
       CS_CHECK_LAUNCH();
       hipLaunchKernelGGL(k_adj_range_density, grid(n_), dim3(kBlock), 0, s_, pos_.p, vel_.p, hydro_.p, dots_.p,
                          hb1_.p, hb2_.p, ngb_offset_.p, ngb_count_.p, list_.p, adj_rbar_.p, xs_.p, pairbuf_.p, n_);
       CS_CHECK_LAUNCH();
-      hipLaunchKernelGGL(k_adj_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, tr_end_.p, pairbuf_.p,
+      hipLaunchKernelGGL(k_adj_gather, grid(n_), dim3(kBlock), 0, s_, pairs_.p, tr_start_.p, pairbuf_.p,
                          xs_.p, vs_.p, hb1_.p, hb2_.p, n_, 3);
       CS_CHECK_LAUNCH();
     }

@@ -108,21 +108,19 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
   ngb_count_.alloc(nd_);
   ngb_offset_.alloc(nd_ + 1);
   list_.alloc(cap_);
-  owner_.alloc(nd_);   // per-j counts of the reaction transpose
+  owner_.alloc(nd_);   // per-j counts of the reaction transpose (zero between them)
   acc_.alloc(cap_);
   pairs_.alloc(cap_);
   pairs_alt_.alloc(cap_);
   tr_start_.alloc(nd_ + 1);
-  tr_end_.alloc(nd_ + 1);
   flags_.alloc(4);
   scan_tmp_.alloc(scan_scratch_ints(std::max<long>(cap_, nd_ + 1)) + 16);
   sort_tmp_.alloc(3 * radix_scratch_ints(nd_));   // three axes' sorts side by side
   dt_cur_.alloc(1);
   dt_next_.alloc(1);
-  partials_.alloc(reduce_partials(nd_) + 64);
+  partials_.alloc(reduce_partials(nd_));
   force6_.alloc(6);
   stats6_.alloc(6);
-  diag_part_.alloc(diag_partials(n_));
   diag_.alloc(19);
   key_hi_.alloc(nd_);
   key_lo_.alloc(nd_);
@@ -153,7 +151,7 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
 
   for (auto* b : {&pos_, &vel_, &hydro_, &dots_, &bdots_, &hydro2_, &grav_, &gpos_, &gvel_, &old_vu_})
     CS_HIP(hipMemsetAsync(b->p, 0, b->bytes(), s_));
-  for (auto* b : {&n_ngb_, &ngb_count_, &ngb_offset_, &tr_start_, &tr_end_, &flags_})
+  for (auto* b : {&n_ngb_, &ngb_count_, &ngb_offset_, &tr_start_, &owner_, &flags_})
     CS_HIP(hipMemsetAsync(b->p, 0, b->bytes(), s_));
   CS_HIP(hipMemsetAsync(dt_cur_, 0, 8, s_));
   CS_HIP(hipMemsetAsync(dt_next_, 0, 8, s_));
@@ -600,8 +598,8 @@ void Engine<T>::hydro() {
 template <class T>
 void Engine<T>::build_transpose() {
   if (tot_stale_) check_total();
-  launch_reaction_transpose(ngb_offset_, ngb_count_, list_, nd_, owner_, tr_start_, tr_end_, pairs_, pairs_alt_,
-                            scan_tmp_, s_);
+  launch_reaction_transpose(ngb_offset_, ngb_count_, list_, nd_, owner_, tr_start_, pairs_, pairs_alt_, scan_tmp_,
+                            s_);
 }
 
 template <class T>
@@ -610,11 +608,11 @@ void Engine<T>::reaction() {
   build_transpose();
   if constexpr (kF32) {
     if (mixed()) {
-      launch_reaction_mixed(pos_, pos_lo_, bdots_, acc_, pairs_, tr_start_, tr_end_, n_, s_);
+      launch_reaction_mixed(pos_, pos_lo_, bdots_, acc_, pairs_, tr_start_, n_, s_);
       return;
     }
   }
-  launch_reaction<T>(pos_, bdots_, acc_, pairs_, tr_start_, tr_end_, n_, s_);
+  launch_reaction<T>(pos_, bdots_, acc_, pairs_, tr_start_, n_, s_);
 }
 
 template <class T>
@@ -707,34 +705,47 @@ void Engine<T>::gravity_kernels(hipStream_t gs) {
   launch_gravity<T>(gpos_, gvel_, grav_, nd_, nd_, p_.grav_mode, T(p_.grav_eps), exact_rsqrt_, gs, grav_sums_);
 }
 
+// add_gravity, the statistics and the timestep (to dt_out), as `what` asks
 template <class T>
-void Engine<T>::add_gravity() {
-  launch_add_gravity<T>(bdots_, grav_, pos_, vel_, n_, partials_, force6_, s_);
+void Engine<T>::step_end(int what, double* dt_out) {
+  StepEnd<T> e{bdots_, grav_, pos_, vel_, hydro_, hydro2_, nullptr, nullptr, nullptr, n_ngb_, ngb_count_, n_,
+               p_.cn_vel, p_.cn_eth, partials_};
+  if (mixed()) {
+    e.pos64 = pos64_;
+    e.vel64 = vel64_;
+    e.u64 = u64_;
+  }
+  launch_step_end<T>(e, what, kF32 && !mixed(), force6_, stats6_, diag_, dt_out, s_);
+}
+
+// ends a step's force evaluation: gravity added, statistics, next timestep
+template <class T>
+void Engine<T>::finish(double* dt_out) {
+  if (adj_mode_ >= kAdjReplay) {   // the recorded timestep of this evaluation
+    step_end(kAddGravity | kStatistics, nullptr);
+    timestep(dt_out);
+    return;
+  }
+  step_end(kAddGravity | kStatistics | kTimestep, dt_out);
+  record_timestep(dt_out);
 }
 
 template <class T>
 void Engine<T>::timestep(double* out) {
-  if (adj_mode_ >= kAdjReplay) {   // the recorded timestep of this evaluation
+  if (adj_mode_ >= kAdjReplay) {
     CS_HIP(hipMemcpyAsync(out, &adj_dt_[adj_f_], 8, hipMemcpyHostToDevice, s_));
     sync();
     return;
   }
-  timestep_compute(out);
-  if (adj_mode_ == kAdjRecord) {
-    sync();
-    CS_HIP(hipMemcpy(&adj_dt_[adj_f_], out, 8, hipMemcpyDeviceToHost));
-  }
+  step_end(kTimestep, out);
+  record_timestep(out);
 }
 
 template <class T>
-void Engine<T>::timestep_compute(double* out) {
-  if constexpr (kF32) {
-    if (mixed()) {
-      launch_timestep_mixed(pos_, u64_, hydro2_, bdots_, n_, p_.cn_vel, p_.cn_eth, partials_, out, s_);
-      return;
-    }
-  }
-  launch_timestep<T>(pos_, hydro_, hydro2_, bdots_, n_, p_.cn_vel, p_.cn_eth, kF32 ? 1 : 0, partials_, out, s_);
+void Engine<T>::record_timestep(const double* dt) {
+  if (adj_mode_ != kAdjRecord) return;
+  sync();
+  CS_HIP(hipMemcpy(&adj_dt_[adj_f_], dt, 8, hipMemcpyDeviceToHost));
 }
 
 template <class T>
@@ -758,19 +769,6 @@ void Engine<T>::correct(const double* dt_new, const double* dt_old) {
     }
   }
   launch_correct<T>(vel_, hydro_, bdots_, old_vu_, dt_new, dt_old, n_, s_);
-}
-
-template <class T>
-void Engine<T>::stats_pass() {
-  if constexpr (kF32) {
-    if (mixed()) {
-      launch_stats_mixed(pos64_, vel64_, u64_, grav_, n_, partials_, stats6_, s_);
-      launch_diagnostics<double>(pos64_, vel64_, n_ngb_, ngb_count_, n_, diag_part_, diag_, s_);
-      return;
-    }
-  }
-  launch_stats<T>(pos_, vel_, hydro_, grav_, n_, partials_, stats6_, s_);
-  launch_diagnostics<T>(pos_, vel_, n_ngb_, ngb_count_, n_, diag_part_, diag_, s_);
 }
 
 // sort_bodies.cpp:119-186 on the GPU: 3*bits-bit Peano-Hilbert keys sorted
@@ -821,9 +819,7 @@ void Engine<T>::init() {
   adj_f_ = 0;
   sph_accelerations();
   gravity();
-  add_gravity();
-  stats_pass();
-  timestep(dt_cur_);
+  finish(dt_cur_);
 }
 
 // step.cpp:13-147
@@ -859,12 +855,10 @@ void Engine<T>::step() {
   if (adj_capture_ >= 0) adj_capture(*adj_eval_[adj_capture_]);
   if (!grav_first) gravity(false);
   gravity_join();
-  add_gravity();
   global_time_ += dt_;
-  stats_pass();
-  timestep(dt_next_);
+  finish(dt_next_);
   correct(dt_next_, dt_cur_);
-  CS_HIP(hipMemcpyAsync(dt_cur_, dt_next_, 8, hipMemcpyDeviceToDevice, s_));
+  std::swap(dt_cur_.p, dt_next_.p);
 }
 
 template <class T>
@@ -879,11 +873,11 @@ void Engine<T>::pass(int id) {
     case SPH_HYDRO: hydro(); break;
     case SPH_REACTION: reaction(); break;
     case SPH_GRAVITY: gravity(); break;
-    case SPH_ADD_GRAVITY: add_gravity(); break;
+    case SPH_ADD_GRAVITY: step_end(kAddGravity, nullptr); break;
     case SPH_TIMESTEP: timestep(dt_cur_); break;
     case SPH_PREDICT: predict(); break;
     case SPH_CORRECT: correct(dt_cur_, dt_cur_); break;
-    case SPH_STATS: stats_pass(); break;
+    case SPH_STATS: step_end(kStatistics, nullptr); break;
     case SPH_PH_SORT: sort_bodies(); break;
     case SPH_SPH_ACC: sph_accelerations(); break;
     case SPH_INIT: init(); break;

@@ -109,12 +109,12 @@ class Engine final : public EngineBase {
   void gravity_join();
   void gravity_pack();
   void gravity_kernels(hipStream_t gs);
-  void add_gravity();
+  void step_end(int what, double* dt_out);
+  void finish(double* dt_out);
   void timestep(double* out);
-  void timestep_compute(double* out);
+  void record_timestep(const double* dt);
   void predict();
   void correct(const double* dt_new, const double* dt_old);
-  void stats_pass();
   void sort_bodies();
   void init();
   void step();
@@ -146,7 +146,7 @@ class Engine final : public EngineBase {
   // recomputation: state at the evaluation, lists and their transpose
   struct EvalSlot {
     DBuf<V4<T>> pos, vel, hyd, dots;
-    DBuf<int> off, cnt, list, tr_start, tr_end;
+    DBuf<int> off, cnt, list, tr_start;
     DBuf<KV> pairs;
     long tot = 0;
   };
@@ -182,10 +182,10 @@ class Engine final : public EngineBase {
 
   DBuf<V4<T>> pos_, vel_, hydro_, dots_, bdots_, hydro2_, grav_, tree_, gpos_, gvel_, old_vu_, tmp4_;
   DBuf<KV> hash_, pairs_, pairs_alt_, perm_;
-  DBuf<int> n_ngb_, ngb_count_, ngb_offset_, list_, owner_, tr_start_, tr_end_, flags_, scan_tmp_, sort_tmp_;
+  DBuf<int> n_ngb_, ngb_count_, ngb_offset_, list_, owner_, tr_start_, flags_, scan_tmp_, sort_tmp_;
   DBuf<T> acc_;
   DBuf<double> dt_cur_, dt_next_, partials_, force6_, stats6_;
-  DBuf<double> diag_part_, diag_;   // system statistics beyond the energies (launch_diagnostics)
+  DBuf<double> diag_;   // system statistics beyond the energies (launch_step_end)
   DBuf<uint32_t> key_hi_, key_lo_;
   // mixed form
   DBuf<D4> pos64_, vel64_, old64_;

@@ -254,10 +254,18 @@ void launch_refresh_mixed(const D4* pos64, const D4* vel64, const double* u64, F
 }
 
 // ---------------------------------------------------------------------------
-// reductions: each block reduces 6 doubles into partials[6*block + c]; one
-// block then sums the partials in index order.
-__device__ __forceinline__ void block_sum6(double v[6], double* partials) {
-  __shared__ double s[6][kRedBlock];
+// The end of a step: adding gravity with the force and torque sums, the
+// energy and angular momentum sums, the rest of system_statistics.cpp:19-64 and
+// the timestep minimum.  All are one pass over the particles and one fold of
+// its blocks' results, so they share two launches (eight before), which at
+// 16 384 particles cost their launches, not their work: with the six launches and
+// copies saved in the scans and the reaction lists, a mixed step there takes 0.49
+// ms in place of 0.53, a plain one 1.02 in place of 1.04.  Reductions are in a
+// fixed order: each block's tree, then one block over the blocks.
+
+// each block reduces 6 doubles into partials[6*block + c]
+__device__ __forceinline__ void block_sum6(double (*s)[kRedBlock], const double v[6], double* partials) {
+  __syncthreads();
   for (int c = 0; c < 6; ++c) s[c][threadIdx.x] = v[c];
   __syncthreads();
   for (int off = kRedBlock / 2; off > 0; off >>= 1) {
@@ -265,130 +273,13 @@ __device__ __forceinline__ void block_sum6(double v[6], double* partials) {
       for (int c = 0; c < 6; ++c) s[c][threadIdx.x] += s[c][threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x < 6) partials[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
+  if (threadIdx.x < 6) partials[threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(kRedBlock) void k_final_sum6(const double* __restrict__ partials, int nb,
-                                                           double* __restrict__ out6) {
-  __shared__ double s[6][kRedBlock];
-  double v[6] = {0, 0, 0, 0, 0, 0};
-  for (int b = threadIdx.x; b < nb; b += kRedBlock)
-    for (int c = 0; c < 6; ++c) v[c] += partials[6 * b + c];
-  for (int c = 0; c < 6; ++c) s[c][threadIdx.x] = v[c];
-  __syncthreads();
-  for (int off = kRedBlock / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off)
-      for (int c = 0; c < 6; ++c) s[c][threadIdx.x] += s[c][threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) out6[threadIdx.x] = s[threadIdx.x][0];
-}
-
-long reduce_partials(int n) { return 6L * ceil_div(n, kRedBlock) + 6; }
-
-template <class T>
-__global__ __launch_bounds__(kRedBlock) void k_add_gravity(V4<T>* __restrict__ bdots, const V4<T>* __restrict__ grav,
-                                                            const V4<T>* __restrict__ pos,
-                                                            const V4<T>* __restrict__ vel, int n,
-                                                            double* __restrict__ partials) {
-  const int i = blockIdx.x * kRedBlock + threadIdx.x;
-  double v[6] = {0, 0, 0, 0, 0, 0};
-  if (i < n) {
-    V4<T> d = bdots[i];
-    const V4<T> g = grav[i], p = pos[i];
-    d.x += g.x;
-    d.y += g.y;
-    d.z += g.z;
-    bdots[i] = d;
-    const T m = vel[i].w;
-    v[0] = m * d.x;
-    v[1] = m * d.y;
-    v[2] = m * d.z;
-    v[3] = m * (p.y * d.z - p.z * d.y);
-    v[4] = m * (p.z * d.x - p.x * d.z);
-    v[5] = m * (p.x * d.y - p.y * d.x);
-  }
-  block_sum6(v, partials);
-}
-
-template <class T>
-void launch_add_gravity(V4<T>* bdots, const V4<T>* grav, const V4<T>* pos, const V4<T>* vel, int n,
-                        double* partials, double* out6, hipStream_t s) {
-  const int nb = ceil_div(n, kRedBlock);
-  hipLaunchKernelGGL(k_add_gravity<T>, dim3(nb), dim3(kRedBlock), 0, s, bdots, grav, pos, vel, n, partials);
-  CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_final_sum6, dim3(1), dim3(kRedBlock), 0, s, partials, nb, out6);
-  CS_CHECK_LAUNCH();
-}
-template void launch_add_gravity<float>(F4*, const F4*, const F4*, const F4*, int, double*, double*, hipStream_t);
-template void launch_add_gravity<double>(D4*, const D4*, const D4*, const D4*, int, double*, double*, hipStream_t);
-
-template <class T>
-__global__ __launch_bounds__(kRedBlock) void k_stats(const V4<T>* __restrict__ pos, const V4<T>* __restrict__ vel,
-                                                      const V4<T>* __restrict__ hydro, const V4<T>* __restrict__ grav,
-                                                      int n, double* __restrict__ partials) {
-  const int i = blockIdx.x * kRedBlock + threadIdx.x;
-  double v[6] = {0, 0, 0, 0, 0, 0};
-  if (i < n) {
-    const V4<T> p = pos[i], u = vel[i];
-    const double m = u.w;
-    v[0] = 0.5 * m * ((double)u.x * u.x + (double)u.y * u.y + (double)u.z * u.z);
-    v[1] = m * (double)hydro[i].z;
-    v[2] = 0.5 * m * (double)grav[i].w;
-    v[3] = m * ((double)p.y * u.z - (double)p.z * u.y);
-    v[4] = m * ((double)p.z * u.x - (double)p.x * u.z);
-    v[5] = m * ((double)p.x * u.y - (double)p.y * u.x);
-  }
-  block_sum6(v, partials);
-}
-
-template <class T>
-void launch_stats(const V4<T>* pos, const V4<T>* vel, const V4<T>* hydro, const V4<T>* grav, int n,
-                  double* partials, double* out6, hipStream_t s) {
-  const int nb = ceil_div(n, kRedBlock);
-  hipLaunchKernelGGL(k_stats<T>, dim3(nb), dim3(kRedBlock), 0, s, pos, vel, hydro, grav, n, partials);
-  CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_final_sum6, dim3(1), dim3(kRedBlock), 0, s, partials, nb, out6);
-  CS_CHECK_LAUNCH();
-}
-template void launch_stats<float>(const F4*, const F4*, const F4*, const F4*, int, double*, double*, hipStream_t);
-template void launch_stats<double>(const D4*, const D4*, const D4*, const D4*, int, double*, double*, hipStream_t);
-
-__global__ __launch_bounds__(kRedBlock) void k_stats_mixed(const D4* __restrict__ pos64, const D4* __restrict__ vel64,
-                                                            const double* __restrict__ u64,
-                                                            const F4* __restrict__ grav, int n,
-                                                            double* __restrict__ partials) {
-  const int i = blockIdx.x * kRedBlock + threadIdx.x;
-  double v[6] = {0, 0, 0, 0, 0, 0};
-  if (i < n) {
-    const D4 p = pos64[i], u = vel64[i];
-    const double m = u.w;
-    v[0] = 0.5 * m * (u.x * u.x + u.y * u.y + u.z * u.z);
-    v[1] = m * u64[i];
-    v[2] = 0.5 * m * (double)grav[i].w;
-    v[3] = m * (p.y * u.z - p.z * u.y);
-    v[4] = m * (p.z * u.x - p.x * u.z);
-    v[5] = m * (p.x * u.y - p.y * u.x);
-  }
-  block_sum6(v, partials);
-}
-
-void launch_stats_mixed(const D4* pos64, const D4* vel64, const double* u64, const F4* grav, int n,
-                        double* partials, double* out6, hipStream_t s) {
-  const int nb = ceil_div(n, kRedBlock);
-  hipLaunchKernelGGL(k_stats_mixed, dim3(nb), dim3(kRedBlock), 0, s, pos64, vel64, u64, grav, n, partials);
-  CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_final_sum6, dim3(1), dim3(kRedBlock), 0, s, partials, nb, out6);
-  CS_CHECK_LAUNCH();
-}
-
-// ---------------------------------------------------------------------------
-// The rest of system_statistics.cpp:19-64: bounding box, mass-weighted sums
-// for the centre of mass, and the h-solve counts n_ngb (min, max, sum, sum of
-// squares), plus the particles whose list length ngb_count differs from
-// n_ngb and the longest list.  Each block writes kDiag values to its partials
-// row; one block folds the rows in a fixed order (sums of integers are exact
-// in doubles, min and max in any order), so the result is deterministic.
+// The rest of the statistics: bounding box, mass-weighted sums for the centre
+// of mass, and the h-solve counts n_ngb (min, max, sum, sum of squares), plus
+// the particles whose list length ngb_count differs from n_ngb and the longest
+// list (sums of integers are exact in doubles, min and max in any order).
 constexpr int kDiag = 19;
 enum { kDgMin = 0, kDgMax = 3, kDgM = 6, kDgMx = 7, kDgMv = 10, kDgSum = 13, kDgSq = 14, kDgMis = 15,
        kDgNmin = 16, kDgNmax = 17, kDgCmax = 18 };
@@ -425,70 +316,28 @@ __device__ __forceinline__ void diag_identity(double v[kDiag]) {
 }
 
 template <class P>
-__global__ __launch_bounds__(kRedBlock) void k_diagnostics(const V4<P>* __restrict__ pos,
-                                                            const V4<P>* __restrict__ vel,
-                                                            const int* __restrict__ n_ngb,
-                                                            const int* __restrict__ ngb_count, int n,
-                                                            double* __restrict__ partials) {
-  const int i = blockIdx.x * kRedBlock + threadIdx.x;
-  double v[kDiag];
-  diag_identity(v);
-  if (i < n) {
-    const V4<P> p = pos[i], u = vel[i];
-    const double m = u.w, x = p.x, y = p.y, z = p.z;
-    v[kDgMin] = v[kDgMax] = x;
-    v[kDgMin + 1] = v[kDgMax + 1] = y;
-    v[kDgMin + 2] = v[kDgMax + 2] = z;
-    v[kDgM] = m;
-    v[kDgMx] = m * x;
-    v[kDgMx + 1] = m * y;
-    v[kDgMx + 2] = m * z;
-    v[kDgMv] = m * (double)u.x;
-    v[kDgMv + 1] = m * (double)u.y;
-    v[kDgMv + 2] = m * (double)u.z;
-    const int k = n_ngb[i], c = ngb_count[i];
-    v[kDgSum] = k;
-    v[kDgSq] = (double)k * k;
-    v[kDgMis] = c != k;
-    v[kDgNmin] = v[kDgNmax] = k;
-    v[kDgCmax] = c;
-  }
-  block_diag(v);
-  if (threadIdx.x == 0)
-    for (int c = 0; c < kDiag; ++c) partials[(size_t)kDiag * blockIdx.x + c] = v[c];
+__device__ __forceinline__ void diag_particle(double v[kDiag], const V4<P>& p, const V4<P>& u, int k, int c) {
+  const double m = u.w, x = p.x, y = p.y, z = p.z;
+  v[kDgMin] = v[kDgMax] = x;
+  v[kDgMin + 1] = v[kDgMax + 1] = y;
+  v[kDgMin + 2] = v[kDgMax + 2] = z;
+  v[kDgM] = m;
+  v[kDgMx] = m * x;
+  v[kDgMx + 1] = m * y;
+  v[kDgMx + 2] = m * z;
+  v[kDgMv] = m * (double)u.x;
+  v[kDgMv + 1] = m * (double)u.y;
+  v[kDgMv + 2] = m * (double)u.z;
+  v[kDgSum] = k;
+  v[kDgSq] = (double)k * k;
+  v[kDgMis] = c != k;
+  v[kDgNmin] = v[kDgNmax] = k;
+  v[kDgCmax] = c;
 }
 
-__global__ __launch_bounds__(kRedBlock) void k_diag_final(const double* __restrict__ partials, int nb,
-                                                           double* __restrict__ out) {
-  double v[kDiag];
-  diag_identity(v);
-  for (int b = threadIdx.x; b < nb; b += kRedBlock)
-    for (int c = 0; c < kDiag; ++c) v[c] = diag_fold(c, v[c], partials[(size_t)kDiag * b + c]);
-  block_diag(v);
-  if (threadIdx.x == 0)
-    for (int c = 0; c < kDiag; ++c) out[c] = v[c];
-}
-
-long diag_partials(int n) { return (long)kDiag * (ceil_div(n, kRedBlock) + 1); }
-
-template <class P>
-void launch_diagnostics(const V4<P>* pos, const V4<P>* vel, const int* n_ngb, const int* ngb_count, int n,
-                        double* partials, double* out, hipStream_t s) {
-  const int nb = ceil_div(n, kRedBlock);
-  hipLaunchKernelGGL(k_diagnostics<P>, dim3(nb), dim3(kRedBlock), 0, s, pos, vel, n_ngb, ngb_count, n, partials);
-  CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(kRedBlock), 0, s, partials, nb, out);
-  CS_CHECK_LAUNCH();
-}
-template void launch_diagnostics<float>(const F4*, const F4*, const int*, const int*, int, double*, double*,
-                                        hipStream_t);
-template void launch_diagnostics<double>(const D4*, const D4*, const int*, const int*, int, double*, double*,
-                                         hipStream_t);
-
-// ---------------------------------------------------------------------------
-// timestep: per-block minimum, then one block's minimum (exact in any order)
-__device__ __forceinline__ void block_min(double v, double* out) {
-  __shared__ double s[kRedBlock];
+// minimum over the block (exact in any order)
+__device__ __forceinline__ void block_min(double* s, double v, double* out) {
+  __syncthreads();
   s[threadIdx.x] = v;
   __syncthreads();
   for (int off = kRedBlock / 2; off > 0; off >>= 1) {
@@ -498,78 +347,134 @@ __device__ __forceinline__ void block_min(double v, double* out) {
   if (threadIdx.x == 0) *out = s[0];
 }
 
+// partials: per block {6 force, 6 stats, kDiag, 1} doubles, kind by kind
+constexpr int kEndForce = 0, kEndStats = 6, kEndDiag = 12, kEndMin = 12 + kDiag, kEndWords = 13 + kDiag;
+long reduce_partials(int n) { return (long)kEndWords * ceil_div(n, kRedBlock) + kEndWords; }
+
+template <class T, bool MIXED>
+__global__ __launch_bounds__(kRedBlock) void k_step_end(StepEnd<T> e, int what) {
+  __shared__ double s[6][kRedBlock];
+  const int i = blockIdx.x * kRedBlock + threadIdx.x, n = e.n;
+  const long nb = gridDim.x, b = blockIdx.x;
+  if (what & kAddGravity) {
+    double v[6] = {0, 0, 0, 0, 0, 0};
+    if (i < n) {
+      V4<T> d = e.bdots[i];
+      const V4<T> g = e.grav[i], p = e.pos[i];
+      d.x += g.x;
+      d.y += g.y;
+      d.z += g.z;
+      e.bdots[i] = d;
+      const T m = e.vel[i].w;
+      v[0] = m * d.x;
+      v[1] = m * d.y;
+      v[2] = m * d.z;
+      v[3] = m * (p.y * d.z - p.z * d.y);
+      v[4] = m * (p.z * d.x - p.x * d.z);
+      v[5] = m * (p.x * d.y - p.y * d.x);
+    }
+    block_sum6(s, v, e.partials + kEndForce * nb + 6 * b);
+  }
+  if (what & kStatistics) {
+    double v[6] = {0, 0, 0, 0, 0, 0}, dg[kDiag];
+    diag_identity(dg);
+    if (i < n) {
+      if constexpr (MIXED) {
+        const D4 p = e.pos64[i], u = e.vel64[i];
+        const double m = u.w;
+        v[0] = 0.5 * m * (u.x * u.x + u.y * u.y + u.z * u.z);
+        v[1] = m * e.u64[i];
+        v[2] = 0.5 * m * (double)e.grav[i].w;
+        v[3] = m * (p.y * u.z - p.z * u.y);
+        v[4] = m * (p.z * u.x - p.x * u.z);
+        v[5] = m * (p.x * u.y - p.y * u.x);
+        diag_particle<double>(dg, p, u, e.n_ngb[i], e.ngb_count[i]);
+      } else {
+        const V4<T> p = e.pos[i], u = e.vel[i];
+        const double m = u.w;
+        v[0] = 0.5 * m * ((double)u.x * u.x + (double)u.y * u.y + (double)u.z * u.z);
+        v[1] = m * (double)e.hydro[i].z;
+        v[2] = 0.5 * m * (double)e.grav[i].w;
+        v[3] = m * ((double)p.y * u.z - (double)p.z * u.y);
+        v[4] = m * ((double)p.z * u.x - (double)p.x * u.z);
+        v[5] = m * ((double)p.x * u.y - (double)p.y * u.x);
+        diag_particle<T>(dg, p, u, e.n_ngb[i], e.ngb_count[i]);
+      }
+    }
+    block_sum6(s, v, e.partials + kEndStats * nb + 6 * b);
+    block_diag(dg);
+    if (threadIdx.x == 0)
+      for (int c = 0; c < kDiag; ++c) e.partials[kEndDiag * nb + kDiag * b + c] = dg[c];
+  }
+  if (what & kTimestep) {
+    double v = 1.0e30;
+    if (i < n) {
+      if constexpr (MIXED) {
+        const double dt_vel = (double)e.cn_vel * fabs((double)e.pos[i].w / (double)e.hydro2[i].x);
+        const double dt_eth = (double)e.cn_eth * fabs(e.u64[i] / (double)e.bdots[i].w);
+        v = 1.0 / (1.0 / dt_vel + 1.0 / dt_eth);
+      } else {
+        const T vsig = e.hydro2[i].x;
+        const double dt_vel = T(e.cn_vel) * dabs(e.pos[i].w / vsig);
+        const double dt_eth = T(e.cn_eth) * dabs(e.hydro[i].z / e.bdots[i].w);
+        v = 1.0 / (1.0 / dt_vel + 1.0 / dt_eth);
+      }
+      if (!(v < 1.0e30)) v = 1.0e30;     // NaN and +inf leave the running minimum unchanged
+    }
+    block_min(s[0], v, e.partials + kEndMin * nb + b);
+  }
+}
+
+// one block per kind of result, in block order
+__global__ __launch_bounds__(kRedBlock) void k_step_end_fold(const double* __restrict__ partials, int nb, int what,
+                                                              int round_float, double* __restrict__ force6,
+                                                              double* __restrict__ stats6, double* __restrict__ diag,
+                                                              double* __restrict__ dt_out) {
+  __shared__ double s[6][kRedBlock];
+  const int kind = blockIdx.x;
+  if (kind < 2 && (what & (kind == 0 ? kAddGravity : kStatistics))) {
+    const double* p = partials + (long)(kind == 0 ? kEndForce : kEndStats) * nb;
+    double v[6] = {0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nb; b += kRedBlock)
+      for (int c = 0; c < 6; ++c) v[c] += p[6 * b + c];
+    block_sum6(s, v, kind == 0 ? force6 : stats6);
+  } else if (kind == 2 && (what & kStatistics)) {
+    const double* p = partials + (long)kEndDiag * nb;
+    double v[kDiag];
+    diag_identity(v);
+    for (int b = threadIdx.x; b < nb; b += kRedBlock)
+      for (int c = 0; c < kDiag; ++c) v[c] = diag_fold(c, v[c], p[(size_t)kDiag * b + c]);
+    block_diag(v);
+    if (threadIdx.x == 0)
+      for (int c = 0; c < kDiag; ++c) diag[c] = v[c];
+  } else if (kind == 3 && (what & kTimestep)) {
+    const double* p = partials + (long)kEndMin * nb;
+    double v = 1.0e30;
+    for (int b = threadIdx.x; b < nb; b += kRedBlock) v = fmin(v, p[b]);
+    __shared__ double m;
+    block_min(s[0], v, &m);
+    if (threadIdx.x == 0) *dt_out = round_float ? (double)(float)m : m;
+  }
+}
+
 template <class T>
-__global__ __launch_bounds__(kRedBlock) void k_timestep(const V4<T>* __restrict__ pos, const V4<T>* __restrict__ hydro,
-                                                         const V4<T>* __restrict__ hydro2,
-                                                         const V4<T>* __restrict__ bdots, int n, T cn_vel, T cn_eth,
-                                                         double* __restrict__ partials) {
-  const int i = blockIdx.x * kRedBlock + threadIdx.x;
-  double v = 1.0e30;
-  if (i < n) {
-    const T vsig = hydro2[i].x;
-    const double dt_vel = cn_vel * dabs(pos[i].w / vsig);
-    const double dt_eth = cn_eth * dabs(hydro[i].z / bdots[i].w);
-    v = 1.0 / (1.0 / dt_vel + 1.0 / dt_eth);
-    if (!(v < 1.0e30)) v = 1.0e30;     // NaN and +inf leave the running minimum unchanged
+void launch_step_end(const StepEnd<T>& e, int what, int round_float, double* force6, double* stats6, double* diag,
+                     double* dt_out, hipStream_t s) {
+  const int nb = ceil_div(e.n, kRedBlock);
+  if constexpr (sizeof(T) == 4) {
+    if (e.pos64) hipLaunchKernelGGL((k_step_end<float, true>), dim3(nb), dim3(kRedBlock), 0, s, e, what);
+    else hipLaunchKernelGGL((k_step_end<float, false>), dim3(nb), dim3(kRedBlock), 0, s, e, what);
+  } else {
+    hipLaunchKernelGGL((k_step_end<double, false>), dim3(nb), dim3(kRedBlock), 0, s, e, what);
   }
-  block_min(v, partials + blockIdx.x);
-}
-
-__global__ __launch_bounds__(kRedBlock) void k_timestep_mixed(const F4* __restrict__ pos,
-                                                               const double* __restrict__ u64,
-                                                               const F4* __restrict__ hydro2,
-                                                               const F4* __restrict__ bdots, int n, float cn_vel,
-                                                               float cn_eth, double* __restrict__ partials) {
-  const int i = blockIdx.x * kRedBlock + threadIdx.x;
-  double v = 1.0e30;
-  if (i < n) {
-    const double dt_vel = (double)cn_vel * fabs((double)pos[i].w / (double)hydro2[i].x);
-    const double dt_eth = (double)cn_eth * fabs(u64[i] / (double)bdots[i].w);
-    v = 1.0 / (1.0 / dt_vel + 1.0 / dt_eth);
-    if (!(v < 1.0e30)) v = 1.0e30;
-  }
-  block_min(v, partials + blockIdx.x);
-}
-
-__global__ __launch_bounds__(kRedBlock) void k_final_min(const double* __restrict__ partials, int nb,
-                                                          int round_float, double* __restrict__ out) {
-  double v = 1.0e30;
-  for (int b = threadIdx.x; b < nb; b += kRedBlock) v = fmin(v, partials[b]);
-  __shared__ double s[kRedBlock];
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = kRedBlock / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off) s[threadIdx.x] = fmin(s[threadIdx.x], s[threadIdx.x + off]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = round_float ? (double)(float)s[0] : s[0];
-}
-
-template <class T>
-void launch_timestep(const V4<T>* pos, const V4<T>* hydro, const V4<T>* hydro2, const V4<T>* bdots, int n,
-                     float cn_vel, float cn_eth, int round_float, double* partials, double* dt_out,
-                     hipStream_t s) {
-  const int nb = ceil_div(n, kRedBlock);
-  hipLaunchKernelGGL(k_timestep<T>, dim3(nb), dim3(kRedBlock), 0, s, pos, hydro, hydro2, bdots, n, T(cn_vel),
-                     T(cn_eth), partials);
   CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_final_min, dim3(1), dim3(kRedBlock), 0, s, partials, nb, round_float, dt_out);
+  hipLaunchKernelGGL(k_step_end_fold, dim3(4), dim3(kRedBlock), 0, s, e.partials, nb, what, round_float, force6,
+                     stats6, diag, dt_out);
   CS_CHECK_LAUNCH();
 }
-template void launch_timestep<float>(const F4*, const F4*, const F4*, const F4*, int, float, float, int, double*,
-                                     double*, hipStream_t);
-template void launch_timestep<double>(const D4*, const D4*, const D4*, const D4*, int, float, float, int, double*,
-                                      double*, hipStream_t);
-
-void launch_timestep_mixed(const F4* pos, const double* u64, const F4* hydro2, const F4* bdots, int n,
-                           float cn_vel, float cn_eth, double* partials, double* dt_out, hipStream_t s) {
-  const int nb = ceil_div(n, kRedBlock);
-  hipLaunchKernelGGL(k_timestep_mixed, dim3(nb), dim3(kRedBlock), 0, s, pos, u64, hydro2, bdots, n, cn_vel, cn_eth,
-                     partials);
-  CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_final_min, dim3(1), dim3(kRedBlock), 0, s, partials, nb, 0, dt_out);
-  CS_CHECK_LAUNCH();
-}
+template void launch_step_end<float>(const StepEnd<float>&, int, int, double*, double*, double*, double*, hipStream_t);
+template void launch_step_end<double>(const StepEnd<double>&, int, int, double*, double*, double*, double*,
+                                      hipStream_t);
 
 // ---------------------------------------------------------------------------
 template <class R>

@@ -108,20 +108,20 @@ void launch_axis_sorts(const V4<T>* pos, int n, KV* kv, KV* alt, int* lists, lon
                        hipStream_t s);
 // the reaction lists: for each of the n particles j, the list slots k
 // naming j in ascending k, as pairs {key = owner i, value = k} in
-// pairs[start[j], end[j]) (end[j] = start[j + 1]; start holds n + 1 ints).
-// tcnt holds n ints of scratch, alt as many pairs as pairs, scan_scratch
-// scan_scratch_ints(n) ints.
+// pairs[start[j], start[j + 1]).  tcnt holds n ints, zero on entry and again
+// on return, alt as many pairs as pairs, scan_scratch scan_scratch_ints(n)
+// ints.
 void launch_reaction_transpose(const int* offset, const int* count, const int* list, int n, int* tcnt,
-                               int* start, int* end, KV* pairs, KV* alt, int* scan_scratch, hipStream_t s);
+                               int* start, KV* pairs, KV* alt, int* scan_scratch, hipStream_t s);
 // kv[t].key = keys[t]
 void launch_set_keys(KV* kv, const uint32_t* keys, int n, hipStream_t s);
 // bdots[j].xyz += ngb_acc[k] (r_i - r_j) over the reaction pairs of j, in
 // ascending k (sph_accelerations.cpp:104-115)
 template <class T>
 void launch_reaction(const V4<T>* pos, V4<T>* bdots, const T* ngb_acc, const KV* pairs, const int* start,
-                     const int* end, int n, hipStream_t s);
+                     int n, hipStream_t s);
 void launch_reaction_mixed(const F4* pos, const F4* pos_lo, F4* bdots, const float* ngb_acc, const KV* pairs,
-                           const int* start, const int* end, int n, hipStream_t s);
+                           const int* start, int n, hipStream_t s);
 // Peano-Hilbert keys on the bounding cube (sort_bodies.cpp:121-163); keys
 // are 3*bits wide, written as (hi,lo) 32-bit halves; scratch holds
 // 6 * (ceil(n / 256) + 1) reals of type T
@@ -168,34 +168,30 @@ void launch_correct_mixed(D4* vel64, double* u64, const D4* old64, F4* vel, F4* 
                           const double* dt_new, const double* dt_old, int n, hipStream_t s);
 void launch_refresh_mixed(const D4* pos64, const D4* vel64, const double* u64, F4* pos, F4* pos_lo, F4* vel,
                           F4* hydro, int n, hipStream_t s);
-// dots += grav, and per-block partial sums of force and torque
+// The end of a step over the n real particles, `what` a sum of:
+enum {
+  kAddGravity = 1,   // bdots += grav; force6: the force and torque sums
+  kStatistics = 2,   // stats6: T U W Jx Jy Jz; diag: bounding box, mass and mass-weighted position and velocity
+                     // sums, the h-solve counts n_ngb (min, max, sum, sum of squares), the number whose list
+                     // length ngb_count differs, the longest list (19 doubles; layout: integrate.hip, kDg*)
+  kTimestep = 4      // dt = min_i 1/(1/dt_vel + 1/dt_eth) (compute_timestep.cpp:3-25); round_float stores the
+                     // float-rounded value as the reference returns float
+};
 template <class T>
-void launch_add_gravity(V4<T>* bdots, const V4<T>* grav, const V4<T>* pos, const V4<T>* vel, int n,
-                        double* partials, double* out6, hipStream_t s);
-// dt = min_i 1/(1/dt_vel + 1/dt_eth) (compute_timestep.cpp:3-25); round_float
-// stores the float-rounded value as the reference returns float
+struct StepEnd {
+  V4<T>* bdots;
+  const V4<T>*grav, *pos, *vel, *hydro, *hydro2;
+  const D4 *pos64, *vel64;   // the mixed form's state, else null
+  const double* u64;
+  const int *n_ngb, *ngb_count;
+  int n;
+  float cn_vel, cn_eth;
+  double* partials;          // reduce_partials(n)
+};
+long reduce_partials(int n);
 template <class T>
-void launch_timestep(const V4<T>* pos, const V4<T>* hydro, const V4<T>* hydro2, const V4<T>* bdots, int n,
-                     float cn_vel, float cn_eth, int round_float, double* partials, double* dt_out,
-                     hipStream_t s);
-void launch_timestep_mixed(const F4* pos, const double* u64, const F4* hydro2, const F4* bdots, int n,
-                           float cn_vel, float cn_eth, double* partials, double* dt_out, hipStream_t s);
-// T U W Jx Jy Jz sums
-template <class T>
-void launch_stats(const V4<T>* pos, const V4<T>* vel, const V4<T>* hydro, const V4<T>* grav, int n,
-                  double* partials, double* out6, hipStream_t s);
-void launch_stats_mixed(const D4* pos64, const D4* vel64, const double* u64, const F4* grav, int n,
-                        double* partials, double* out6, hipStream_t s);
-long reduce_partials(int n);   // doubles needed for partial sums of n items (x6 components)
-// bounding box, mass and mass-weighted position and velocity sums, and the
-// h-solve counts n_ngb (min, max, sum, sum of squares) of the n real
-// particles, the number whose list length ngb_count differs from n_ngb, and
-// the longest list: 19 doubles into out (layout: integrate.hip, kDg*);
-// partials holds diag_partials(n) doubles
-long diag_partials(int n);
-template <class P>
-void launch_diagnostics(const V4<P>* pos, const V4<P>* vel, const int* n_ngb, const int* ngb_count, int n,
-                        double* partials, double* out, hipStream_t s);
+void launch_step_end(const StepEnd<T>& e, int what, int round_float, double* force6, double* stats6, double* diag,
+                     double* dt_out, hipStream_t s);
 // permutation gather of a 4-record array: dst[t] = src[perm[t]]
 template <class R>
 void launch_gather(const R* src, R* dst, const KV* perm, int n, hipStream_t s);

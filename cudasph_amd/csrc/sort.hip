@@ -45,39 +45,32 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int* __restric
   if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
-// one block scans the tile partials in chunks of 256, carrying the sum
-__global__ __launch_bounds__(kScanBlock) void k_scan_partials(int* __restrict__ partial, int n_part) {
-  __shared__ int s_tmp[kScanBlock];
-  int carry = 0;
-  for (int c0 = 0; c0 < n_part; c0 += kScanBlock) {
-    const int idx = c0 + threadIdx.x;
-    const int v = idx < n_part ? partial[idx] : 0;
-    int total;
-    const int ex = block_exclusive_scan(v, s_tmp, total);
-    if (idx < n_part) partial[idx] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) partial[n_part] = carry;
-}
-
+// each block adds the tiles before its own itself (a few loads per lane; a
+// launch of one block in between cost more)
 __global__ __launch_bounds__(kScanBlock) void k_scan_down(const int* __restrict__ in, long n, int mode,
-                                                           const int* __restrict__ partial, int* __restrict__ out,
-                                                           int n_part) {
-  __shared__ int s_tmp[kScanBlock];
+                                                           const int* __restrict__ partial, int* __restrict__ out) {
+  __shared__ int s_tmp[kScanBlock], s_before[kScanBlock / 64];
   const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
   int v[kScanItems];
-  int sum = 0;
+  int sum = 0, before = 0;
+  for (int t = threadIdx.x; t < (int)blockIdx.x; t += kScanBlock) before += partial[t];
+  for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+  if ((threadIdx.x & 63) == 0) s_before[threadIdx.x >> 6] = before;
   for (int k = 0; k < kScanItems; ++k) {
     v[k] = scan_load(in, base + k, n, mode);
     sum += v[k];
   }
   int total;
-  int run = block_exclusive_scan(sum, s_tmp, total) + partial[blockIdx.x];
+  int run = block_exclusive_scan(sum, s_tmp, total);   // (its barriers publish s_before)
+  for (int w = 0; w < kScanBlock / 64; ++w) {
+    run += s_before[w];
+    total += s_before[w];
+  }
   for (int k = 0; k < kScanItems; ++k) {
     if (base + k < n) out[base + k] = run;
     run += v[k];
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = partial[n_part];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = total;
 }
 
 long scan_scratch_ints(long n) { return (n + kScanTile - 1) / kScanTile + 1; }
@@ -90,9 +83,7 @@ void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scrat
   }
   hipLaunchKernelGGL(k_scan_reduce, dim3(n_part), dim3(kScanBlock), 0, s, in, n, mode, scratch);
   CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kScanBlock), 0, s, scratch, n_part);
-  CS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_scan_down, dim3(n_part), dim3(kScanBlock), 0, s, in, n, mode, scratch, out, n_part);
+  hipLaunchKernelGGL(k_scan_down, dim3(n_part), dim3(kScanBlock), 0, s, in, n, mode, scratch, out);
   CS_CHECK_LAUNCH();
 }
 
@@ -402,7 +393,8 @@ __global__ __launch_bounds__(kBlock) void k_tr_count(const int* __restrict__ off
   for (int k = off + lane; k < off + c; k += 64) atomicAdd(&tcnt[list[k]], 1);
 }
 
-// each real slot takes a place in its j's bucket; tcnt counts down to zero
+// each real slot takes a place in its j's bucket; tcnt counts down to zero,
+// which is what the next transpose starts from
 __global__ __launch_bounds__(kBlock) void k_tr_fill(const int* __restrict__ offset, const int* __restrict__ count,
                                                      const int* __restrict__ list, const int* __restrict__ start,
                                                      int* __restrict__ tcnt, KV* __restrict__ pairs, int n) {
@@ -475,13 +467,11 @@ __global__ __launch_bounds__(64) void k_tr_sort(KV* __restrict__ pairs, KV* __re
 }
 
 void launch_reaction_transpose(const int* offset, const int* count, const int* list, int n, int* tcnt,
-                               int* start, int* end, KV* pairs, KV* alt, int* scan_scratch, hipStream_t s) {
-  CS_HIP(hipMemsetAsync(tcnt, 0, (size_t)n * sizeof(int), s));
+                               int* start, KV* pairs, KV* alt, int* scan_scratch, hipStream_t s) {
   const dim3 waves(ceil_div(n, kBlock / 64));
   hipLaunchKernelGGL(k_tr_count, waves, dim3(kBlock), 0, s, offset, count, list, tcnt, n);
   CS_CHECK_LAUNCH();
   launch_exclusive_scan(tcnt, start, n, 0, scan_scratch, s);
-  CS_HIP(hipMemcpyAsync(end, start + 1, (size_t)n * sizeof(int), hipMemcpyDeviceToDevice, s));
   hipLaunchKernelGGL(k_tr_fill, waves, dim3(kBlock), 0, s, offset, count, list, start, tcnt, pairs, n);
   CS_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_tr_sort, dim3(n), dim3(64), 0, s, pairs, alt, start, n);
@@ -500,13 +490,12 @@ void launch_set_keys(KV* kv, const uint32_t* keys, int n, hipStream_t s) {
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_reaction(const V4<T>* __restrict__ pos, V4<T>* __restrict__ bdots,
                                                       const T* __restrict__ ngb_acc, const KV* __restrict__ pairs,
-                                                      const int* __restrict__ start, const int* __restrict__ end,
-                                                      int n) {
+                                                      const int* __restrict__ start, int n) {
   const int j = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (j >= n) return;
   const V4<T> pj = pos[j];
   V4<T> d = bdots[j];
-  const int p0 = start[j], p1 = end[j];
+  const int p0 = start[j], p1 = start[j + 1];
   // software pipeline: the next slot's owner, coefficient and position are
   // requested before the current term is added (the sum keeps slot order)
   KV e = p0 < p1 ? pairs[p0] : KV{(uint32_t)j, 0u};
@@ -530,15 +519,13 @@ __global__ __launch_bounds__(kBlock) void k_reaction(const V4<T>* __restrict__ p
 
 template <class T>
 void launch_reaction(const V4<T>* pos, V4<T>* bdots, const T* ngb_acc, const KV* pairs, const int* start,
-                     const int* end, int n, hipStream_t s) {
+                     int n, hipStream_t s) {
   hipLaunchKernelGGL(k_reaction<T>, dim3(ceil_div(n, kBlock)), dim3(kBlock), 0, s, pos, bdots, ngb_acc, pairs,
-                     start, end, n);
+                     start, n);
   CS_CHECK_LAUNCH();
 }
-template void launch_reaction<float>(const F4*, F4*, const float*, const KV*, const int*, const int*, int,
-                                     hipStream_t);
-template void launch_reaction<double>(const D4*, D4*, const double*, const KV*, const int*, const int*, int,
-                                      hipStream_t);
+template void launch_reaction<float>(const F4*, F4*, const float*, const KV*, const int*, int, hipStream_t);
+template void launch_reaction<double>(const D4*, D4*, const double*, const KV*, const int*, int, hipStream_t);
 
 // mixed form: the same gather with split positions and compensated sums; a
 // group of 8 lanes per j, each lane taking every 8th of j's slots, partial
@@ -546,8 +533,7 @@ template void launch_reaction<double>(const D4*, D4*, const double*, const KV*, 
 __global__ __launch_bounds__(kBlock) void k_reaction_mixed(const F4* __restrict__ pos, const F4* __restrict__ lo,
                                                             F4* __restrict__ bdots, const float* __restrict__ ngb_acc,
                                                             const KV* __restrict__ pairs,
-                                                            const int* __restrict__ start,
-                                                            const int* __restrict__ end, int n) {
+                                                            const int* __restrict__ start, int n) {
   constexpr int kG = 8;
   const int g = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int j = g / kG, lane = g % kG;
@@ -560,7 +546,7 @@ __global__ __launch_bounds__(kBlock) void k_reaction_mixed(const F4* __restrict_
     c[q] = (t - s[q]) - y;
     s[q] = t;
   };
-  for (int p = start[j] + lane; p < end[j]; p += kG) {
+  for (int p = start[j] + lane, p1 = start[j + 1]; p < p1; p += kG) {
     const KV e = pairs[p];
     const int i = (int)e.key;
     const float acc = ngb_acc[e.value];
@@ -587,9 +573,9 @@ __global__ __launch_bounds__(kBlock) void k_reaction_mixed(const F4* __restrict_
 }
 
 void launch_reaction_mixed(const F4* pos, const F4* pos_lo, F4* bdots, const float* ngb_acc, const KV* pairs,
-                           const int* start, const int* end, int n, hipStream_t s) {
+                           const int* start, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_reaction_mixed, dim3(ceil_div(n * 8, kBlock)), dim3(kBlock), 0, s, pos, pos_lo, bdots, ngb_acc,
-                     pairs, start, end, n);
+                     pairs, start, n);
   CS_CHECK_LAUNCH();
 }
 
