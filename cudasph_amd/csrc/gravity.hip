@@ -112,6 +112,24 @@ struct GAcc<double, 2> {
   __device__ __forceinline__ double get() const { return v; }
 };
 
+// v_rsq_f32 between scalar instructions.  A wavefront whose next vector
+// operation follows a transcendental one directly holds up the SIMD's vector
+// issue for the other wavefronts too: 11 multiplies and a v_rsq_f32 take 54
+// cycles of a SIMD with 4 or 8 wavefronts, 40 with a scalar instruction after
+// the v_rsq_f32 (the wait state its use needs anyway) and 33 with one on
+// either side, the sum of their issue times.  Raising the issue priority for
+// the v_rsq_f32 is the scalar instruction that helped the gravity kernels
+// most: mixed gravity at 2^20 particles 284 -> 275 ms in the same process (in
+// cycles 7 %; the clock falls from 2.24 to 2.14 GHz as the SIMDs fill), s_nop
+// on both sides 290-292 against 293.  Not for k_gravity_lane's pipelined loop,
+// whose order it breaks (100 003 particles 11.4 -> 13.2 ms), nor where the
+// caller has raised its own priority (it returns to 0).
+__device__ __forceinline__ float rsq_spaced(float x) {
+  float r;
+  asm("s_setprio 1\n\tv_rsq_f32 %0, %1\n\ts_setprio 0" : "=v"(r) : "v"(x));
+  return r;
+}
+
 template <bool EXACT>
 __device__ __forceinline__ float inv_sqrt(float x) {
   if constexpr (EXACT) return 1.0f / __builtin_sqrtf(x);
@@ -208,7 +226,6 @@ __device__ __forceinline__ void pair_plummer(A&& a, T rx, T ry, T rz, T mj, T ep
 constexpr int kGravBlock = 256;
 constexpr int kTile = 64;        // j per blocked-compensation partial (mixed form)
 constexpr int kJTile = 512;      // j records staged in LDS per block iteration (reference-layout kernels)
-constexpr int kGravParts = kGravMixedParts;
 // j records per LDS tile of the mixed Plummer kernel: one 64-record sub-tile
 // per wavefront.  Its 12 KB of LDS lets 8 blocks share a CU (the kernel's 63
 // VGPRs allow 8 waves per SIMD), so the 4096 x 8 blocks at N = 2^20 run in
@@ -852,7 +869,7 @@ __global__ __launch_bounds__(kGravBlock) void k_cell_moments(const F4* __restric
 __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx, float yy, float yz, float eps2,
                                           float& gx, float& gy, float& gz, float& pot) {
   const float s2 = __builtin_fmaf(yx, yx, __builtin_fmaf(yy, yy, __builtin_fmaf(yz, yz, eps2)));
-  const float inv = __builtin_amdgcn_rsqf(s2), i2 = inv * inv;
+  const float inv = rsq_spaced(s2), i2 = inv * inv;
   const float g0 = inv, g1 = -inv * i2, g2 = -3.f * g1 * i2, g3 = -5.f * g2 * i2, g4 = -7.f * g3 * i2,
               g5 = -9.f * g4 * i2;
   const float M0 = M[4], trM2 = M[5], trQ = M[6];
@@ -931,15 +948,23 @@ __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx,
 // partial acceleration, 1 subtraction for the potential.  With every mass
 // equal, tile-form sub-tiles skip r altogether (the expanded body below).
 //
-// Grid: `parts` j-parts per i-block, block b = i_block * parts + part.
-// Workgroups are dispatched round-robin over the 8 XCDs, so with 8 parts
-// part p runs on XCD p and each XCD streams only its 1/8 of the j-set
-// (4 MiB of hi+lo records at N = 2^20), which its L2 holds; without the
-// split every XCD streams the whole j-set and re-fetches it from HBM.  Each
-// block writes its compensated (hi, lo) partial sums; k_gravity_combine adds
-// the parts in order.  (Fewer parts leave the SPH passes beside gravity more
-// room but lengthen it: mixed step, 4 / 6 / 8 parts, 65 536 particles 2.30 /
-// 2.31 / 2.04 ms, 50 000: 1.57 / 1.44 / 1.40, 40 000: 1.20 / 1.02 / 1.00.)
+// Grid: `parts` j-parts per i-block, block b = i_block * parts + part.  Part p
+// takes the units p, p + parts, ... of j_unit records: tiles of 256, so that
+// the sub-tiles near an i-block, which are slower, fall to its parts evenly
+// (one contiguous unit per part below two tiles each, and for the far field,
+// whose cells must lie inside a part).  Workgroups are dispatched round-robin
+// over the 8 XCDs, so with a multiple of 8 parts each XCD streams only its 1/8
+// of the j-set (4 MiB of hi+lo records at N = 2^20), which its L2 holds;
+// without the split every XCD streams the whole j-set and re-fetches it from
+// HBM.  Each block writes its compensated (hi, lo) partial sums;
+// k_gravity_combine adds the parts in order.  The engine's parts are divided
+// further below kMixedQueueMaxN, since with 8 the last blocks ran alone for
+// long (65 536 particles: 4.9 wavefronts per SIMD in the mean of 8).  Gravity
+// alone, ms, contiguous 8 / tiles 8 / 16 / 24 / 40 parts: 16 384 particles 0.213
+// / 0.214 / 0.165 / 0.175 / 0.186, 32 768: 0.578 / 0.572 / 0.554 / 0.530 / 0.524,
+// 65 536: 1.95 / 1.89 / 1.72 / 1.67 / 1.65, 131 072: 6.05 / 5.81 / 5.48 / 5.25 /
+// 5.21, 250 007: 18.6 / 18.4 / 17.8 / 17.3 / 17.2, 500 000: 66.0 / 65.4 / 63.9 /
+// 63.0 / 62.6, 2^20: 274.6 / 272.3 / 271.1.
 // The far-field instantiation holds the 48 moment words of an expansion in
 // VGPRs next to the pairwise state: left alone the compiler takes 127
 // registers (4 wavefronts per SIMD); capped at 5 wavefronts it fits 96
@@ -947,19 +972,14 @@ __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx,
 // slower).  The pairwise instantiation is left unbounded (63 registers, 8
 // wavefronts).
 template <int JT, bool FAR>
-__global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(FAR ? 5 : 1)))
-void k_gravity_mixed_plummer(const F4* __restrict__ hi,
-                                                                       const F4* __restrict__ lo,
-                                                                       F4* __restrict__ part_hi,
-                                                                       F4* __restrict__ part_lo, int n_i,
-                                                                       int n_j, int j_chunk, float eps2,
-                                                                       int split_only,
-                                                                       const float* __restrict__ mass_range,
-                                                                       const float* __restrict__ mom,
-                                                                       FarRatios far_q2,
-                                                                       const float* __restrict__ cells,
-                                                                       const float* __restrict__ halves,
-                                                                       int n_real, int parts) {
+__device__ __forceinline__ void mixed_plummer_item(const F4* __restrict__ hi, const F4* __restrict__ lo,
+                                                   F4* __restrict__ part_hi, F4* __restrict__ part_lo, int n_i,
+                                                   int n_j, int j_unit, float eps2, int split_only,
+                                                   const float* __restrict__ mass_range,
+                                                   const float* __restrict__ mom, const FarRatios& far_q2,
+                                                   const float* __restrict__ cells,
+                                                   const float* __restrict__ halves, int n_real, int parts,
+                                                   int part, int i_block) {
   // every mass equal (mass_range = {min, max} over the real particles): the
   // pair body drops its mass factor and k_gravity_combine scales by m once;
   // padding records sit at 1e30, where r^2 overflows and rsq returns 0, so
@@ -978,8 +998,7 @@ void k_gravity_mixed_plummer(const F4* __restrict__ hi,
   __shared__ float s_r2[kSub];
   __shared__ __align__(16) float s_mom[kSub][FAR ? kMomWords : 1];
   static_assert(kTile == 64 && JT % kGravBlock == 0, "each wavefront stages whole sub-tiles");
-  const int part = blockIdx.x % parts;
-  const int i = (blockIdx.x / parts) * kGravBlock + threadIdx.x;
+  const int i = i_block * kGravBlock + threadIdx.x;
   const int ii = i < n_i ? i : n_i - 1;
   const int lane = threadIdx.x & 63;
   const F4 pi = hi[ii], li = lo[ii];
@@ -997,9 +1016,16 @@ void k_gravity_mixed_plummer(const F4* __restrict__ hi,
       a[3].part += pt;
     }
   };
-  const int j_begin = min(part * j_chunk, n_j), j_end = min(j_begin + j_chunk, n_j);
-  int skip_end = j_begin;   // this wavefront is done with the records below
-  for (int t0 = j_begin; t0 < j_end; t0 += JT) {
+  int j_begin = part * j_unit, j_end = min(j_begin + j_unit, n_j);
+  auto next_tile = [&](int t) {
+    t += JT;
+    if (t < j_end) return t;
+    j_begin += parts * j_unit;
+    j_end = min(j_begin + j_unit, n_j);
+    return j_begin;
+  };
+  int skip_end = j_begin;   // this wavefront is done with the records below (FAR: one unit per part)
+  for (int t0 = j_begin; t0 < j_end; t0 = next_tile(t0)) {
     const int cnt = min(JT, j_end - t0);
     bool need = true;
     if constexpr (FAR) {
@@ -1078,7 +1104,7 @@ void k_gravity_mixed_plummer(const F4* __restrict__ hi,
     if (FAR && !need) continue;   // a cell covered this tile for this wavefront
     auto pair = [&](float rx, float ry, float rz, float mj) {
       const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-      const float inv = __builtin_amdgcn_rsqf(d2);
+      const float inv = rsq_spaced(d2);
       const float mi = mj * inv;
       const float s3 = mi * (inv * inv);
       a[0].fsub(rx, s3);
@@ -1088,7 +1114,7 @@ void k_gravity_mixed_plummer(const F4* __restrict__ hi,
     };
     auto pair_unit = [&](float rx, float ry, float rz) {   // unit mass: 12 VALU + rsq
       const float d2 = __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, __builtin_fmaf(rz, rz, eps2)));
-      const float inv = __builtin_amdgcn_rsqf(d2);
+      const float inv = rsq_spaced(d2);
       const float s3 = inv * (inv * inv);
       a[0].fsub(rx, s3);
       a[1].fsub(ry, s3);
@@ -1179,7 +1205,7 @@ void k_gravity_mixed_plummer(const F4* __restrict__ hi,
               const F4 pj = s_rel[base + j];
               const float d2 =
                   __builtin_fmaf(pj.x, bx, __builtin_fmaf(pj.y, by, __builtin_fmaf(pj.z, bz, ci + pj.w)));
-              const float inv = __builtin_amdgcn_rsqf(d2);
+              const float inv = rsq_spaced(d2);
               const float s3 = inv * (inv * inv);
               sa += s3;
               mx = __builtin_fmaf(pj.x, s3, mx);
@@ -1240,6 +1266,73 @@ void k_gravity_mixed_plummer(const F4* __restrict__ hi,
   }
 }
 
+// one block per item (i_block, part)
+template <int JT, bool FAR>
+__global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(FAR ? 5 : 8)))
+void k_gravity_mixed_plummer(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ part_hi,
+                             F4* __restrict__ part_lo, int n_i, int n_j, int j_unit, float eps2, int split_only,
+                             const float* __restrict__ mass_range, const float* __restrict__ mom,
+                             FarRatios far_q2, const float* __restrict__ cells,
+                             const float* __restrict__ halves, int n_real, int parts) {
+  mixed_plummer_item<JT, FAR>(hi, lo, part_hi, part_lo, n_i, n_j, j_unit, eps2, split_only, mass_range, mom, far_q2,
+                              cells, halves, n_real, parts, blockIdx.x % parts, blockIdx.x / parts);
+}
+
+// Few particles: a limited number of blocks (gravity_mixed_blocks) take the
+// items from 8 queues, item t from queue t % 8, so a block starts with the
+// parts of its XCD and goes on with the others' at the end.  queue holds 8
+// zeroed counters.  With one block per item, 65 536 particles fill every
+// wavefront slot of the GPU until gravity ends, and the SPH passes of the other
+// stream wait for it, one after another; blocks that stay leave room for them
+// from the start, and items smaller than a block's share end together.
+template <int JT>
+__global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(8)))
+void k_gravity_mixed_queue(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ part_hi,
+                           F4* __restrict__ part_lo, int n_i, int n_j, int j_unit, float eps2, int split_only,
+                           const float* __restrict__ mass_range, int n_real, int parts, int n_items,
+                           int* __restrict__ queue) {
+  __shared__ int s_item;
+  int q = 0;   // queues found empty
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int t = -1;
+      for (; q < 8; ++q) {
+        const int x = (blockIdx.x + q) & 7, k = atomicAdd(&queue[x], 1);
+        if (8 * k + x < n_items) {
+          t = 8 * k + x;
+          break;
+        }
+      }
+      s_item = t;
+    }
+    __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(s_item);
+    if (t < 0) break;
+    mixed_plummer_item<JT, false>(hi, lo, part_hi, part_lo, n_i, n_j, j_unit, eps2, split_only, mass_range, nullptr,
+                                  FarRatios{}, nullptr, nullptr, n_real, parts, t % parts, t / parts);
+  }
+}
+
+static int gpu_cus() {
+  int dev = 0, cus = 0;
+  CS_HIP(hipGetDevice(&dev));
+  CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return cus;
+}
+
+// Blocks per CU of the queue kernel, 0 for one block per item.  Measured, ms
+// per mixed step, one block per item (8 parts) / 2 / 3 / 4 / 6 / 7 blocks per CU
+// (24 parts): 16 384 particles 0.482 / 0.477 / 0.514 / 0.545 / 0.673 / 0.672,
+// 24 000: 0.541 / 0.561 / 0.542 / 0.559 / 0.749 / 0.740, 32 768: 0.668 / 0.888 /
+// 0.738 / 0.667 / 0.951 / 0.998, 49 152: 1.281 / 1.693 / 1.337 / 1.186 / 1.233 /
+// 1.327, 65 536: 1.913 / 2.785 / 2.146 / 1.907 / 1.809 / 2.010, 131 072: 6.15 /
+// 9.52 / 7.13 / 6.20 / 6.00 / 6.27; 6 and 7 at 200 000: 12.70 / 12.72 / 12.91,
+// 400 000: 42.5 / 43.7 / 43.6.
+static int gravity_mixed_blocks(int n_j) {
+  return n_j < 20480 ? 2 : n_j < 28672 ? 3 : n_j < 57344 ? 4 : n_j < kMixedQueueMaxN ? 6 : 0;
+}
+
 // sum of the `parts` compensated partials of each i, in part order, times
 // the common mass when every mass is equal
 __global__ __launch_bounds__(kBlock) void k_gravity_combine(const F4* __restrict__ part_hi,
@@ -1287,7 +1380,9 @@ __global__ __launch_bounds__(kBlock) void k_mass_range_partials(const F4* __rest
   }
 }
 __global__ __launch_bounds__(kBlock) void k_mass_range_final(const float* __restrict__ partial, int nb,
-                                                             float* __restrict__ out) {
+                                                             float* __restrict__ out,
+                                                             int* __restrict__ queue) {
+  if (threadIdx.x < 8) queue[threadIdx.x] = 0;
   __shared__ float smin[kBlock], smax[kBlock];
   float lo = partial[0], hi = partial[1];
   for (int b = threadIdx.x; b < nb; b += kBlock) {
@@ -1409,9 +1504,7 @@ __global__ __launch_bounds__(kBlock) void k_gravity64_combine(const D4* __restri
 int gravity64_parts(int n_i) {
   const int blocks = ceil_div(n_i, kGravBlock);
   if (blocks >= 2048) return 1;
-  int dev = 0, cus = 0;
-  CS_HIP(hipGetDevice(&dev));
-  CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const int cus = gpu_cus();
   int best = 8;
   for (int p = 7; p >= 2 && (long)p * blocks >= 4l * cus; --p)   // fewer: too few wavefronts per SIMD
     // fullest CU's blocks per unit of work: ceil(p blocks / cus) / p
@@ -1476,18 +1569,23 @@ void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F
   if (soft == 0) {
     hipLaunchKernelGGL(k_gravity_mixed_spline, grid, block, 0, s, hi, lo, gvel, out, n_i, n_j);
   } else {
-    // mass_range: 2 floats of result followed by 2 per block of n_real
+    // mass_range: 2 floats of result followed by 2 per block of n_real and the
+    // 8 item queues, cleared with the result
     const int nb = ceil_div(n_real, kBlock);
+    int* queue = (int*)(mass_range + 2 + 2 * nb);
     hipLaunchKernelGGL(k_mass_range_partials, dim3(nb), dim3(kBlock), 0, s, hi, n_real, mass_range + 2);
     CS_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_mass_range_final, dim3(1), dim3(kBlock), 0, s, mass_range + 2, nb, mass_range);
+    hipLaunchKernelGGL(k_mass_range_final, dim3(1), dim3(kBlock), 0, s, mass_range + 2, nb, mass_range,
+                       queue);
     CS_CHECK_LAUNCH();
     const bool far = (split_only & 16) && moments;
-    if (parts <= 0 || far) parts = kGravParts;
-    if (parts > kGravParts) throw std::invalid_argument("gravity: at most 8 j-parts");
-    const int chunk = ceil_div(ceil_div(n_j, parts), kTile) * kTile;
+    if (parts <= 0 || far) parts = kGravMixedParts;
+    if (parts > kGravMixedParts) throw std::invalid_argument("gravity: at most 8 j-parts");
+    if (!far) parts *= gravity_mixed_pieces(n_j);
+    int unit = ceil_div(ceil_div(n_j, parts), kTile) * kTile;
+    if (!far && unit >= 2 * kJTileMixed) unit = kJTileMixed;
     F4* part_hi = part;
-    F4* part_lo = part + (size_t)kGravParts * n_i;
+    F4* part_lo = part + (size_t)parts * n_i;
     float* cells = nullptr;
     float* halves = nullptr;
     if ((split_only & 16) && moments) {
@@ -1524,15 +1622,19 @@ void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F
       const float q = far_ratio * powf(c, far_grade);
       fq.q2[L] = q * q;
     }
-    const dim3 ggrid(ceil_div(n_i, kGravBlock) * parts);
-    if ((split_only & 16) && moments)
-      hipLaunchKernelGGL((k_gravity_mixed_plummer<kJTileMixed, true>), ggrid, block, 0, s, hi, lo, part_hi, part_lo,
-                         n_i, n_j, chunk, eps * eps, split_only, mass_range, moments, fq, cells, halves, n_real,
-                         parts);
+    const int n_items = ceil_div(n_i, kGravBlock) * parts;
+    if (far)
+      hipLaunchKernelGGL((k_gravity_mixed_plummer<kJTileMixed, true>), dim3(n_items), block, 0, s, hi, lo, part_hi,
+                         part_lo, n_i, n_j, unit, eps * eps, split_only, mass_range, moments, fq, cells, halves,
+                         n_real, parts);
+    else if (const int per_cu = gravity_mixed_blocks(n_j))
+      hipLaunchKernelGGL((k_gravity_mixed_queue<kJTileMixed>), dim3(min(n_items, per_cu * gpu_cus())), block, 0, s,
+                         hi, lo, part_hi, part_lo, n_i, n_j, unit, eps * eps, split_only, mass_range, n_real, parts,
+                         n_items, queue);
     else
-      hipLaunchKernelGGL((k_gravity_mixed_plummer<kJTileMixed, false>), ggrid, block, 0, s, hi, lo, part_hi, part_lo,
-                         n_i, n_j, chunk, eps * eps, split_only, mass_range, nullptr, fq, nullptr, nullptr, n_real,
-                         parts);
+      hipLaunchKernelGGL((k_gravity_mixed_plummer<kJTileMixed, false>), dim3(n_items), block, 0, s, hi, lo, part_hi,
+                         part_lo, n_i, n_j, unit, eps * eps, split_only, mass_range, nullptr, fq, nullptr, nullptr,
+                         n_real, parts);
     CS_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_gravity_combine, dim3(ceil_div(n_i, kBlock)), dim3(kBlock), 0, s, part_hi, part_lo, out,
                        n_i, mass_range, split_only, parts);

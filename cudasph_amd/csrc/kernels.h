@@ -6,6 +6,13 @@
 
 namespace cudasph {
 
+// The SPH passes are short and latency-bound: a wavefront waits on a fetch or
+// a launch and then needs only a few instructions.  Beside gravity, whose
+// wavefronts always have VALU work ready, they would wait for issue behind
+// them too.  Their wavefronts take the highest issue priority instead, so they
+// issue as soon as their data is back and gravity fills the remaining cycles.
+__device__ __forceinline__ void chain_priority() { __builtin_amdgcn_s_setprio(3); }
+
 struct WalkParams {
   int n_nodes;        // real particles (the reference passes n_bodies, CUDA_calls.cpp:5)
   int fix_phantom;
@@ -70,17 +77,22 @@ void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, i
 int gravity64_parts(int n_i);
 void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_j, double eps, hipStream_t s,
                               int parts = 0);
-// part: scratch of 2 * 8 * n_i records (per-j-part partial sums, Plummer only);
-// mass_range: scratch of 2 + 2 * ceil(n_real / 256) floats ({min, max} of the
-// real particles' masses, then per-block partials)
+// part: scratch of 2 * kGravMixedParts * gravity_mixed_pieces(n_j) * n_i records
+// (per-j-part partial sums, Plummer only); mass_range: scratch of
+// 10 + 2 * ceil(n_real / 256) floats ({min, max} of the real particles' masses,
+// per-block partials and 8 work queues)
 // moments: scratch of 52 floats per 64-record j sub-tile followed by 52 per
 // cell of 16384, 4096, 1024 and 256 records and, with split_only bit 6, 52
 // per 32-record half sub-tile (the optional multipole far
 // field, split_only bit 4, taken where every lane of a wavefront is
 // far_ratio radii away, the ratio at a level of C records scaled by
 // (C / 16384)^far_grade; may be null otherwise)
-// parts: the number of j-parts, 1 .. kGravMixedParts; 0 for the most
+// parts: the number of j-parts, 1 .. kGravMixedParts; 0 for the most.  Each
+// part is cut into gravity_mixed_pieces(n_j) (not with the far field).
 constexpr int kGravMixedParts = 8;   // one per XCD
+constexpr int kMixedQueueMaxN = 196608;
+// (few particles: fewer partial sums to combine)
+inline int gravity_mixed_pieces(int n_j) { return n_j >= 8192 && n_j < kMixedQueueMaxN ? 3 : 1; }
 void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F4* part, float* mass_range,
                           float* moments, float far_ratio, float far_grade, int n_i, int n_j, int n_real,
                           int soft, float eps, int split_only, hipStream_t s, int parts = 0);

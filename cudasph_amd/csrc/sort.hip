@@ -36,6 +36,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_tmp, int& tota
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int* __restrict__ in, long n, int mode,
                                                              int* __restrict__ partial) {
+  chain_priority();
   __shared__ int s_tmp[kScanBlock];
   const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
   int sum = 0;
@@ -49,6 +50,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int* __restric
 // launch of one block in between cost more)
 __global__ __launch_bounds__(kScanBlock) void k_scan_down(const int* __restrict__ in, long n, int mode,
                                                            const int* __restrict__ partial, int* __restrict__ out) {
+  chain_priority();
   __shared__ int s_tmp[kScanBlock], s_before[kScanBlock / 64];
   const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
   int v[kScanItems];
@@ -318,6 +320,7 @@ __device__ __forceinline__ T coordinate(const V4<T>& p, int axis) {
 template <class T>
 __global__ __launch_bounds__(kRadixBlock) void k_axis_keys(const V4<T>* __restrict__ pos, KV* __restrict__ kv, int n,
                                                             int* __restrict__ scratch, long stride) {
+  chain_priority();
   constexpr int P = (int)sizeof(T);   // passes
   __shared__ int s_hist[P][256];
   const int axis = blockIdx.y;
@@ -345,7 +348,7 @@ __global__ __launch_bounds__(kRadixBlock) void k_axis_pass(const KV* __restrict_
                                                             int* __restrict__ lists, long list_stride, int n, int pass,
                                                             int* __restrict__ scratch, long stride,
                                                             const V4<T>* __restrict__ pos) {
-  __builtin_amdgcn_s_setprio(3);   // a chain of short passes; beside gravity it would wait for issue
+  chain_priority();
   const int axis = blockIdx.y;
   radix_pass(in + (size_t)axis * n, out + (size_t)axis * n,
              pass == (int)sizeof(T) - 1 ? lists + axis * list_stride : nullptr, n, 8 * (pass & 3), pass,
@@ -386,6 +389,7 @@ template void launch_axis_sorts<double>(const D4*, int, KV*, KV*, int*, long, in
 // its j's count
 __global__ __launch_bounds__(kBlock) void k_tr_count(const int* __restrict__ offset, const int* __restrict__ count,
                                                       const int* __restrict__ list, int* __restrict__ tcnt, int n) {
+  chain_priority();
   const int i = blockIdx.x * (kBlock / 64) + (int)(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (i >= n) return;
@@ -398,6 +402,7 @@ __global__ __launch_bounds__(kBlock) void k_tr_count(const int* __restrict__ off
 __global__ __launch_bounds__(kBlock) void k_tr_fill(const int* __restrict__ offset, const int* __restrict__ count,
                                                      const int* __restrict__ list, const int* __restrict__ start,
                                                      int* __restrict__ tcnt, KV* __restrict__ pairs, int n) {
+  chain_priority();
   const int i = blockIdx.x * (kBlock / 64) + (int)(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (i >= n) return;
@@ -447,6 +452,7 @@ __device__ __forceinline__ void bucket_sort(KV* __restrict__ p, int m, unsigned 
 constexpr int kTrSortMax = 512;
 __global__ __launch_bounds__(64) void k_tr_sort(KV* __restrict__ pairs, KV* __restrict__ alt,
                                                  const int* __restrict__ start, int n) {
+  chain_priority();
   __shared__ unsigned long long s[kTrSortMax];
   const int j = blockIdx.x, lane = threadIdx.x;
   if (j >= n) return;
@@ -491,6 +497,7 @@ template <class T>
 __global__ __launch_bounds__(kBlock) void k_reaction(const V4<T>* __restrict__ pos, V4<T>* __restrict__ bdots,
                                                       const T* __restrict__ ngb_acc, const KV* __restrict__ pairs,
                                                       const int* __restrict__ start, int n) {
+  chain_priority();
   const int j = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (j >= n) return;
   const V4<T> pj = pos[j];
@@ -534,6 +541,7 @@ __global__ __launch_bounds__(kBlock) void k_reaction_mixed(const F4* __restrict_
                                                             F4* __restrict__ bdots, const float* __restrict__ ngb_acc,
                                                             const KV* __restrict__ pairs,
                                                             const int* __restrict__ start, int n) {
+  chain_priority();
   constexpr int kG = 8;
   const int g = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int j = g / kG, lane = g % kG;

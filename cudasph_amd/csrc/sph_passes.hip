@@ -66,6 +66,7 @@ __global__ __launch_bounds__(kBlock) void k_density(const V4<T>* __restrict__ po
                                                      V4<T>* __restrict__ dots, const KV* __restrict__ hash,
                                                      const int* __restrict__ offset, const int* __restrict__ count,
                                                      const int* __restrict__ list, int n_dev) {
+  chain_priority();
   const int t = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (t >= n_dev) return;
   const int i = (int)hash[t].value;
@@ -117,6 +118,7 @@ __global__ __launch_bounds__(kBlock) void k_density(const V4<T>* __restrict__ po
 // dev_compute_pressure.cu:99-111 (every record, no hash, as the reference)
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_eos(V4<T>* __restrict__ hydro, int n_dev, EosConst c) {
+  chain_priority();
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n_dev) return;
   hydro[i].y = eos_record<T>(hydro[i], c);
@@ -130,6 +132,7 @@ __global__ __launch_bounds__(kBlock) void k_eos(V4<T>* __restrict__ hydro, int n
 __global__ __launch_bounds__(kBlock) void k_eos_mixed(F4* __restrict__ hydro, const double* __restrict__ u64,
                                                        const F4* __restrict__ pos, const F4* __restrict__ dots,
                                                        F4* __restrict__ hydro2, int n, EosConst c) {
+  chain_priority();
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   const F4 hd = hydro[i];
@@ -158,6 +161,7 @@ __global__ __launch_bounds__(kBlock) void k_hydro(const V4<T>* __restrict__ pos,
                                                    const KV* __restrict__ hash, const int* __restrict__ offset,
                                                    const int* __restrict__ count, const int* __restrict__ list,
                                                    int n_dev, T alpha, T beta) {
+  chain_priority();
   const int t = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   if (t >= n_dev) return;
   const int i = (int)hash[t].value;
@@ -221,6 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_density_mixed(const F4* __restrict__
                                                           const int* __restrict__ offset,
                                                           const int* __restrict__ count,
                                                           const int* __restrict__ list, int n_dev) {
+  chain_priority();
   const int g = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int t = g / kGroup, lane = g % kGroup;
   if (t >= n_dev) return;   // whole groups leave together
@@ -287,6 +292,7 @@ __global__ __launch_bounds__(kBlock) void k_hydro_mixed(const F4* __restrict__ p
                                                         const KV* __restrict__ hash, const int* __restrict__ offset,
                                                         const int* __restrict__ count, const int* __restrict__ list,
                                                         int n_dev, float alpha, float beta) {
+  chain_priority();
   const int gl = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
   const int t = gl / kGroup, lane = gl % kGroup;
   if (t >= n_dev) return;   // whole groups leave together

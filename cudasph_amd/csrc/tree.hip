@@ -110,6 +110,7 @@ template <class T>
 __global__ __launch_bounds__(kBlock) void k_tree_fixed(V4<T>* __restrict__ tree, KV* __restrict__ hash, int n,
                                                         int n_dev, int heap_order, int* __restrict__ scratch,
                                                         int clear, long stride, int* __restrict__ ties) {
+  chain_priority();
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t < clear)
     for (int a = 0; a < 3; ++a) scratch[a * stride + t] = 0;
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_count(const int* __restrict__ l
                                                         const int* __restrict__ lc, const V4<T>* __restrict__ pos,
                                                         uint8_t* __restrict__ side, int2* __restrict__ tile_counts,
                                                         int m, int L, int n, int axis) {
-  __builtin_amdgcn_s_setprio(3);
+  chain_priority();
   __shared__ int2 s_wave[kBlock / 64];
   const int* l = blockIdx.y ? lc : lb;
   side += (size_t)blockIdx.y * n;
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_move(const int* __restrict__ la
                                                        const V4<T>* __restrict__ pos, V4<T>* __restrict__ tree,
                                                        KV* __restrict__ hash, int m, int L, int n, int axis,
                                                        int heap_order, int* __restrict__ ties) {
-  __builtin_amdgcn_s_setprio(3);
+  chain_priority();
   if (blockIdx.y == 0) {
 #pragma unroll
     for (int r = 0; r < kLevelRounds; ++r) {
@@ -289,10 +290,10 @@ __global__ __launch_bounds__(kBlock) void k_tree_move(const int* __restrict__ la
 // that level's layout.  The level kernels' dependent global-memory passes
 // (the build's cost at small N) become LDS passes; the results are the same
 // nodes in the same places.
-constexpr int kLdsMax = 2048;
+constexpr int kLdsMax = 1024;
 // threads of a finishing block: few blocks run (one per subtree), so each
 // takes a whole CU's worth of wavefronts to keep its passes short
-constexpr int kLdsThreads = 1024;
+constexpr int kLdsThreads = 512;
 
 struct LocalLevel {
   int L, r0, r1, r0n;        // level, the runs' range in its layout, and their start at level L+1
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_tree_lds(const int* __restrict_
                                                       int L0, int cur0, int cur1, int cur2,
                                                       const V4<T>* __restrict__ pos, V4<T>* __restrict__ tree,
                                                       KV* __restrict__ hash, int heap_order, int* __restrict__ ties) {
-  __builtin_amdgcn_s_setprio(3);
+  chain_priority();
   __shared__ uint16_t s_list[3][2][kLdsMax];   // slots, per axis, double-buffered
   __shared__ int s_tag[kLdsMax];               // the heap node each slot's particle belongs to
   __shared__ uint8_t s_fb[kLdsMax], s_fc[kLdsMax];
@@ -558,6 +559,7 @@ __device__ __forceinline__ void box_node(const V4<T>* __restrict__ tree, F4* box
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_tree_boxes_sub(const V4<T>* __restrict__ tree, F4* box, int n_nodes,
                                                             int fix_phantom, int S, int levels, int last_node) {
+  chain_priority();
   const long r = (1l << S) + blockIdx.x;
   for (int L = levels; L >= S; --L) {
     const long first = r << (L - S), cnt = 1l << (L - S);
@@ -571,6 +573,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_boxes_sub(const V4<T>* __restri
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_tree_boxes_top(const V4<T>* __restrict__ tree, F4* box, int n_nodes,
                                                             int fix_phantom, int S, int last_node) {
+  chain_priority();
   for (int L = S - 1; L >= 0; --L) {
     const int last = (int)std::min<long>((2l << L) - 1, (long)last_node);
     for (int k = (1 << L) + (int)threadIdx.x; k <= last; k += kBlock) box_node<T>(tree, box, n_nodes, fix_phantom, k);

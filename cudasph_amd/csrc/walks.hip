@@ -535,21 +535,13 @@ __device__ __forceinline__ void solve_range(V4<T> q, S& s, T& range, T& count) {
   range = q.w;
 }
 
-// The walk kernels are latency-bound: a wavefront waits on one dependent
-// tree fetch after another and then needs only a few instructions.  Beside
-// gravity, whose wavefronts always have VALU work ready, they would wait for
-// issue behind them too.  Their wavefronts take the highest issue priority
-// instead, so they issue as soon as their data is back and gravity fills the
-// remaining cycles.
-__device__ __forceinline__ void walk_priority() { __builtin_amdgcn_s_setprio(3); }
-
 // dev_solve_range.cu:174-189
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_solve_range(V4<T>* __restrict__ pos, int* __restrict__ n_ngb,
                                                          const KV* __restrict__ hash,
                                                          const V4<T>* __restrict__ tree, int n_dev,
                                                          WalkParams wp) {
-  walk_priority();
+  chain_priority();
   extern __shared__ __align__(16) char s_mem[];   // WalkLds<T, true> per group
   WalkLds<T, true>& s = reinterpret_cast<WalkLds<T, true>*>(s_mem)[threadIdx.x / kWalkGroup];
   const int t = (xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + (int)threadIdx.x) / kWalkGroup;
@@ -580,7 +572,7 @@ __global__ __launch_bounds__(kBlock) void k_find_ngb(const V4<T>* __restrict__ p
                                                       const int* cap_count, int* count_out,
                                                       int* __restrict__ list, int* __restrict__ flags,
                                                       int n_dev, WalkParams wp, int clamp) {
-  walk_priority();
+  chain_priority();
   extern __shared__ __align__(16) char s_mem[];   // WalkLds<int, false> per group
   WalkLds<int, false>& s = reinterpret_cast<WalkLds<int, false>*>(s_mem)[threadIdx.x / kWalkGroup];
   const int t = (xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + (int)threadIdx.x) / kWalkGroup;
@@ -653,7 +645,7 @@ __global__ __launch_bounds__(kBlock) void k_solve_range_lane(V4<T>* __restrict__
                                                               const KV* __restrict__ hash,
                                                               const V4<T>* __restrict__ tree, int n_dev,
                                                               WalkParams wp) {
-  walk_priority();
+  chain_priority();
   extern __shared__ int s_stack[];   // walk_stack_depth(n_nodes) entries per lane
   const int t = xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + threadIdx.x;
   if (t >= n_dev) return;
@@ -676,7 +668,7 @@ __global__ __launch_bounds__(kBlock) void k_find_ngb_lane(const V4<T>* __restric
                                                            int* count_out, int* __restrict__ list,
                                                            int* __restrict__ flags, int n_dev, WalkParams wp,
                                                            int clamp) {
-  walk_priority();
+  chain_priority();
   extern __shared__ int s_stack[];   // walk_stack_depth(n_nodes) entries per lane
   const int t = xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + threadIdx.x;
   if (t >= n_dev) return;
