@@ -32,6 +32,7 @@
 // counts still recorded).
 #include <stdexcept>
 
+#include "pairs64.h"
 #include "engine_impl.h"
 
 namespace cudasph {
@@ -395,7 +396,9 @@ __global__ __launch_bounds__(kBlock) void k_adj_density(const D4v* __restrict__ 
 
 // Plummer gravity reversed: a_i = -sum_j m_j r_ij / s^3, s^2 = |r_ij|^2 + eps^2
 //   x_bar_i += sum_j T_ij (m_i a_bar_j - m_j a_bar_i),  T = I/s^3 - 3 r r^T / s^5
-// One FP64 N^2 pass: j-tiles of (x, m, a_bar) staged in LDS, one i per lane,
+// The sum is antisymmetric in i and j, so pairs64.h's kernel takes a pair once
+// for both where it fits; below and above, every ordered pair:
+// one FP64 N^2 pass: j-tiles of (x, m, a_bar) staged in LDS, one i per lane,
 // the pair body in fused multiply-adds.  As in the forward FP64 kernel, with
 // few i-blocks the j-range is split into gravity64_parts(n) parts whose sums
 // (in `part`) are added in part order.
@@ -477,6 +480,61 @@ __global__ __launch_bounds__(kBlock) void k_adj_gravity_combine(const D4v* __res
   x.y += gy;
   x.z += gz;
   xs[i] = x;
+}
+
+// the same pair body for both particles: the terms of a pair are opposite
+struct AdjointPairs {
+  static constexpr int kRec = 4, kAcc = 3;
+  const D4v *pos, *vel, *abar;
+  double eps2;
+  struct Particle {
+    D4v p, a;   // p.w the mass
+  };
+  __device__ __forceinline__ Particle load(int i, int n) const {
+    if (i >= n) return {{1e30, 1e30, 1e30, 0.0}, {0.0, 0.0, 0.0, 0.0}};   // terms of exactly nothing
+    const D4v p = pos[i];
+    return {{p.x, p.y, p.z, vel[i].w}, abar[i]};
+  }
+  template <class S>
+  __device__ __forceinline__ void stage(S&& put, int j, int n) const {
+    const Particle q = load(j, n);
+    put(0, make_double2(q.p.x, q.p.y));
+    put(1, make_double2(q.p.z, q.p.w));
+    put(2, make_double2(q.a.x, q.a.y));
+    put(3, make_double2(q.a.z, 0.0));
+  }
+  template <bool REACT>
+  __device__ __forceinline__ void pair(const Particle& q, const double2 (&r)[4], double (&g)[3],
+                                       double (&c)[3]) const {
+    const double rx = q.p.x - r[0].x, ry = q.p.y - r[0].y, rz = q.p.z - r[1].x;
+    const double d2 = __builtin_fma(rx, rx, __builtin_fma(ry, ry, __builtin_fma(rz, rz, eps2)));
+    double inv = __builtin_amdgcn_rsq(d2);
+    inv = inv * __builtin_fma(-0.5 * d2, inv * inv, 1.5);   // one Newton step: ~1e-14 relative
+    const double inv2 = inv * inv, inv3 = inv2 * inv;
+    const double mi = q.p.w, mj = r[1].y;
+    const double bx = __builtin_fma(mi, r[2].x, -mj * q.a.x);
+    const double by = __builtin_fma(mi, r[2].y, -mj * q.a.y);
+    const double bz = __builtin_fma(mi, r[3].x, -mj * q.a.z);
+    const double t = 3.0 * __builtin_fma(rx, bx, __builtin_fma(ry, by, rz * bz)) * inv2;
+    const double vx = inv3 * __builtin_fma(-t, rx, bx), vy = inv3 * __builtin_fma(-t, ry, by),
+                 vz = inv3 * __builtin_fma(-t, rz, bz);
+    g[0] += vx;
+    g[1] += vy;
+    g[2] += vz;
+    if constexpr (REACT) {
+      c[0] -= vx;
+      c[1] -= vy;
+      c[2] -= vz;
+    }
+  }
+};
+
+__global__ __launch_bounds__(kBlock) void k_adj_gravity_pairs_sum(const double* __restrict__ own,
+                                                                  const double* __restrict__ react,
+                                                                  double* __restrict__ xs, int n, int tiles,
+                                                                  int parts) {
+  const int i = blockIdx.x * kBlock + threadIdx.x, k = blockIdx.y;
+  if (i < n) xs[4 * (size_t)i + k] += pairs64_sum<3>(own, react, i, k, tiles, parts);
 }
 
 // corrector reversed: a_bar += v_bar f, udot_bar += u_bar f
@@ -899,15 +957,24 @@ void Engine<T>::adj_forces_backward(bool seed_rho) {
     const double eps = (double)p_.grav_eps;
     const int parts = grav_parts_ ? grav_parts_ : gravity64_parts(n_);
     const int chunk = ceil_div(ceil_div(n_, parts), kAdjTile) * kAdjTile;
-    const bool beside = overlap_ && parts > 1;
-    if (parts > 1 && gpart64_.n < (size_t)parts * nd_) gpart64_.alloc((size_t)parts * nd_);
+    const bool pairs = pairs64_fits(n_);
+    const bool beside = overlap_ && (parts > 1 || pairs);
+    reserve_gpart64(parts);
+    double* ws = (double*)gpart64_.p;
+    const auto launch_gravity_terms = [&](hipStream_t gs) {
+      if (pairs) {
+        launch_pairs64(AdjointPairs{pos_.p, vel_.p, aa_.p, eps * eps}, n_, parts, ws, gs);
+        return;
+      }
+      hipLaunchKernelGGL(k_adj_gravity, dim3(ceil_div(n_, kBlock) * parts), dim3(kBlock), 0, gs, pos_.p, vel_.p,
+                         aa_.p, xs_.p, (D4v*)gpart64_.p, n_, parts, chunk, eps * eps);
+      CS_CHECK_LAUNCH();
+    };
     if (beside) {
       CS_HIP(hipEventRecord(ev_fork_, s_));
       CS_HIP(hipStreamWaitEvent(gs_, ev_fork_, 0));
       TimerScope tg(timers_, "adjoint_gravity", gs_);
-      hipLaunchKernelGGL(k_adj_gravity, dim3(ceil_div(n_, kBlock) * parts), dim3(kBlock), 0, gs_, pos_.p, vel_.p,
-                         aa_.p, xs_.p, (D4v*)gpart64_.p, n_, parts, chunk, eps * eps);
-      CS_CHECK_LAUNCH();
+      launch_gravity_terms(gs_);
       CS_HIP(hipEventRecord(ev_join_, gs_));
     }
     TimerScope ts(timers_, "adjoint_sph", s_);
@@ -948,11 +1015,13 @@ void Engine<T>::adj_forces_backward(bool seed_rho) {
       CS_HIP(hipStreamWaitEvent(s_, ev_join_, 0));
     } else {
       ts.t.begin("adjoint_gravity", s_);
-      hipLaunchKernelGGL(k_adj_gravity, dim3(ceil_div(n_, kBlock) * parts), dim3(kBlock), 0, s_, pos_.p, vel_.p,
-                         aa_.p, xs_.p, (D4v*)gpart64_.p, n_, parts, chunk, eps * eps);
-      CS_CHECK_LAUNCH();
+      launch_gravity_terms(s_);
     }
-    if (parts > 1) {
+    if (pairs) {
+      hipLaunchKernelGGL(k_adj_gravity_pairs_sum, dim3(ceil_div(n_, kBlock), 3), dim3(kBlock), 0, s_, ws,
+                         ws + pairs64_own(n_, parts), (double*)xs_.p, n_, pairs64_tiles(n_), parts);
+      CS_CHECK_LAUNCH();
+    } else if (parts > 1) {
       hipLaunchKernelGGL(k_adj_gravity_combine, grid(n_), dim3(kBlock), 0, s_, (const D4v*)gpart64_.p, xs_.p, n_,
                          parts);
       CS_CHECK_LAUNCH();

@@ -1,4 +1,5 @@
 // Device-resident SPH engine: the passes of step.cpp:13-147 over HBM state.
+#include "pairs64.h"
 #include "engine_impl.h"
 
 namespace cudasph {
@@ -98,10 +99,7 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
   tree_.alloc(nd_ + 2);
   ties_.alloc(1);
   boxes_.alloc(2 * ((size_t)nd_ + 2));
-  if (!kF32) {
-    const int parts = gravity64_parts(nd_);
-    if (parts > 1) gpart64_.alloc((size_t)parts * nd_);
-  }
+  if (!kF32) reserve_gpart64(gravity64_parts(nd_));
   hash_.alloc(nd_);
   perm_.alloc(nd_);
   n_ngb_.alloc(nd_);
@@ -680,6 +678,15 @@ void Engine<T>::gravity_pack() {
   launch_gravity_pack<T>(pos_, vel_, gpos_, gvel_, n_, nd_, s_);
 }
 
+// the partial sums of FP64 gravity and of its reverse pass (at most nd_ particles)
+template <class T>
+void Engine<T>::reserve_gpart64(int parts) {
+  size_t need = parts > 1 ? (size_t)parts * nd_ : 0;
+  for (const int n : {n_, nd_})
+    if (pairs64_fits(n)) need = std::max(need, (pairs64_words(n, parts) + 3) / 4);
+  if (gpart64_.n < need) gpart64_.alloc(need);
+}
+
 template <class T>
 void Engine<T>::gravity_kernels(hipStream_t gs) {
   TimerScope ts(timers_, "gravity", gs);
@@ -697,7 +704,7 @@ void Engine<T>::gravity_kernels(hipStream_t gs) {
   if constexpr (!kF32) {
     if (p_.grav_mode == 1) {
       const int parts = grav_parts_ ? grav_parts_ : gravity64_parts(nd_);
-      if (parts > 1 && gpart64_.n < (size_t)parts * nd_) gpart64_.alloc((size_t)parts * nd_);
+      reserve_gpart64(parts);
       launch_gravity64_plummer(gpos_, grav_, gpart64_.p, nd_, nd_, (double)p_.grav_eps, gs, parts);
       return;
     }

@@ -108,6 +108,7 @@ class Engine final : public EngineBase {
   void gravity(bool async = false);
   void gravity_join();
   void gravity_pack();
+  void reserve_gpart64(int parts);
   void gravity_kernels(hipStream_t gs);
   void step_end(int what, double* dt_out);
   void finish(double* dt_out);

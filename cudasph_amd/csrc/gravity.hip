@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "pairs64.h"
 #include "sph_math.h"
 
 namespace cudasph {
@@ -1445,7 +1446,9 @@ __global__ __launch_bounds__(kGravBlock) void k_gravity_mixed_spline(const F4* _
 // 3 sub, 3 FMA for s^2 = r^2 + eps^2, v_rsq_f64 refined by one third-order
 // step (y0 (1 + e (1/2 + 3/8 e)), e = 1 - s^2 y0^2: 5 operations, its remainder
 // 5/16 e^3 below one rounding), 3 for m/s^3, 3 FMA into the acceleration and one
-// into the potential.  With few i-blocks (N below 2^19) the j-range is split
+// into the potential.  Here every ordered pair is evaluated: below kPairs64MinN
+// and above kPairs64MaxN particles, or with other j than i (pairs64.h between).
+// With few i-blocks (N below 2^19) the j-range is split
 // into parts, one block per (i-block, part), so that the GPU holds enough
 // wavefronts to hide the FP64 latencies; the parts' sums are added in part
 // order (deterministic).
@@ -1498,9 +1501,11 @@ __global__ __launch_bounds__(kBlock) void k_gravity64_combine(const D4* __restri
 // Parts for the passes of the FP64 form: of 2 .. 8 (1 from 2^19 particles on)
 // the count whose blocks fill the CUs most evenly, the larger of equals.
 // Every block is resident at once and takes the same time, so a pass lasts as
-// long as its fullest CU.  FP64 step, 2 / 4 / 6 / 8 parts, ms: 50 021 particles
-// (196 i-blocks on 256 CUs) 3.00 / 2.77 / 2.30 / 2.47, 65 536: 4.30 / 3.65 / 4.02 / 3.55,
-// 131 072: 14.6 / 13.7 / 13.2 / 13.3.
+// long as its fullest CU.  Pairs taken once, gravity alone, 8 / 7 / 6 / 5 / 4 / 2
+// parts, ms: 50 021 particles (196 tiles on 256 CUs) 1.54 / 1.47 / 1.41 / 1.37 /
+// 1.65 / 1.80, 65 536: 2.22 / 2.20 / 2.17 / 2.20 / 2.23 / 2.41, 100 003: 5.55 / 5.35 /
+// 5.69 / 5.52 / 6.15 / 7.31.  Two or three times the parts are as fast alone and
+// leave the SPH passes less room: steps of 65 536 2.75 / 2.92 / 3.01.
 int gravity64_parts(int n_i) {
   const int blocks = ceil_div(n_i, kGravBlock);
   if (blocks >= 2048) return 1;
@@ -1512,10 +1517,63 @@ int gravity64_parts(int n_i) {
   return best;
 }
 
+// the pair body above, for both particles
+struct GravityPairs {
+  static constexpr int kRec = 2, kAcc = 4;
+  const D4* gpos;
+  double eps2;
+  __device__ __forceinline__ D4 load(int i, int n) const {
+    if (i < n) return gpos[i];
+    return {1e30, 1e30, 1e30, 0.0};   // no mass: its partners get exactly nothing
+  }
+  template <class S>
+  __device__ __forceinline__ void stage(S&& put, int j, int n) const {
+    const D4 p = load(j, n);
+    put(0, make_double2(p.x, p.y));
+    put(1, make_double2(p.z, p.w));
+  }
+  template <bool REACT>
+  __device__ __forceinline__ void pair(const D4& pi, const double2 (&r)[2], double (&g)[4], double (&a)[4]) const {
+    const double rx = pi.x - r[0].x, ry = pi.y - r[0].y, rz = pi.z - r[1].x;
+    const double d2 = __builtin_fma(rx, rx, __builtin_fma(ry, ry, __builtin_fma(rz, rz, eps2)));
+    const double y0 = __builtin_amdgcn_rsq(d2);
+    const double e = __builtin_fma(-(d2 * y0), y0, 1.0);
+    const double y = __builtin_fma(__builtin_fma(e, 0.375, 0.5), y0 * e, y0);
+    const double y3 = y * (y * y), mj = r[1].y * y3;
+    g[0] = __builtin_fma(-rx, mj, g[0]);
+    g[1] = __builtin_fma(-ry, mj, g[1]);
+    g[2] = __builtin_fma(-rz, mj, g[2]);
+    g[3] = __builtin_fma(-r[1].y, y, g[3]);
+    if constexpr (REACT) {
+      const double mi = pi.w * y3;
+      a[0] = __builtin_fma(rx, mi, a[0]);
+      a[1] = __builtin_fma(ry, mi, a[1]);
+      a[2] = __builtin_fma(rz, mi, a[2]);
+      a[3] = __builtin_fma(-pi.w, y, a[3]);
+    }
+  }
+};
+
+__global__ __launch_bounds__(kBlock) void k_gravity64_pairs_sum(const double* __restrict__ own,
+                                                                const double* __restrict__ react,
+                                                                double* __restrict__ out, int n, int tiles,
+                                                                int parts) {
+  const int i = blockIdx.x * kBlock + threadIdx.x, k = blockIdx.y;
+  if (i < n) out[4 * (size_t)i + k] = pairs64_sum<4>(own, react, i, k, tiles, parts);
+}
+
 void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_j, double eps, hipStream_t s,
                               int parts) {
   if (parts <= 0) parts = gravity64_parts(n_i);
   if (parts > 8) throw std::invalid_argument("gravity: at most 8 j-parts");
+  if (n_i == n_j && pairs64_fits(n_i)) {
+    double* ws = (double*)part;
+    launch_pairs64(GravityPairs{gpos, eps * eps}, n_i, parts, ws, s);
+    hipLaunchKernelGGL(k_gravity64_pairs_sum, dim3(ceil_div(n_i, kBlock), 4), dim3(kBlock), 0, s, ws,
+                       ws + pairs64_own(n_i, parts), (double*)out, n_i, pairs64_tiles(n_i), parts);
+    CS_CHECK_LAUNCH();
+    return;
+  }
   const int chunk = ceil_div(ceil_div(n_j, parts), kG64Tile) * kG64Tile;
   hipLaunchKernelGGL(k_gravity64_plummer, dim3(ceil_div(n_i, kGravBlock) * parts), dim3(kGravBlock), 0, s, gpos,
                      parts > 1 ? part : out, n_i, n_j, parts, chunk, eps * eps);
