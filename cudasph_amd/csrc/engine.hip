@@ -131,8 +131,8 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
     ghi_.alloc(nd_);
     glo_.alloc(nd_);
     gvel32_.alloc(nd_);
-    gpart_.alloc(2 * kGravMixedParts * (size_t)gravity_mixed_pieces(nd_) * nd_);
-    gmass_.alloc(2 + 2 * (size_t)ceil_div(n_, kBlock) + 8);
+    gpart_.alloc(mixed_part_words(nd_));
+    gmass_.alloc(2 + 2 * (size_t)ceil_div(n_, kBlock));
     // far-field records: 64-record sub-tiles, then cells of 16384, 4096, 1024, 256,
     // then the sub-tiles' 32-record halves
     gmom_.alloc(52 * ((size_t)ceil_div(nd_, 64) + ceil_div(nd_, 16384) + ceil_div(nd_, 4096) + ceil_div(nd_, 1024) +

@@ -18,6 +18,7 @@
 //   EXACT 1: 1/sqrt correctly rounded (bit-exact with the CPU restatement);
 //         0: hardware reciprocal square root (the reference uses rsqrtf)
 //   HILO  positions carry low words (mixed form): r_ij = (hi_i-hi_j)+(lo_i-lo_j)
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.h"
@@ -949,23 +950,19 @@ __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx,
 // partial acceleration, 1 subtraction for the potential.  With every mass
 // equal, tile-form sub-tiles skip r altogether (the expanded body below).
 //
+// This kernel evaluates every ordered pair: with the far field, with a
+// measurement switch, and below kMixedPairsMinN particles
+// (k_gravity_mixed_pairs otherwise).
 // Grid: `parts` j-parts per i-block, block b = i_block * parts + part.  Part p
 // takes the units p, p + parts, ... of j_unit records: tiles of 256, so that
 // the sub-tiles near an i-block, which are slower, fall to its parts evenly
 // (one contiguous unit per part below two tiles each, and for the far field,
 // whose cells must lie inside a part).  Workgroups are dispatched round-robin
-// over the 8 XCDs, so with a multiple of 8 parts each XCD streams only its 1/8
-// of the j-set (4 MiB of hi+lo records at N = 2^20), which its L2 holds;
-// without the split every XCD streams the whole j-set and re-fetches it from
-// HBM.  Each block writes its compensated (hi, lo) partial sums;
-// k_gravity_combine adds the parts in order.  The engine's parts are divided
-// further below kMixedQueueMaxN, since with 8 the last blocks ran alone for
-// long (65 536 particles: 4.9 wavefronts per SIMD in the mean of 8).  Gravity
-// alone, ms, contiguous 8 / tiles 8 / 16 / 24 / 40 parts: 16 384 particles 0.213
-// / 0.214 / 0.165 / 0.175 / 0.186, 32 768: 0.578 / 0.572 / 0.554 / 0.530 / 0.524,
-// 65 536: 1.95 / 1.89 / 1.72 / 1.67 / 1.65, 131 072: 6.05 / 5.81 / 5.48 / 5.25 /
-// 5.21, 250 007: 18.6 / 18.4 / 17.8 / 17.3 / 17.2, 500 000: 66.0 / 65.4 / 63.9 /
-// 63.0 / 62.6, 2^20: 274.6 / 272.3 / 271.1.
+// over the 8 XCDs, so with 8 parts part p runs on XCD p and each XCD streams
+// only its 1/8 of the j-set (4 MiB of hi+lo records at N = 2^20), which its L2
+// holds; without the split every XCD streams the whole j-set and re-fetches it
+// from HBM.  Each block writes its compensated (hi, lo) partial sums;
+// k_gravity_combine adds the parts in order.
 // The far-field instantiation holds the 48 moment words of an expansion in
 // VGPRs next to the pairwise state: left alone the compiler takes 127
 // registers (4 wavefronts per SIMD); capped at 5 wavefronts it fits 96
@@ -973,14 +970,12 @@ __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx,
 // slower).  The pairwise instantiation is left unbounded (63 registers, 8
 // wavefronts).
 template <int JT, bool FAR>
-__device__ __forceinline__ void mixed_plummer_item(const F4* __restrict__ hi, const F4* __restrict__ lo,
-                                                   F4* __restrict__ part_hi, F4* __restrict__ part_lo, int n_i,
-                                                   int n_j, int j_unit, float eps2, int split_only,
-                                                   const float* __restrict__ mass_range,
-                                                   const float* __restrict__ mom, const FarRatios& far_q2,
-                                                   const float* __restrict__ cells,
-                                                   const float* __restrict__ halves, int n_real, int parts,
-                                                   int part, int i_block) {
+__global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(FAR ? 5 : 8)))
+void k_gravity_mixed_plummer(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ part_hi,
+                             F4* __restrict__ part_lo, int n_i, int n_j, int j_unit, float eps2, int split_only,
+                             const float* __restrict__ mass_range, const float* __restrict__ mom,
+                             FarRatios far_q2, const float* __restrict__ cells,
+                             const float* __restrict__ halves, int n_real, int parts) {
   // every mass equal (mass_range = {min, max} over the real particles): the
   // pair body drops its mass factor and k_gravity_combine scales by m once;
   // padding records sit at 1e30, where r^2 overflows and rsq returns 0, so
@@ -999,7 +994,8 @@ __device__ __forceinline__ void mixed_plummer_item(const F4* __restrict__ hi, co
   __shared__ float s_r2[kSub];
   __shared__ __align__(16) float s_mom[kSub][FAR ? kMomWords : 1];
   static_assert(kTile == 64 && JT % kGravBlock == 0, "each wavefront stages whole sub-tiles");
-  const int i = i_block * kGravBlock + threadIdx.x;
+  const int part = blockIdx.x % parts;
+  const int i = (blockIdx.x / parts) * kGravBlock + threadIdx.x;
   const int ii = i < n_i ? i : n_i - 1;
   const int lane = threadIdx.x & 63;
   const F4 pi = hi[ii], li = lo[ii];
@@ -1267,71 +1263,303 @@ __device__ __forceinline__ void mixed_plummer_item(const F4* __restrict__ hi, co
   }
 }
 
-// one block per item (i_block, part)
-template <int JT, bool FAR>
-__global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(FAR ? 5 : 8)))
-void k_gravity_mixed_plummer(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ part_hi,
-                             F4* __restrict__ part_lo, int n_i, int n_j, int j_unit, float eps2, int split_only,
-                             const float* __restrict__ mass_range, const float* __restrict__ mom,
-                             FarRatios far_q2, const float* __restrict__ cells,
-                             const float* __restrict__ halves, int n_real, int parts) {
-  mixed_plummer_item<JT, FAR>(hi, lo, part_hi, part_lo, n_i, n_j, j_unit, eps2, split_only, mass_range, mom, far_q2,
-                              cells, halves, n_real, parts, blockIdx.x % parts, blockIdx.x / parts);
+// The mixed form with each pair of particles evaluated once for both: tiles of
+// 512 meet each other once, as the tiles of pairs64.h do (order of tiles and
+// rows, rotation of the reactions, slots).  A lane keeps two particles, so the
+// rotation of a record's reactions, one move per component, serves two pairs; a
+// wavefront's 128 particles choose the body per sub-tile as above:
+//  expanded: s3 (d_j, 1) for i and s3 (d_i, 1) for j, 16 VALU and a rsq for the
+//            two interactions in place of 22 and 2; the reaction on j is
+//            sum s3 d_i - d_j sum s3, |d_i| >= 3 |d_j|;
+//  split:    r once, 3 FMAs for each.
+// A move between lanes takes 4.2 cycles of a SIMD and, like a transcendental
+// operation, holds up the other wavefronts where vector operations directly
+// follow it (3 multiplies and a move: 16.4 cycles against 4 x 2.1), so the moves
+// of a step stand together between scalar instructions, and so do its two
+// v_rsq_f32.
+// A wavefront's reaction on a sub-tile is a plain FP32 sum of 4 sums of 32 terms
+// (one sum of 128 had twice the rounding error of a particle's own sums of 64);
+// the four wavefronts' are added and written, and
+// k_gravity_mixed_pairs_sum adds a particle's own (hi, lo) sums and its
+// reactions in two-sums, in a fixed order.
+struct Reaction {
+  float x = 0.f, y = 0.f, z = 0.f, w = 0.f, s = 0.f;
+  // to the previous lane of the row of 16 (cyclic), with the record it is for
+  __device__ __forceinline__ void turn() {
+    asm("s_nop 1\n\t"
+        "v_mov_b32_dpp %0, %0 row_ror:15 row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %1, %1 row_ror:15 row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %2, %2 row_ror:15 row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %3, %3 row_ror:15 row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %4, %4 row_ror:15 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0"
+        : "+v"(x), "+v"(y), "+v"(z), "+v"(w), "+v"(s));
+  }
+  __device__ __forceinline__ void add(const Reaction& r) {
+    x += r.x;
+    y += r.y;
+    z += r.z;
+    w += r.w;
+    s += r.s;
+  }
+  __device__ __forceinline__ void next_row(int from) {
+    x = __shfl(x, from);
+    y = __shfl(y, from);
+    z = __shfl(z, from);
+    w = __shfl(w, from);
+    s = __shfl(s, from);
+  }
+};
+
+// two rsq_spaced in one
+__device__ __forceinline__ void rsq_spaced(float (&v)[2]) {
+  float a, b;
+  asm("s_setprio 1\n\tv_rsq_f32 %0, %2\n\tv_rsq_f32 %1, %3\n\ts_setprio 0" : "=&v"(a), "=v"(b) : "v"(v[0]), "v"(v[1]));
+  v[0] = a;
+  v[1] = b;
 }
 
-// Few particles: a limited number of blocks (gravity_mixed_blocks) take the
-// items from 8 queues, item t from queue t % 8, so a block starts with the
-// parts of its XCD and goes on with the others' at the end.  queue holds 8
-// zeroed counters.  With one block per item, 65 536 particles fill every
-// wavefront slot of the GPU until gravity ends, and the SPH passes of the other
-// stream wait for it, one after another; blocks that stay leave room for them
-// from the start, and items smaller than a block's share end together.
-template <int JT>
-__global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(8)))
-void k_gravity_mixed_queue(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ part_hi,
-                           F4* __restrict__ part_lo, int n_i, int n_j, int j_unit, float eps2, int split_only,
-                           const float* __restrict__ mass_range, int n_real, int parts, int n_items,
-                           int* __restrict__ queue) {
-  __shared__ int s_item;
-  int q = 0;   // queues found empty
-  for (;;) {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int t = -1;
-      for (; q < 8; ++q) {
-        const int x = (blockIdx.x + q) & 7, k = atomicAdd(&queue[x], 1);
-        if (8 * k + x < n_items) {
-          t = 8 * k + x;
-          break;
+// 4 wavefronts per SIMD (128 VGPRs; the folded sums wait in scratch between
+// sub-tiles): 5 reload in the loop (steps of 65 536 particles 1.72 against 1.68
+// ms, 80 000: 2.66 / 2.35), 3 issue worse (2^20: 235 against 229 ms).
+constexpr int kMixTile = 512, kMixHalf = 256;
+__global__ __launch_bounds__(kMixHalf) __attribute__((amdgpu_waves_per_eu(4)))
+void k_gravity_mixed_pairs(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ own_hi,
+                           F4* __restrict__ own_lo, F4* __restrict__ react, int n, int n_real, int tiles, int parts,
+                           int d0, int d1, float eps2, const float* __restrict__ mass_range) {
+  static_assert(kMixHalf == 4 * kTile, "a wavefront stages a sub-tile");
+  const bool uniform = mass_range[0] == mass_range[1];
+  // records relative to their sub-tile's origin: -2 d_j, |d_j|^2 (equal masses)
+  // or d_j, m; twice in a row of 16, whose place 31 stays free and holds the
+  // sub-tile's origin and squared radius (so 5 blocks share a CU's LDS)
+  __shared__ F4 s_rel[kMixHalf / 16][32], s_hi[kMixHalf], s_lo[kMixHalf], s_acc[4][kMixHalf];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c16 = lane & 15, row = lane >> 4;
+  const int tile = (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;
+  const int np = tiles * kMixTile;
+  const auto load = [&](int i, F4& h, F4& l) {
+    if (i < n) {
+      h = hi[i];
+      l = lo[i];
+    } else {   // as the padding records: r^2 overflows and rsq returns 0
+      h = {1e30f, 1e30f, 1e30f, 0.f};
+      l = {0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  const int i0 = tile * kMixTile + 2 * kTile * wave + lane;
+  F4 pi[2], li[2];
+  GAcc<float, 1> a[2][4];
+  for (int p = 0; p < 2; ++p) load(i0 + kTile * p, pi[p], li[p]);
+  for (int d = d0 + part; d < d1; d += parts) {
+    if (2 * d == tiles && tile >= d) break;   // the opposite tile's block has this pair of tiles
+    const int other = tile + d < tiles ? tile + d : tile + d - tiles;
+    for (int j_half = other * kMixTile; j_half < (other + 1) * kMixTile; j_half += kMixHalf) {
+      __syncthreads();
+      {
+        const int sub0 = j_half + wave * kTile, nr = min(kTile, n_real - sub0);
+        F4 h, l;
+        load(sub0 + lane, h, l);
+        if (nr > 0) {
+          const F4 c = hi[sub0 + nr / 2];
+          F4 dj{(h.x - c.x) + l.x, (h.y - c.y) + l.y, (h.z - c.z) + l.z, h.w};
+          float r2 = __builtin_fmaf(dj.x, dj.x, __builtin_fmaf(dj.y, dj.y, dj.z * dj.z));
+          if (uniform) dj = {-2.f * dj.x, -2.f * dj.y, -2.f * dj.z, r2};
+          s_rel[tid >> 4][c16] = dj;
+          if (c16 < 15) s_rel[tid >> 4][c16 + 16] = dj;
+          s_hi[tid] = h;
+          s_lo[tid] = l;
+          for (int o = 32; o > 0; o >>= 1) r2 = fmaxf(r2, __shfl_xor(r2, o));
+          if (lane == 0) s_rel[4 * wave][31] = {c.x, c.y, c.z, r2};
+        } else if (lane == 0) {
+          s_rel[4 * wave][31].w = -1.f;   // only padding
         }
       }
-      s_item = t;
+      __syncthreads();
+      for (int sub = 0; sub < 4; ++sub) {
+        Reaction R, total;   // of 16 records' steps, of all
+        const F4 c = s_rel[4 * sub][31];
+        if (c.w >= 0.f) {
+          float dx[2], dy[2], dz[2], di2[2];
+          for (int p = 0; p < 2; ++p) {
+            dx[p] = (pi[p].x - c.x) + li[p].x;
+            dy[p] = (pi[p].y - c.y) + li[p].y;
+            dz[p] = (pi[p].z - c.z) + li[p].z;
+            di2[p] = __builtin_fmaf(dx[p], dx[p], __builtin_fmaf(dy[p], dy[p], dz[p] * dz[p]));
+          }
+          const bool tile_form = d > 0 && __all(fminf(di2[0], di2[1]) >= 9.9f * c.w);
+          // body(group, step) over the 64 records, the reactions moving with them
+          const auto sweep = [&](auto&& body) {
+            for (int q = 0; q < 4; ++q) {
+              const int grp = sub * 4 + ((row + q) & 3);
+#pragma unroll
+              for (int s = 0; s < 16; ++s) {
+                body(grp, s);
+                R.turn();
+              }
+              total.add(R);
+              R = Reaction{};
+              total.next_row((lane + 16) & 63);
+            }
+            R = total;
+          };
+          const auto split = [&](int j, float (&rx)[2], float (&ry)[2], float (&rz)[2], float (&inv)[2]) {
+            const F4 pj = s_hi[j], lj = s_lo[j];
+            for (int p = 0; p < 2; ++p) {
+              rx[p] = (pi[p].x - pj.x) + (li[p].x - lj.x);
+              ry[p] = (pi[p].y - pj.y) + (li[p].y - lj.y);
+              rz[p] = (pi[p].z - pj.z) + (li[p].z - lj.z);
+              inv[p] = __builtin_fmaf(rx[p], rx[p], __builtin_fmaf(ry[p], ry[p], __builtin_fmaf(rz[p], rz[p], eps2)));
+            }
+            rsq_spaced(inv);
+            return pj.w;
+          };
+          if (d == 0) {   // all ordered pairs of the tile, without reactions
+            for (int j = sub * kTile; j < sub * kTile + kTile; ++j) {
+              float rx[2], ry[2], rz[2], inv[2];
+              const float mj = split(j, rx, ry, rz, inv);
+              for (int p = 0; p < 2; ++p) {
+                const float m = uniform ? inv[p] : mj * inv[p], s3 = m * (inv[p] * inv[p]);
+                a[p][0].fsub(rx[p], s3);
+                a[p][1].fsub(ry[p], s3);
+                a[p][2].fsub(rz[p], s3);
+                a[p][3].sub(m);
+              }
+            }
+          } else if (uniform && tile_form) {
+            float sa[2] = {}, mx[2] = {}, my[2] = {}, mz[2] = {};   // of -2 d_j
+            for (int p = 0; p < 2; ++p) di2[p] += eps2;
+            sweep([&](int grp, int s) {
+              const F4 pj = s_rel[grp][c16 + s];
+              float inv[2];
+              for (int p = 0; p < 2; ++p)
+                inv[p] = __builtin_fmaf(pj.x, dx[p], __builtin_fmaf(pj.y, dy[p], __builtin_fmaf(pj.z, dz[p], di2[p] + pj.w)));
+              rsq_spaced(inv);
+              for (int p = 0; p < 2; ++p) {
+                const float s3 = inv[p] * (inv[p] * inv[p]);
+                sa[p] += s3;
+                mx[p] = __builtin_fmaf(pj.x, s3, mx[p]);
+                my[p] = __builtin_fmaf(pj.y, s3, my[p]);
+                mz[p] = __builtin_fmaf(pj.z, s3, mz[p]);
+                a[p][3].sub(inv[p]);
+                R.s += s3;
+                R.x = __builtin_fmaf(dx[p], s3, R.x);
+                R.y = __builtin_fmaf(dy[p], s3, R.y);
+                R.z = __builtin_fmaf(dz[p], s3, R.z);
+                R.w -= inv[p];
+              }
+            });
+            for (int p = 0; p < 2; ++p) {
+              a[p][0].part += __builtin_fmaf(-dx[p], sa[p], -0.5f * mx[p]);
+              a[p][1].part += __builtin_fmaf(-dy[p], sa[p], -0.5f * my[p]);
+              a[p][2].part += __builtin_fmaf(-dz[p], sa[p], -0.5f * mz[p]);
+            }
+            const F4 dj = s_rel[sub * 4 + row][c16];
+            R.x = __builtin_fmaf(0.5f * dj.x, R.s, R.x);
+            R.y = __builtin_fmaf(0.5f * dj.y, R.s, R.y);
+            R.z = __builtin_fmaf(0.5f * dj.z, R.s, R.z);
+          } else if (uniform) {
+            sweep([&](int grp, int s) {
+              float rx[2], ry[2], rz[2], inv[2];
+              split(grp * 16 + ((c16 + s) & 15), rx, ry, rz, inv);
+              for (int p = 0; p < 2; ++p) {
+                const float s3 = inv[p] * (inv[p] * inv[p]);
+                a[p][0].fsub(rx[p], s3);
+                a[p][1].fsub(ry[p], s3);
+                a[p][2].fsub(rz[p], s3);
+                a[p][3].sub(inv[p]);
+                R.x = __builtin_fmaf(rx[p], s3, R.x);
+                R.y = __builtin_fmaf(ry[p], s3, R.y);
+                R.z = __builtin_fmaf(rz[p], s3, R.z);
+                R.w -= inv[p];
+              }
+            });
+          } else {
+            sweep([&](int grp, int s) {
+              float rx[2], ry[2], rz[2], inv[2];
+              float mj;
+              if (tile_form) {
+                const F4 pj = s_rel[grp][c16 + s];
+                for (int p = 0; p < 2; ++p) {
+                  rx[p] = dx[p] - pj.x;
+                  ry[p] = dy[p] - pj.y;
+                  rz[p] = dz[p] - pj.z;
+                  inv[p] =
+                      __builtin_fmaf(rx[p], rx[p], __builtin_fmaf(ry[p], ry[p], __builtin_fmaf(rz[p], rz[p], eps2)));
+                }
+                rsq_spaced(inv);
+                mj = pj.w;
+              } else {
+                mj = split(grp * 16 + ((c16 + s) & 15), rx, ry, rz, inv);
+              }
+              for (int p = 0; p < 2; ++p) {
+                const float i2 = inv[p] * inv[p], wj = mj * inv[p], wi = pi[p].w * inv[p], sj = wj * i2, si = wi * i2;
+                a[p][0].fsub(rx[p], sj);
+                a[p][1].fsub(ry[p], sj);
+                a[p][2].fsub(rz[p], sj);
+                a[p][3].sub(wj);
+                R.x = __builtin_fmaf(rx[p], si, R.x);
+                R.y = __builtin_fmaf(ry[p], si, R.y);
+                R.z = __builtin_fmaf(rz[p], si, R.z);
+                R.w -= wi;
+              }
+            });
+          }
+        }
+        if (sub & 1)
+          for (int p = 0; p < 2; ++p)
+            for (int k = 0; k < 4; ++k) a[p][k].tile_end();
+        s_acc[wave][sub * kTile + lane] = {R.x, R.y, R.z, R.w};
+      }
+      if (d == 0) continue;
+      __syncthreads();
+      const F4 r0 = s_acc[0][tid], r1 = s_acc[1][tid], r2 = s_acc[2][tid], r3 = s_acc[3][tid];
+      react[(size_t)(d - d0) * np + j_half + tid] = {(r0.x + r1.x) + (r2.x + r3.x), (r0.y + r1.y) + (r2.y + r3.y),
+                                                     (r0.z + r1.z) + (r2.z + r3.z), (r0.w + r1.w) + (r2.w + r3.w)};
     }
-    __syncthreads();
-    const int t = __builtin_amdgcn_readfirstlane(s_item);
-    if (t < 0) break;
-    mixed_plummer_item<JT, false>(hi, lo, part_hi, part_lo, n_i, n_j, j_unit, eps2, split_only, mass_range, nullptr,
-                                  FarRatios{}, nullptr, nullptr, n_real, parts, t % parts, t / parts);
+  }
+  for (int p = 0; p < 2; ++p) {
+    const size_t o = (size_t)part * np + i0 + kTile * p;
+    own_hi[o] = {a[p][0].v.hi, a[p][1].v.hi, a[p][2].v.hi, a[p][3].v.hi};
+    own_lo[o] = {a[p][0].v.lo, a[p][1].v.lo, a[p][2].v.lo, a[p][3].v.lo};
   }
 }
 
-static int gpu_cus() {
-  int dev = 0, cus = 0;
-  CS_HIP(hipGetDevice(&dev));
-  CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  return cus;
-}
-
-// Blocks per CU of the queue kernel, 0 for one block per item.  Measured, ms
-// per mixed step, one block per item (8 parts) / 2 / 3 / 4 / 6 / 7 blocks per CU
-// (24 parts): 16 384 particles 0.482 / 0.477 / 0.514 / 0.545 / 0.673 / 0.672,
-// 24 000: 0.541 / 0.561 / 0.542 / 0.559 / 0.749 / 0.740, 32 768: 0.668 / 0.888 /
-// 0.738 / 0.667 / 0.951 / 0.998, 49 152: 1.281 / 1.693 / 1.337 / 1.186 / 1.233 /
-// 1.327, 65 536: 1.913 / 2.785 / 2.146 / 1.907 / 1.809 / 2.010, 131 072: 6.15 /
-// 9.52 / 7.13 / 6.20 / 6.00 / 6.27; 6 and 7 at 200 000: 12.70 / 12.72 / 12.91,
-// 400 000: 42.5 / 43.7 / 43.6.
-static int gravity_mixed_blocks(int n_j) {
-  return n_j < 20480 ? 2 : n_j < 28672 ? 3 : n_j < 57344 ? 4 : n_j < kMixedQueueMaxN ? 6 : 0;
+// The offsets [d0, d1) of a particle: own sums and reactions, added to what the
+// offsets before left in acc (hi, then lo); the last call writes the result.
+__global__ __launch_bounds__(kBlock) void k_gravity_mixed_pairs_sum(const F4* __restrict__ own_hi,
+                                                                    const F4* __restrict__ own_lo,
+                                                                    const F4* __restrict__ react,
+                                                                    F4* __restrict__ acc, F4* __restrict__ out, int n,
+                                                                    int tiles, int parts, int d0, int d1, int last,
+                                                                    const float* __restrict__ mass_range) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int np = tiles * kMixTile;
+  DR a[4] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
+  const auto add = [&](const F4& v) {
+    dr_add(a[0], v.x);
+    dr_add(a[1], v.y);
+    dr_add(a[2], v.z);
+    dr_add(a[3], v.w);
+  };
+  if (d0 > 0) {
+    add(acc[i]);
+    add(acc[np + i]);
+  }
+  for (int p = 0; p < parts; ++p) {
+    add(own_hi[(size_t)p * np + i]);
+    add(own_lo[(size_t)p * np + i]);
+  }
+  int d_end = d1;
+  if (2 * (d1 - 1) == tiles && i / kMixTile < tiles / 2) --d_end;   // met by the opposite tile's block
+#pragma unroll 4
+  for (int d = max(d0, 1); d < d_end; ++d) add(react[(size_t)(d - d0) * np + i]);
+  if (!last) {
+    acc[i] = {a[0].hi, a[1].hi, a[2].hi, a[3].hi};
+    acc[np + i] = {a[0].lo, a[1].lo, a[2].lo, a[3].lo};
+    return;
+  }
+  const float m = mass_range[0] == mass_range[1] ? mass_range[0] : 1.f;
+  out[i] = {m * (a[0].hi + a[0].lo), m * (a[1].hi + a[1].lo), m * (a[2].hi + a[2].lo), m * (a[3].hi + a[3].lo)};
 }
 
 // sum of the `parts` compensated partials of each i, in part order, times
@@ -1381,9 +1609,7 @@ __global__ __launch_bounds__(kBlock) void k_mass_range_partials(const F4* __rest
   }
 }
 __global__ __launch_bounds__(kBlock) void k_mass_range_final(const float* __restrict__ partial, int nb,
-                                                             float* __restrict__ out,
-                                                             int* __restrict__ queue) {
-  if (threadIdx.x < 8) queue[threadIdx.x] = 0;
+                                                             float* __restrict__ out) {
   __shared__ float smin[kBlock], smax[kBlock];
   float lo = partial[0], hi = partial[1];
   for (int b = threadIdx.x; b < nb; b += kBlock) {
@@ -1496,6 +1722,13 @@ __global__ __launch_bounds__(kBlock) void k_gravity64_combine(const D4* __restri
     a = {a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
   }
   out[i] = a;
+}
+
+static int gpu_cus() {
+  int dev = 0, cus = 0;
+  CS_HIP(hipGetDevice(&dev));
+  CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return cus;
 }
 
 // Parts for the passes of the FP64 form: of 2 .. 8 (1 from 2^19 particles on)
@@ -1620,6 +1853,18 @@ void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, i
   CS_CHECK_LAUNCH();
 }
 
+int mixed_pairs_chunk(int n) {
+  const int tiles = ceil_div(n, kMixTile);
+  const size_t slot = sizeof(F4) * kMixTile * (size_t)tiles;
+  return (int)std::min<size_t>(tiles / 2 + 1, std::max<size_t>(1, ((size_t)2 << 30) / slot));
+}
+size_t mixed_part_words(int n) {
+  const size_t items = 2 * kGravMixedParts * (size_t)n;
+  if (!mixed_pairs_fit(n)) return items;
+  const size_t np = (size_t)ceil_div(n, kMixTile) * kMixTile;
+  return std::max(items, (2 * kGravMixedParts + 2 + mixed_pairs_chunk(n)) * np);
+}
+
 void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F4* part, float* mass_range,
                           float* moments, float far_ratio, float far_grade, int n_i, int n_j, int n_real,
                           int soft, float eps, int split_only, hipStream_t s, int parts) {
@@ -1627,19 +1872,33 @@ void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F
   if (soft == 0) {
     hipLaunchKernelGGL(k_gravity_mixed_spline, grid, block, 0, s, hi, lo, gvel, out, n_i, n_j);
   } else {
-    // mass_range: 2 floats of result followed by 2 per block of n_real and the
-    // 8 item queues, cleared with the result
+    // mass_range: 2 floats of result followed by 2 per block of n_real
     const int nb = ceil_div(n_real, kBlock);
-    int* queue = (int*)(mass_range + 2 + 2 * nb);
     hipLaunchKernelGGL(k_mass_range_partials, dim3(nb), dim3(kBlock), 0, s, hi, n_real, mass_range + 2);
     CS_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_mass_range_final, dim3(1), dim3(kBlock), 0, s, mass_range + 2, nb, mass_range,
-                       queue);
+    hipLaunchKernelGGL(k_mass_range_final, dim3(1), dim3(kBlock), 0, s, mass_range + 2, nb, mass_range);
     CS_CHECK_LAUNCH();
+    if (n_i == n_j && split_only == 0 && mixed_pairs_fit(n_j)) {
+      if (parts <= 0) parts = kGravMixedParts;
+      if (parts > kGravMixedParts) throw std::invalid_argument("gravity: at most 8 j-parts");
+      const int tiles = ceil_div(n_j, kMixTile), np = tiles * kMixTile, d_end = tiles / 2 + 1,
+                chunk = mixed_pairs_chunk(n_j);
+      F4 *own_hi = part, *own_lo = own_hi + (size_t)parts * np, *acc = own_lo + (size_t)parts * np,
+         *react = acc + 2 * (size_t)np;
+      for (int d0 = 0; d0 < d_end; d0 += chunk) {
+        const int d1 = min(d_end, d0 + chunk);
+        hipLaunchKernelGGL(k_gravity_mixed_pairs, dim3(tiles * parts), dim3(kMixHalf), 0, s, hi, lo, own_hi, own_lo,
+                           react, n_j, n_real, tiles, parts, d0, d1, eps * eps, mass_range);
+        CS_CHECK_LAUNCH();
+        hipLaunchKernelGGL(k_gravity_mixed_pairs_sum, dim3(ceil_div(n_i, kBlock)), dim3(kBlock), 0, s, own_hi, own_lo,
+                           react, acc, out, n_i, tiles, parts, d0, d1, (int)(d1 == d_end), mass_range);
+        CS_CHECK_LAUNCH();
+      }
+      return;
+    }
     const bool far = (split_only & 16) && moments;
     if (parts <= 0 || far) parts = kGravMixedParts;
     if (parts > kGravMixedParts) throw std::invalid_argument("gravity: at most 8 j-parts");
-    if (!far) parts *= gravity_mixed_pieces(n_j);
     int unit = ceil_div(ceil_div(n_j, parts), kTile) * kTile;
     if (!far && unit >= 2 * kJTileMixed) unit = kJTileMixed;
     F4* part_hi = part;
@@ -1685,10 +1944,6 @@ void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F
       hipLaunchKernelGGL((k_gravity_mixed_plummer<kJTileMixed, true>), dim3(n_items), block, 0, s, hi, lo, part_hi,
                          part_lo, n_i, n_j, unit, eps * eps, split_only, mass_range, moments, fq, cells, halves,
                          n_real, parts);
-    else if (const int per_cu = gravity_mixed_blocks(n_j))
-      hipLaunchKernelGGL((k_gravity_mixed_queue<kJTileMixed>), dim3(min(n_items, per_cu * gpu_cus())), block, 0, s,
-                         hi, lo, part_hi, part_lo, n_i, n_j, unit, eps * eps, split_only, mass_range, n_real, parts,
-                         n_items, queue);
     else
       hipLaunchKernelGGL((k_gravity_mixed_plummer<kJTileMixed, false>), dim3(n_items), block, 0, s, hi, lo, part_hi,
                          part_lo, n_i, n_j, unit, eps * eps, split_only, mass_range, nullptr, fq, nullptr, nullptr,

@@ -77,22 +77,25 @@ void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, i
 int gravity64_parts(int n_i);
 void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_j, double eps, hipStream_t s,
                               int parts = 0);
-// part: scratch of 2 * kGravMixedParts * gravity_mixed_pieces(n_j) * n_i records
-// (per-j-part partial sums, Plummer only); mass_range: scratch of
-// 10 + 2 * ceil(n_real / 256) floats ({min, max} of the real particles' masses,
-// per-block partials and 8 work queues)
+// part: scratch of mixed_part_words(n_j) records (Plummer only): the parts' sums,
+// and where pairs are taken once running sums and a chunk of reactions (at
+// most 2 GiB); mass_range: scratch of 2 + 2 * ceil(n_real / 256) floats ({min, max}
+// of the real particles' masses, then per-block partials)
 // moments: scratch of 52 floats per 64-record j sub-tile followed by 52 per
 // cell of 16384, 4096, 1024 and 256 records and, with split_only bit 6, 52
 // per 32-record half sub-tile (the optional multipole far
 // field, split_only bit 4, taken where every lane of a wavefront is
 // far_ratio radii away, the ratio at a level of C records scaled by
 // (C / 16384)^far_grade; may be null otherwise)
-// parts: the number of j-parts, 1 .. kGravMixedParts; 0 for the most.  Each
-// part is cut into gravity_mixed_pieces(n_j) (not with the far field).
+// parts: the number of j-parts, 1 .. kGravMixedParts; 0 for the most.
 constexpr int kGravMixedParts = 8;   // one per XCD
-constexpr int kMixedQueueMaxN = 196608;
-// (few particles: fewer partial sums to combine)
-inline int gravity_mixed_pieces(int n_j) { return n_j >= 8192 && n_j < kMixedQueueMaxN ? 3 : 1; }
+// Pairs taken once (k_gravity_mixed_pairs).  Steps, ms, every ordered pair / once:
+// 8 192 particles 0.449 / 0.407, 16 384: 0.483 / 0.469, 32 768: 0.669 / 0.630, 65 536:
+// 1.81 / 1.68, 131 072: 6.05 / 4.95, 250 007: 18.9 / 16.1, 2^20: 274 / 236.
+constexpr int kMixedPairsMinN = 8192;   // (from 2 048 to here both are as fast)
+inline bool mixed_pairs_fit(int n) { return n >= kMixedPairsMinN; }
+int mixed_pairs_chunk(int n);
+size_t mixed_part_words(int n);   // F4s of `part`
 void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F4* part, float* mass_range,
                           float* moments, float far_ratio, float far_grade, int n_i, int n_j, int n_real,
                           int soft, float eps, int split_only, hipStream_t s, int parts = 0);

@@ -1,26 +1,29 @@
 """Mixed Plummer gravity at the sizes where its launch changes: one contiguous
-unit of records per part or tiles of 256 dealt out to the parts, blocks that
-take items from the queues or one block per item, and 2, 3, 4 or 6 of them per
-CU.  Accelerations and potentials of sampled particles against an FP64 direct
-sum over the same (split) positions."""
+unit of records per part or tiles of 256 dealt out to the parts; pairs taken
+once, with odd and even counts of tiles of 512, a last tile with one particle,
+and unequal masses.  Accelerations and potentials of sampled particles against
+an FP64 direct sum over the same (split) positions."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-# tiles in place of units from 512 records per part on (8 parts below 8 192
-# particles: 3 585; 24 parts above: 10 753); queues below 196 608
-@pytest.mark.parametrize("n", [3, 64, 257, 1000, 3583, 3585, 8191, 8193, 10751, 10753, 20479, 20481, 28673, 57343, 57345, 65536, 196607,
-                               196609])
-def test_items_cover_every_pair(cs, n):
-    print(f"mixed gravity items n={n}", flush=True)
+# tiles in place of units from 512 records per part on (3 585); pairs taken once
+# from 8 192; 17, 18, 33 tiles
+@pytest.mark.parametrize("masses", ["equal", "unequal"])
+@pytest.mark.parametrize("n", [3, 64, 257, 1000, 3583, 3585, 8191, 8192, 8193, 8704, 9216, 9217, 16385, 65536, 81921])
+def test_items_cover_every_pair(cs, n, masses):
+    print(f"mixed gravity items n={n} {masses}", flush=True)
     e = cs.make_engine("mixed", 2, n, 7, ph_sort=True)
-    for _ in range(2):   # the second evaluation starts from cleared queues
-        e.run_pass(cs.GRAVITY)
+    if masses == "unequal":
+        v = e.get("vel64")
+        v[:n, 3] *= 10.0 ** np.random.default_rng(n).uniform(-1, 1, n)
+        e.set("vel64", v)
+    e.run_pass(cs.GRAVITY)
     got = e.get("grav")[:n].astype(np.float64)
     x = e.get("pos64")[:n, :3]
-    m = e.get("vel")[:n, 3].astype(np.float64)
+    m = e.get("vel64")[:n, 3]
     eps2 = float(cs.preset_params(2, n).grav_eps) ** 2
     e.close()
     pick = np.unique(np.linspace(0, n - 1, min(n, 96)).astype(int))
