@@ -677,13 +677,16 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// the factors of the stored moments (far_field)
+constexpr float kTrM2 = 0.5f, kTrQ = 0.375f, kM2 = 3.f, kT3 = -1.5f, kQ = 7.5f, kM3 = -7.5f, kM4 = 17.5f;
+
 // record of sub-tile s: [0..2] centre-of-mass offset from the origin record
 // (the middle real record; its coordinates in [48..50]), [3] R^2, [4] M0
 // (0: no real record, the sub-tile is skipped), [5] tr M2,
 // [6] tr Q, [8..13] M2 (xx xy xz yy yz zz), [14..16] t3, [17..22] Q,
 // [23..32] M3 (xxx xxy xxz xyy xyz xzz yyy yyz yzz zzz), [33..47] M4
 // (xxxx xxxy xxxz xxyy xxyz xxzz xyyy xyyz xyzz xzzz yyyy yyyz yyzz yzzz
-// zzzz).  Masses as the kernel uses them (1 when every mass is equal);
+// zzzz), [5..47] times their factors.  Masses as the kernel uses them (1 when every mass is equal);
 // padding records (j >= n_real) are left out.  One wavefront per sub-tile.
 __global__ __launch_bounds__(kGravBlock) void k_subtile_moments(const F4* __restrict__ hi, const F4* __restrict__ lo,
                                                                 float* __restrict__ mom, int n_j, int n_real,
@@ -739,20 +742,20 @@ __global__ __launch_bounds__(kGravBlock) void k_subtile_moments(const F4* __rest
     r[2] = mz;
     r[3] = r2;
     r[4] = M0;
-    r[5] = M2[0] + M2[3] + M2[5];
-    r[6] = Q[0] + Q[3] + Q[5];
+    r[5] = kTrM2 * (M2[0] + M2[3] + M2[5]);
+    r[6] = kTrQ * (Q[0] + Q[3] + Q[5]);
     r[7] = 0.f;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) r[8 + k] = M2[k];
-    r[14] = M3[0] + M3[3] + M3[5];
-    r[15] = M3[1] + M3[6] + M3[8];
-    r[16] = M3[2] + M3[7] + M3[9];
+    for (int k = 0; k < 6; ++k) r[8 + k] = kM2 * M2[k];
+    r[14] = kT3 * (M3[0] + M3[3] + M3[5]);
+    r[15] = kT3 * (M3[1] + M3[6] + M3[8]);
+    r[16] = kT3 * (M3[2] + M3[7] + M3[9]);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) r[17 + k] = Q[k];
+    for (int k = 0; k < 6; ++k) r[17 + k] = kQ * Q[k];
 #pragma unroll
-    for (int k = 0; k < 10; ++k) r[23 + k] = M3[k];
+    for (int k = 0; k < 10; ++k) r[23 + k] = kM3 * M3[k];
 #pragma unroll
-    for (int k = 0; k < 15; ++k) r[33 + k] = M4[k];
+    for (int k = 0; k < 15; ++k) r[33 + k] = kM4 * M4[k];
     r[48] = c.x;
     r[49] = c.y;
     r[50] = c.z;
@@ -849,16 +852,16 @@ __global__ __launch_bounds__(kGravBlock) void k_cell_moments(const F4* __restric
     r[2] = (float)mz;
     r[3] = r2;
     r[4] = (float)m0;
-    r[5] = (float)(M2[0] + M2[3] + M2[5]);
-    r[6] = (float)(Q[0] + Q[3] + Q[5]);
+    r[5] = (float)(kTrM2 * (M2[0] + M2[3] + M2[5]));
+    r[6] = (float)(kTrQ * (Q[0] + Q[3] + Q[5]));
     r[7] = 0.f;
-    for (int k = 0; k < 6; ++k) r[8 + k] = (float)M2[k];
-    r[14] = (float)(M3[0] + M3[3] + M3[5]);
-    r[15] = (float)(M3[1] + M3[6] + M3[8]);
-    r[16] = (float)(M3[2] + M3[7] + M3[9]);
-    for (int k = 0; k < 6; ++k) r[17 + k] = (float)Q[k];
-    for (int k = 0; k < 10; ++k) r[23 + k] = (float)M3[k];
-    for (int k = 0; k < 15; ++k) r[33 + k] = (float)M4[k];
+    for (int k = 0; k < 6; ++k) r[8 + k] = (float)(kM2 * M2[k]);
+    r[14] = (float)(kT3 * (M3[0] + M3[3] + M3[5]));
+    r[15] = (float)(kT3 * (M3[1] + M3[6] + M3[8]));
+    r[16] = (float)(kT3 * (M3[2] + M3[7] + M3[9]));
+    for (int k = 0; k < 6; ++k) r[17 + k] = (float)(kQ * Q[k]);
+    for (int k = 0; k < 10; ++k) r[23 + k] = (float)(kM3 * M3[k]);
+    for (int k = 0; k < 15; ++k) r[33 + k] = (float)(kM4 * M4[k]);
     r[48] = c.x;
     r[49] = c.y;
     r[50] = c.z;
@@ -867,61 +870,61 @@ __global__ __launch_bounds__(kGravBlock) void k_cell_moments(const F4* __restric
 }
 
 // acceleration G = sum_j m_j (x_j - x_i) s^-3 and potential -sum_j m_j / s of
-// one sub-tile from its record M, at y = x_i - COM (order-4 expansion)
+// one sub-tile from its record M, at y = x_i - COM (order-4 expansion):
+//   sum m_j / s = sum_k g_k B_k and G = y sum_k g_(k+1) B_k + sum_k g_k V_k with
+//   V_2 = M2.y - t3 / 2, V_3 = (Q.y - M3.yy) / 2, V_4 = M4.yyy / 6,
+//   B_0 = M0, B_1 = tr M2 / 2, B_2 = y.M2.y / 2 - t3.y / 2 + tr Q / 8,
+//   B_3 = y.Q.y / 4 - M3.yyy / 6, B_4 = M4.yyyy / 24,
+// that is B_3 = y.(V_3 + Q.y / 4) / 3 and B_4 = y.V_4 / 4.  The kernel with the far
+// field is bound by the operations here, about two thirds of its VALU work.
+// The moments are stored with the factors (2 k - 1)!! of g_k, so that the G_k are
+// plain powers, and every line is a chain of multiply-adds: 141 operations
+// and a v_rsq_f32 (196 term by term).
 __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx, float yy, float yz, float eps2,
                                           float& gx, float& gy, float& gz, float& pot) {
-  const float s2 = __builtin_fmaf(yx, yx, __builtin_fmaf(yy, yy, __builtin_fmaf(yz, yz, eps2)));
-  const float inv = rsq_spaced(s2), i2 = inv * inv;
-  const float g0 = inv, g1 = -inv * i2, g2 = -3.f * g1 * i2, g3 = -5.f * g2 * i2, g4 = -7.f * g3 * i2,
-              g5 = -9.f * g4 * i2;
-  const float M0 = M[4], trM2 = M[5], trQ = M[6];
+  const auto fma = [](float a, float b, float c) { return __builtin_fmaf(a, b, c); };
+  const float s2 = fma(yx, yx, fma(yy, yy, fma(yz, yz, eps2)));
+  const float G0 = rsq_spaced(s2), h = -G0 * G0;
+  const float G1 = G0 * h, G2 = G1 * h, G3 = G2 * h, G4 = G3 * h, G5 = G4 * h;
   const float* m2 = M + 8;
   const float* t3 = M + 14;
   const float* Q = M + 17;
   const float* m3 = M + 23;
   const float* m4 = M + 33;
-  const float M2x = __builtin_fmaf(m2[0], yx, __builtin_fmaf(m2[1], yy, m2[2] * yz));
-  const float M2y = __builtin_fmaf(m2[1], yx, __builtin_fmaf(m2[3], yy, m2[4] * yz));
-  const float M2z = __builtin_fmaf(m2[2], yx, __builtin_fmaf(m2[4], yy, m2[5] * yz));
-  const float yM2y = __builtin_fmaf(M2x, yx, __builtin_fmaf(M2y, yy, M2z * yz));
-  const float Qx = __builtin_fmaf(Q[0], yx, __builtin_fmaf(Q[1], yy, Q[2] * yz));
-  const float Qy = __builtin_fmaf(Q[1], yx, __builtin_fmaf(Q[3], yy, Q[4] * yz));
-  const float Qz = __builtin_fmaf(Q[2], yx, __builtin_fmaf(Q[4], yy, Q[5] * yz));
-  const float yQy = __builtin_fmaf(Qx, yx, __builtin_fmaf(Qy, yy, Qz * yz));
-  const float t3y = __builtin_fmaf(t3[0], yx, __builtin_fmaf(t3[1], yy, t3[2] * yz));
+  const float V2x = fma(m2[0], yx, fma(m2[1], yy, fma(m2[2], yz, t3[0])));
+  const float V2y = fma(m2[1], yx, fma(m2[3], yy, fma(m2[4], yz, t3[1])));
+  const float V2z = fma(m2[2], yx, fma(m2[4], yy, fma(m2[5], yz, t3[2])));
+  const float B2 = fma(0.5f, fma(V2x + t3[0], yx, fma(V2y + t3[1], yy, (V2z + t3[2]) * yz)), M[6]);
   // quadratic monomials, off-diagonal ones doubled: (M3 . y y)_k
-  const float qxx = yx * yx, qxy = 2.f * yx * yy, qxz = 2.f * yx * yz, qyy = yy * yy, qyz = 2.f * yy * yz,
-              qzz = yz * yz;
-  auto dot6 = [&](float a, float b, float c, float d, float e, float f) {
-    return __builtin_fmaf(qxx, a, __builtin_fmaf(qxy, b, __builtin_fmaf(qxz, c,
-           __builtin_fmaf(qyy, d, __builtin_fmaf(qyz, e, qzz * f)))));
+  const float yx2 = 2.f * yx, yy2 = 2.f * yy;
+  const float qxx = yx * yx, qxy = yx2 * yy, qxz = yx2 * yz, qyy = yy * yy, qyz = yy2 * yz, qzz = yz * yz;
+  const float Qx = fma(Q[0], yx, fma(Q[1], yy, Q[2] * yz));
+  const float Qy = fma(Q[1], yx, fma(Q[3], yy, Q[4] * yz));
+  const float Qz = fma(Q[2], yx, fma(Q[4], yy, Q[5] * yz));
+  const auto dot6 = [&](float a, float b, float c, float d, float e, float f, float to) {
+    return fma(qxx, a, fma(qxy, b, fma(qxz, c, fma(qyy, d, fma(qyz, e, fma(qzz, f, to))))));
   };
-  const float M3x = dot6(m3[0], m3[1], m3[2], m3[3], m3[4], m3[5]);
-  const float M3y = dot6(m3[1], m3[3], m3[4], m3[6], m3[7], m3[8]);
-  const float M3z = dot6(m3[2], m3[4], m3[5], m3[7], m3[8], m3[9]);
-  const float T3 = __builtin_fmaf(M3x, yx, __builtin_fmaf(M3y, yy, M3z * yz));
+  const float V3x = dot6(m3[0], m3[1], m3[2], m3[3], m3[4], m3[5], Qx);
+  const float V3y = dot6(m3[1], m3[3], m3[4], m3[6], m3[7], m3[8], Qy);
+  const float V3z = dot6(m3[2], m3[4], m3[5], m3[7], m3[8], m3[9], Qz);
+  const float B3 = (1.f / 3.f) * fma(fma(0.5f, Qx, V3x), yx, fma(fma(0.5f, Qy, V3y), yy, fma(0.5f, Qz, V3z) * yz));
   // cubic monomials with their multinomial weights: (M4 . y y y)_k
-  const float cxxx = qxx * yx, cxxy = 3.f * qxx * yy, cxxz = 3.f * qxx * yz, cxyy = 3.f * yx * qyy,
-              cxyz = 3.f * qxy * yz, cxzz = 3.f * yx * qzz, cyyy = qyy * yy, cyyz = 3.f * qyy * yz,
-              cyzz = 3.f * yy * qzz, czzz = qzz * yz;
-  auto dot10 = [&](int a, int b, int c, int d, int e, int f, int g, int h, int k, int l) {
-    return __builtin_fmaf(cxxx, m4[a], __builtin_fmaf(cxxy, m4[b], __builtin_fmaf(cxxz, m4[c],
-           __builtin_fmaf(cxyy, m4[d], __builtin_fmaf(cxyz, m4[e], __builtin_fmaf(cxzz, m4[f],
-           __builtin_fmaf(cyyy, m4[g], __builtin_fmaf(cyyz, m4[h], __builtin_fmaf(cyzz, m4[k], czzz * m4[l])))))))));
+  const float qxx3 = 3.f * qxx, qyy3 = 3.f * qyy, qzz3 = 3.f * qzz;
+  const float cxxx = qxx * yx, cxxy = qxx3 * yy, cxxz = qxx3 * yz, cxyy = qyy3 * yx, cxyz = 3.f * qxy * yz,
+              cxzz = qzz3 * yx, cyyy = qyy * yy, cyyz = qyy3 * yz, cyzz = qzz3 * yy, czzz = qzz * yz;
+  const auto dot10 = [&](int a, int b, int c, int d, int e, int f, int g, int k, int l, int m) {
+    return fma(cxxx, m4[a], fma(cxxy, m4[b], fma(cxxz, m4[c], fma(cxyy, m4[d], fma(cxyz, m4[e],
+           fma(cxzz, m4[f], fma(cyyy, m4[g], fma(cyyz, m4[k], fma(cyzz, m4[l], czzz * m4[m])))))))));
   };
-  const float M4x = dot10(0, 1, 2, 3, 4, 5, 6, 7, 8, 9);
-  const float M4y = dot10(1, 3, 4, 6, 7, 8, 10, 11, 12, 13);
-  const float M4z = dot10(2, 4, 5, 7, 8, 9, 11, 12, 13, 14);
-  const float T4 = __builtin_fmaf(M4x, yx, __builtin_fmaf(M4y, yy, M4z * yz));
-  const float S = M0 * g0 + 0.5f * (g2 * yM2y + g1 * trM2) - (g3 * T3 + 3.f * g2 * t3y) * (1.f / 6.f) +
-                  (g4 * T4 + 6.f * g3 * yQy + 3.f * g2 * trQ) * (1.f / 24.f);
-  const float A = M0 * g1 + 0.5f * (g3 * yM2y + g2 * trM2) - (g4 * T3 + 3.f * g3 * t3y) * (1.f / 6.f) +
-                  (g5 * T4 + 6.f * g4 * yQy + 3.f * g3 * trQ) * (1.f / 24.f);
-  const float b2 = g2, b3 = -0.5f * g3, bt = -0.5f * g2, b4 = g4 * (1.f / 6.f), bq = 0.5f * g3;
-  gx = A * yx + b2 * M2x + b3 * M3x + bt * t3[0] + b4 * M4x + bq * Qx;
-  gy = A * yy + b2 * M2y + b3 * M3y + bt * t3[1] + b4 * M4y + bq * Qy;
-  gz = A * yz + b2 * M2z + b3 * M3z + bt * t3[2] + b4 * M4z + bq * Qz;
-  pot = -S;
+  const float V4x = dot10(0, 1, 2, 3, 4, 5, 6, 7, 8, 9);
+  const float V4y = dot10(1, 3, 4, 6, 7, 8, 10, 11, 12, 13);
+  const float V4z = dot10(2, 4, 5, 7, 8, 9, 11, 12, 13, 14);
+  const float B4 = 0.25f * fma(V4x, yx, fma(V4y, yy, V4z * yz));
+  const float A = fma(M[4], G1, fma(3.f * M[5], G2, fma(5.f * B2, G3, fma(7.f * B3, G4, 9.f * B4 * G5))));
+  pot = -fma(M[4], G0, fma(M[5], G1, fma(B2, G2, fma(B3, G3, B4 * G4))));
+  gx = fma(A, yx, fma(G2, V2x, fma(G3, V3x, G4 * V4x)));
+  gy = fma(A, yy, fma(G2, V2y, fma(G3, V3y, G4 * V4y)));
+  gz = fma(A, yz, fma(G2, V2z, fma(G3, V3z, G4 * V4z)));
 }
 
 // mixed form, Plummer: split positions, FMA pair arithmetic, blocked
