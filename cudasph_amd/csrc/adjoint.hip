@@ -1019,7 +1019,8 @@ void Engine<T>::adj_forces_backward(bool seed_rho) {
     }
     if (pairs) {
       hipLaunchKernelGGL(k_adj_gravity_pairs_sum, dim3(ceil_div(n_, kBlock), 3), dim3(kBlock), 0, s_, ws,
-                         ws + pairs64_own(n_, parts), (double*)xs_.p, n_, pairs64_tiles(n_), parts);
+                         ws + pairs64_own(n_, parts), (double*)xs_.p, n_, pairs64_tiles(n_),
+                         pairs64_parts(n_, parts));
       CS_CHECK_LAUNCH();
     } else if (parts > 1) {
       hipLaunchKernelGGL(k_adj_gravity_combine, grid(n_), dim3(kBlock), 0, s_, (const D4v*)gpart64_.p, xs_.p, n_,

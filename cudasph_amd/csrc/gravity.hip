@@ -1737,17 +1737,16 @@ static int gpu_cus() {
 // Parts for the passes of the FP64 form: of 2 .. 8 (1 from 2^19 particles on)
 // the count whose blocks fill the CUs most evenly, the larger of equals.
 // Every block is resident at once and takes the same time, so a pass lasts as
-// long as its fullest CU.  Pairs taken once, gravity alone, 8 / 7 / 6 / 5 / 4 / 2
-// parts, ms: 50 021 particles (196 tiles on 256 CUs) 1.54 / 1.47 / 1.41 / 1.37 /
-// 1.65 / 1.80, 65 536: 2.22 / 2.20 / 2.17 / 2.20 / 2.23 / 2.41, 100 003: 5.55 / 5.35 /
-// 5.69 / 5.52 / 6.15 / 7.31.  Two or three times the parts are as fast alone and
-// leave the SPH passes less room: steps of 65 536 2.75 / 2.92 / 3.01.
+// long as its fullest CU.  Pairs taken once, gravity alone, 8 / 5 parts, ms:
+// 50 021 particles (98 tiles on 256 CUs) 1.59 / 1.34, 65 536 (128): 2.06 / 2.36,
+// 100 003 (196): 5.42 / 5.09, 131 072 (256): 7.9 / 8.2.
 int gravity64_parts(int n_i) {
-  const int blocks = ceil_div(n_i, kGravBlock);
+  const bool pairs = pairs64_fits(n_i);
+  const int blocks = pairs ? pairs64_tiles(n_i) : ceil_div(n_i, kGravBlock);
   if (blocks >= 2048) return 1;
   const int cus = gpu_cus();
   int best = 8;
-  for (int p = 7; p >= 2 && (long)p * blocks >= 4l * cus; --p)   // fewer: too few wavefronts per SIMD
+  for (int p = 7; p >= 2 && (pairs || (long)p * blocks >= 4l * cus); --p)   // fewer: too few wavefronts per SIMD
     // fullest CU's blocks per unit of work: ceil(p blocks / cus) / p
     if ((long)ceil_div((long)p * blocks, cus) * best < (long)ceil_div((long)best * blocks, cus) * p) best = p;
   return best;
@@ -1806,7 +1805,7 @@ void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_
     double* ws = (double*)part;
     launch_pairs64(GravityPairs{gpos, eps * eps}, n_i, parts, ws, s);
     hipLaunchKernelGGL(k_gravity64_pairs_sum, dim3(ceil_div(n_i, kBlock), 4), dim3(kBlock), 0, s, ws,
-                       ws + pairs64_own(n_i, parts), (double*)out, n_i, pairs64_tiles(n_i), parts);
+                       ws + pairs64_own(n_i, parts), (double*)out, n_i, pairs64_tiles(n_i), pairs64_parts(n_i, parts));
     CS_CHECK_LAUNCH();
     return;
   }

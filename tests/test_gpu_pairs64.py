@@ -9,8 +9,9 @@ import adjoint_reference as ar
 pytestmark = pytest.mark.gpu
 
 
-# 8 192 is the first size; 33, 34, 37 and 257 tiles
-@pytest.mark.parametrize("n", [8191, 8192, 8193, 8449, 8704, 9217, 65537])
+# 8 192 is the first size, 12 287 the last with more parts; 16, 17, 18, 19, 24, 25
+# and 129 tiles
+@pytest.mark.parametrize("n", [8191, 8192, 8193, 8449, 8704, 9217, 12287, 12289, 65537])
 def test_pairs_give_the_direct_sum(cs, n):
     print(f"fp64 pairs n={n}", flush=True)
     p = cs.preset_params(2, n)
@@ -40,7 +41,7 @@ def test_pairs_give_the_direct_sum(cs, n):
 
 
 def test_reverse_pass_against_the_cpu_reference(cs):
-    """One step at 33 tiles, as test_adjoint_matches_fp64_cpu_reference_gradient
+    """One step at 17 tiles, as test_adjoint_matches_fp64_cpu_reference_gradient
     (same tolerance)."""
     n, K = 8193, 1
     print(f"adjoint pairs n={n}", flush=True)
