@@ -179,7 +179,7 @@ float host_sph_accelerations(int n_bodies, int /*ngb_tot*/, float av_alpha, floa
   guarded([&] {
     CS_HIP(hipMemset(a.flags, 0, 16));
     launch_find_ngb<float>(a.pos, a.tree, (KV*)bodies_hash, ngb_offset, a.n_ngb, a.n_ngb, ngb_list, a.flags,
-                           n_bodies, walk(a, a.n_nodes, a.p.rel_err), 1, nullptr);
+                           n_bodies, walk(a, a.n_nodes, a.p.rel_err), 1, -1, nullptr);
     int fl = 0;
     CS_HIP(hipMemcpy(&fl, a.flags, 4, hipMemcpyDeviceToHost));
     if (fl)

@@ -97,7 +97,9 @@ class Engine final : public EngineBase {
   void tree_build();
   void sph_after_tree();
   void solve();
-  void offsets();
+  void offsets(bool check);
+  long accept_total(int tot);
+  void collect_dt();
   long check_total();
   void find();
   void density();

@@ -34,9 +34,11 @@ struct EosConst;  // sph_math.h
 template <class T>
 void launch_solve_range(V4<T>* pos, int* n_ngb, const KV* hash, const V4<T>* tree, int n_dev,
                         const WalkParams& wp, hipStream_t s);
+// list_cap >= 0: the slots of list; the total offset[n_dev] goes to flags[3],
+// and nothing is written if it exceeds them (or is negative)
 template <class T>
 void launch_find_ngb(const V4<T>* pos, const V4<T>* tree, KV* hash, const int* offset, const int* cap_count,
-                     int* count_out, int* list, int* flags, int n_dev, const WalkParams& wp, int clamp,
+                     int* count_out, int* list, int* flags, int n_dev, const WalkParams& wp, int clamp, int list_cap,
                      hipStream_t s);
 // ---- sph_passes.hip ----
 // plain and FP64 forms

@@ -559,6 +559,18 @@ __global__ __launch_bounds__(kBlock) void k_solve_range(V4<T>* __restrict__ pos,
   }
 }
 
+// Whether the lists' total, offset[n_dev], exceeds their allocation of list_cap
+// slots (list_cap < 0: not asked, offset then has no such entry).  The launch
+// reports the total in flags[3] and then writes nothing, so the walk can be
+// queued before the host has seen the total.
+__device__ __forceinline__ bool list_overflow(const int* __restrict__ offset, int n_dev, int list_cap,
+                                              int* __restrict__ flags) {
+  if (list_cap < 0) return false;
+  const int total = offset[n_dev];
+  if (blockIdx.x == 0 && threadIdx.x == 0) flags[3] = total;
+  return total < 0 || total > list_cap;
+}
+
 // dev_find_ngb.cu:75-87.  Capacity of particle i's slot is
 // n_norm(cap_count[i], 4) (the layout of sph_accelerations.cpp:58-64); at most
 // that many ids are written, the true count goes to count_out[i], and
@@ -571,8 +583,9 @@ __global__ __launch_bounds__(kBlock) void k_find_ngb(const V4<T>* __restrict__ p
                                                       KV* __restrict__ hash, const int* __restrict__ offset,
                                                       const int* cap_count, int* count_out,
                                                       int* __restrict__ list, int* __restrict__ flags,
-                                                      int n_dev, WalkParams wp, int clamp) {
+                                                      int n_dev, WalkParams wp, int clamp, int list_cap) {
   chain_priority();
+  if (list_overflow(offset, n_dev, list_cap, flags)) return;
   extern __shared__ __align__(16) char s_mem[];   // WalkLds<int, false> per group
   WalkLds<int, false>& s = reinterpret_cast<WalkLds<int, false>*>(s_mem)[threadIdx.x / kWalkGroup];
   const int t = (xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + (int)threadIdx.x) / kWalkGroup;
@@ -667,8 +680,9 @@ __global__ __launch_bounds__(kBlock) void k_find_ngb_lane(const V4<T>* __restric
                                                            const int* __restrict__ offset, const int* cap_count,
                                                            int* count_out, int* __restrict__ list,
                                                            int* __restrict__ flags, int n_dev, WalkParams wp,
-                                                           int clamp) {
+                                                           int clamp, int list_cap) {
   chain_priority();
+  if (list_overflow(offset, n_dev, list_cap, flags)) return;
   extern __shared__ int s_stack[];   // walk_stack_depth(n_nodes) entries per lane
   const int t = xcd_block(blockIdx.x, gridDim.x) * (int)blockDim.x + threadIdx.x;
   if (t >= n_dev) return;
@@ -744,17 +758,17 @@ void launch_solve_range(V4<T>* pos, int* n_ngb, const KV* hash, const V4<T>* tre
 
 template <class T>
 void launch_find_ngb(const V4<T>* pos, const V4<T>* tree, KV* hash, const int* offset, const int* cap_count,
-                     int* count_out, int* list, int* flags, int n_dev, const WalkParams& wp, int clamp,
+                     int* count_out, int* list, int* flags, int n_dev, const WalkParams& wp, int clamp, int list_cap,
                      hipStream_t s) {
   const int bs = walk_block(n_dev);
   if (walk_alone(n_dev)) {
     const size_t lds = (size_t)walk_stack_depth(wp.n_nodes) * bs * sizeof(int);
     hipLaunchKernelGGL(k_find_ngb_lane<T>, dim3(ceil_div(n_dev, bs)), dim3(bs), lds, s, pos, tree, hash, offset,
-                       cap_count, count_out, list, flags, n_dev, wp, clamp);
+                       cap_count, count_out, list, flags, n_dev, wp, clamp, list_cap);
   } else {
     const int per = bs / kWalkGroup;
     hipLaunchKernelGGL(k_find_ngb<T>, dim3(ceil_div(n_dev, per)), dim3(bs), per * sizeof(WalkLds<int, false>), s, pos,
-                       tree, hash, offset, cap_count, count_out, list, flags, n_dev, wp, clamp);
+                       tree, hash, offset, cap_count, count_out, list, flags, n_dev, wp, clamp, list_cap);
   }
   CS_CHECK_LAUNCH();
 }
@@ -763,7 +777,7 @@ void launch_find_ngb(const V4<T>* pos, const V4<T>* tree, KV* hash, const int* o
   template void launch_solve_range<T>(V4<T>*, int*, const KV*, const V4<T>*, int, const WalkParams&,      \
                                       hipStream_t);                                                       \
   template void launch_find_ngb<T>(const V4<T>*, const V4<T>*, KV*, const int*, const int*, int*, int*,   \
-                                   int*, int, const WalkParams&, int, hipStream_t);
+                                   int*, int, const WalkParams&, int, int, hipStream_t);
 CS_INST(float)
 CS_INST(double)
 #undef CS_INST

@@ -100,3 +100,22 @@ def test_both_walks_give_the_tree_s_lists(cs, n):
         want = np.nonzero(d2 < q[i, 3] * q[i, 3])[0]
         assert np.array_equal(np.sort(lst[off[i]:off[i] + cnt[i]]), want), i
     e.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "mixed", "fp64"])
+def test_whole_evaluation_refuses_lists_beyond_the_allocation(cs, form):
+    """A neighbour target of 100 needs more than the 100 slots per particle:
+    init() refuses, as the offsets pass by itself, and no list was written."""
+    n = 2000
+    print(f"refusal {form}", flush=True)
+    p = cs.preset_params(2, n)
+    p.desired_ngb = 100.0
+    e = cs.Engine(form, p)
+    e.load_ic(*cs.generate_ic(2, n, 5))
+    e.set("ngb_list", np.full_like(e.get("ngb_list"), 7))   # (allocated, not cleared)
+    with pytest.raises(RuntimeError, match="overflow"):
+        e.init()
+    assert (e.get("ngb_list") == 7).all() and not e.get("ngb_count").any()
+    with pytest.raises(RuntimeError, match="overflow"):
+        e.run_pass(cs.OFFSETS)
+    e.close()
