@@ -13,6 +13,41 @@ namespace cudasph {
 // issue as soon as their data is back and gravity fills the remaining cycles.
 __device__ __forceinline__ void chain_priority() { __builtin_amdgcn_s_setprio(3); }
 
+// orders this wavefront's LDS writes before its later LDS reads (the LDS
+// serves one wavefront's accesses in order; this holds the compiler to it)
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sums of NC terms over a list by a group of 16 lanes, in list order (so with
+// the bits of one lane's running sums): each lane computes the terms of one
+// entry, the group hands them over through its LDS row, and lane c adds component
+// c % NC of the 16 one after another.  Lanes past the end of the list hand over
+// none(), which changes no sum.
+template <class T, int NC>
+struct OrderedSums {
+  static constexpr int kRow = NC * 16 + 16;   // LDS of a group (16 more, so that the groups' banks differ)
+  T s;
+  T* row;
+  int l;
+  static __device__ __forceinline__ T none() { return T(-0.0); }
+  __device__ __forceinline__ void add(const T (&t)[NC]) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) row[c * 16 + l] = t[c];
+    lds_order();
+    const T* r = row + (l % NC) * 16;
+    T v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = r[k];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s += v[k];
+    lds_order();
+  }
+  __device__ __forceinline__ T get(int c) const { return __shfl(s, c, 16); }
+};
+
 struct WalkParams {
   int n_nodes;        // real particles (the reference passes n_bodies, CUDA_calls.cpp:5)
   int fix_phantom;

@@ -6,7 +6,7 @@
 // kd-tree heap order, or with memory order when the particles are already in
 // Peano-Hilbert order; either way a wavefront holds spatially adjacent
 // particles and their neighbour gathers hit the same cache lines.  Plain and
-// FP64 forms: one lane per particle, its sums in list order, so in the plain
+// FP64 forms: 16 lanes per particle, its sums in list order, so in the plain
 // form each particle's result is the same bit pattern as the CPU
 // restatement's.  The mixed form has its own density and hydro kernels (FP32
 // pair arithmetic, compensated sums).
@@ -49,17 +49,12 @@ __device__ __forceinline__ float group_max(float v) {
   for (int o = kGroup / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kGroup));
   return v;
 }
-// plain running sum in list order (the reference's accumulation)
-template <class T>
-struct Sum {
-  T s = T(0);
-  __device__ __forceinline__ void add(T x) { s += x; }
-  __device__ __forceinline__ void sub(T x) { s -= x; }
-  __device__ __forceinline__ T get() const { return s; }
-};
-
 // density, grad-h terms, div v and |curl v| (dev_density_loop.cu:29-111);
-// plain and FP64 forms
+// plain and FP64 forms.  A group of 16 lanes per particle, its sums in list
+// order (OrderedSums).  One lane per particle waited for one neighbour's records
+// after another.  Density / hydro, one lane -> this, us: plain 1 000 particles 110 ->
+// 13 / 141 -> 16, 16 384: 80 -> 16 / 97 -> 20, 131 072: 90 -> 63 / 241 -> 97, 600 000:
+// 649 -> 280 / 1278 -> 443; FP64 65 536: 76 -> 48 / 116 -> 68.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_density(const V4<T>* __restrict__ pos, const V4<T>* __restrict__ vel,
                                                      V4<T>* __restrict__ hydro,
@@ -67,49 +62,50 @@ __global__ __launch_bounds__(kBlock) void k_density(const V4<T>* __restrict__ po
                                                      const int* __restrict__ offset, const int* __restrict__ count,
                                                      const int* __restrict__ list, int n_dev) {
   chain_priority();
-  const int t = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  if (t >= n_dev) return;
+  using Sums = OrderedSums<T, 8>;   // rho, omega, psi, -den, div v, curl v
+  __shared__ __align__(16) T s_rows[kBlock / 16][Sums::kRow];
+  const int t = (xcd_block(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) / 16, l = threadIdx.x % 16;
+  if (t >= n_dev) return;   // whole groups leave together
   const int i = (int)hash[t].value;
   const V4<T> bp = pos[i], bv = vel[i];
-  Sum<T> rho, om, psi, den, divv, cx, cy, cz;
+  Sums sums{T(0), s_rows[threadIdx.x / 16], l};
   const int off = offset[i], n = count[i];
-  // software pipeline: the next neighbour's id and records are requested
-  // before the current pair is computed (the sums keep list order)
-  int jn = n > 0 ? list[off] : i;
-  V4<T> pn = pos[jn], vn = vel[jn];
-  for (int k = off; k < off + n; ++k) {
-    const V4<T> pj = pn, vj = vn;
-    if (k + 1 < off + n) {
-      jn = list[k + 1];
-      pn = pos[jn];
-      vn = vel[jn];
+  for (int k = l; k - l < n; k += 16) {
+    T a[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) a[c] = Sums::none();
+    if (k < n) {
+      const int j = list[off + k];
+      const V4<T> pj = pos[j], vj = vel[j];
+      const T dx = bp.x - pj.x, dy = bp.y - pj.y, dz = bp.z - pj.z;
+      const T u = T(2) * dsqrt(dx * dx + dy * dy + dz * dz) / bp.w;
+      a[0] = vj.w * kern_w<T>(u);
+      a[1] = vj.w * kern_dwdh<T>(u);
+      a[2] = vj.w * kern_dphidh<T>(u);
+      a[3] = -kern_digdh<T>(u);
+      const T dvx = bv.x - vj.x, dvy = bv.y - vj.y, dvz = bv.z - vj.z;
+      const T mdw = bv.w * kern_dw<T>(u);
+      a[4] = mdw * (dx * dvx + dy * dvy + dz * dvz);
+      a[5] = mdw * (dy * dvz - dz * dvy);
+      a[6] = mdw * (dz * dvx - dx * dvz);
+      a[7] = mdw * (dx * dvy - dy * dvx);
     }
-    const T dx = bp.x - pj.x, dy = bp.y - pj.y, dz = bp.z - pj.z;
-    const T u = T(2) * dsqrt(dx * dx + dy * dy + dz * dz) / bp.w;
-    rho.add(vj.w * kern_w<T>(u));
-    om.add(vj.w * kern_dwdh<T>(u));
-    psi.add(vj.w * kern_dphidh<T>(u));
-    den.sub(kern_digdh<T>(u));
-    const T dvx = bv.x - vj.x, dvy = bv.y - vj.y, dvz = bv.z - vj.z;
-    const T mdw = bv.w * kern_dw<T>(u);
-    divv.add(mdw * (dx * dvx + dy * dvy + dz * dvz));
-    cx.add(mdw * (dy * dvz - dz * dvy));
-    cy.add(mdw * (dz * dvx - dx * dvz));
-    cz.add(mdw * (dx * dvy - dy * dvx));
+    sums.add(a);
   }
+  const T rho = sums.get(0), om = sums.get(1), psi = sums.get(2), d = sums.get(3), divv = sums.get(4),
+          x = sums.get(5), y = sums.get(6), z = sums.get(7);
+  if (l != 0) return;
   const T h = T(0.5 * (double)bp.w);
   const T h3 = h * h * h, h5 = h * h * h * h * h;
-  T o = om.get(), p = psi.get();
-  const T d = den.get();
+  T o, p;
   if (d != T(0)) {
-    o = T((double)o * (1.0 / (double)h3 / (double)d));
-    p = T((double)p * (1.0 / (double)h / (double)d));
+    o = T((double)om * (1.0 / (double)h3 / (double)d));
+    p = T((double)psi * (1.0 / (double)h / (double)d));
   } else {
     o = p = T(0);
   }
-  const T r = T((double)rho.get() * (1.0 / (double)h3));
-  const T dv = T((double)divv.get() * (1.0 / (double)r / (double)h5));
-  const T x = cx.get(), y = cy.get(), z = cz.get();
+  const T r = T((double)rho * (1.0 / (double)h3));
+  const T dv = T((double)divv * (1.0 / (double)r / (double)h5));
   const T curl = dsqrt(x * x + y * y + z * z) / r / h5;
   hydro[i].x = r;
   dots[i] = {dv, curl, o, p};
@@ -152,7 +148,7 @@ __global__ __launch_bounds__(kBlock) void k_eos_mixed(F4* __restrict__ hydro, co
 
 // hydro accelerations, du/dt and max signal speed (dev_hydro_dots.cu:25-113);
 // writes the per-pair reaction coefficient m_i*acc to ngb_acc[k]; plain and
-// FP64 forms
+// FP64 forms, 16 lanes per particle as k_density
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_hydro(const V4<T>* __restrict__ pos, const V4<T>* __restrict__ vel,
                                                    const V4<T>* __restrict__ hydro,
@@ -162,8 +158,10 @@ __global__ __launch_bounds__(kBlock) void k_hydro(const V4<T>* __restrict__ pos,
                                                    const int* __restrict__ count, const int* __restrict__ list,
                                                    int n_dev, T alpha, T beta) {
   chain_priority();
-  const int t = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  if (t >= n_dev) return;
+  using Sums = OrderedSums<T, 4>;   // acceleration, du/dt
+  __shared__ __align__(16) T s_rows[kBlock / 16][Sums::kRow];
+  const int t = (xcd_block(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) / 16, l = threadIdx.x % 16;
+  if (t >= n_dev) return;   // whole groups leave together
   const int i = (int)hash[t].value;
   const V4<T> bp = pos[i], bv = vel[i], hd = hydro[i], dd = dots[i];
   const T prho2 = hd.y / (hd.x * hd.x);
@@ -171,42 +169,40 @@ __global__ __launch_bounds__(kBlock) void k_hydro(const V4<T>* __restrict__ pos,
   // POW5(0.5*range) and POW2(0.5*range) expand left to right in the reference
   const double pow5 = hw * 0.5 * (double)bp.w * 0.5 * (double)bp.w * 0.5 * (double)bp.w * 0.5 * (double)bp.w;
   const double pow2 = hw * 0.5 * (double)bp.w;
-  Sum<T> ax, ay, az, ud;
+  Sums sums{T(0), s_rows[threadIdx.x / 16], l};
   T vsig = T(0);
   const int off = offset[i], n = count[i];
-  // software pipeline, as in k_density
-  int jn = n > 0 ? list[off] : i;
-  V4<T> pn = pos[jn], vn = vel[jn], hn = hydro[jn], dn = dots[jn];
-  for (int k = off; k < off + n; ++k) {
-    const V4<T> pj = pn, vj = vn, hj = hn, dj = dn;
-    if (k + 1 < off + n) {
-      jn = list[k + 1];
-      pn = pos[jn];
-      vn = vel[jn];
-      hn = hydro[jn];
-      dn = dots[jn];
+  for (int k = l; k - l < n; k += 16) {
+    T a[4] = {Sums::none(), Sums::none(), Sums::none(), Sums::none()};
+    if (k < n) {
+      const int j = list[off + k];
+      const V4<T> pj = pos[j], vj = vel[j], hj = hydro[j], dj = dots[j];
+      const T dx = bp.x - pj.x, dy = bp.y - pj.y, dz = bp.z - pj.z;
+      const T dvx = bv.x - vj.x, dvy = bv.y - vj.y, dvz = bv.z - vj.z;
+      const T ds = dsqrt(dx * dx + dy * dy + dz * dz);
+      const T u = T((double)ds / hw);
+      const T drdv = dx * dvx + dy * dvy + dz * dvz;
+      const Visc<T> av = art_visc<T>(bp.w, pj.w, ds, drdv, hd, dd, hj, dj, alpha, beta);
+      vsig = dmax(vsig, av.vsig);
+      const double w1 = (double)kern_dw<T>(u);
+      const T g = kern_dig<T>(u);
+      const double pv = (double)prho2 + 0.5 * (double)av.pi;
+      T acc = T(pv * w1 / pow5);
+      acc = T((double)acc - ((double)(prho2 * dd.z) + 0.5 * (double)dd.w) / (double)vj.w * (double)g / pow2);
+      a[0] = -(vj.w * acc * dx);
+      a[1] = -(vj.w * acc * dy);
+      a[2] = -(vj.w * acc * dz);
+      ngb_acc[off + k] = bv.w * acc;
+      T udot = T((double)vj.w * pv * w1 / pow5);
+      udot = T((double)udot - (double)(prho2 * dd.z * g) / pow2);
+      a[3] = udot * drdv;
     }
-    const T dx = bp.x - pj.x, dy = bp.y - pj.y, dz = bp.z - pj.z;
-    const T dvx = bv.x - vj.x, dvy = bv.y - vj.y, dvz = bv.z - vj.z;
-    const T ds = dsqrt(dx * dx + dy * dy + dz * dz);
-    const T u = T((double)ds / hw);
-    const T drdv = dx * dvx + dy * dvy + dz * dvz;
-    const Visc<T> av = art_visc<T>(bp.w, pj.w, ds, drdv, hd, dd, hj, dj, alpha, beta);
-    vsig = dmax(vsig, av.vsig);
-    const double w1 = (double)kern_dw<T>(u);
-    const T g = kern_dig<T>(u);
-    const double pv = (double)prho2 + 0.5 * (double)av.pi;
-    T acc = T(pv * w1 / pow5);
-    acc = T((double)acc - ((double)(prho2 * dd.z) + 0.5 * (double)dd.w) / (double)vj.w * (double)g / pow2);
-    ax.sub(vj.w * acc * dx);
-    ay.sub(vj.w * acc * dy);
-    az.sub(vj.w * acc * dz);
-    ngb_acc[k] = bv.w * acc;
-    T udot = T((double)vj.w * pv * w1 / pow5);
-    udot = T((double)udot - (double)(prho2 * dd.z * g) / pow2);
-    ud.add(udot * drdv);
+    sums.add(a);
   }
-  bdots[i] = {ax.get(), ay.get(), az.get(), ud.get()};
+  for (int o = 8; o > 0; o >>= 1) vsig = dmax(vsig, __shfl_xor(vsig, o, 16));
+  const V4<T> b{sums.get(0), sums.get(1), sums.get(2), sums.get(3)};
+  if (l != 0) return;
+  bdots[i] = b;
   hydro2[i].x = vsig;
 }
 
@@ -351,7 +347,7 @@ __global__ __launch_bounds__(kBlock) void k_hydro_mixed(const F4* __restrict__ p
 template <class T>
 void launch_density(const V4<T>* pos, const V4<T>* vel, V4<T>* hydro, V4<T>* dots, const KV* hash,
                     const int* offset, const int* count, const int* list, int n_dev, hipStream_t s) {
-  hipLaunchKernelGGL(k_density<T>, dim3(ceil_div(n_dev, kBlock)), dim3(kBlock), 0, s, pos, vel, hydro, dots, hash,
+  hipLaunchKernelGGL(k_density<T>, dim3(ceil_div(n_dev, kBlock / 16)), dim3(kBlock), 0, s, pos, vel, hydro, dots, hash,
                      offset, count, list, n_dev);
   CS_CHECK_LAUNCH();
 }
@@ -387,7 +383,7 @@ template <class T>
 void launch_hydro(const V4<T>* pos, const V4<T>* vel, const V4<T>* hydro, const V4<T>* dots, V4<T>* bdots,
                   V4<T>* hydro2, T* ngb_acc, const KV* hash, const int* offset, const int* count, const int* list,
                   int n_dev, T alpha, T beta, hipStream_t s) {
-  hipLaunchKernelGGL(k_hydro<T>, dim3(ceil_div(n_dev, kBlock)), dim3(kBlock), 0, s, pos, vel, hydro, dots, bdots,
+  hipLaunchKernelGGL(k_hydro<T>, dim3(ceil_div(n_dev, kBlock / 16)), dim3(kBlock), 0, s, pos, vel, hydro, dots, bdots,
                      hydro2, ngb_acc, hash, offset, count, list, n_dev, alpha, beta);
   CS_CHECK_LAUNCH();
 }

@@ -68,14 +68,6 @@ struct Lane {
   __device__ __forceinline__ int before(unsigned mask) const { return __popc(mask & ((1u << l) - 1u)); }
 };
 
-// orders this wavefront's LDS writes before its later LDS reads (the LDS
-// serves one wavefront's accesses in order; this holds the compiler to it)
-__device__ __forceinline__ void lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // lane S of the row, in every lane of the row
 template <int S>
 __device__ __forceinline__ int row_bcast(int v) {
