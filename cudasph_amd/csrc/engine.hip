@@ -467,10 +467,10 @@ void Engine<T>::collect_dt() {
   std::memcpy(&dt_, &h_small_[0], 8);
 }
 
-// the subtree boxes of the current tree, when the walks use them
+// the subtree boxes of the current tree
 template <class T>
 void Engine<T>::ensure_boxes() {
-  if (!walk_boxes_ || !boxes_stale_) return;
+  if (!boxes_stale_) return;
   TimerScope ts(timers_, "tree_boxes", s_);
   launch_tree_boxes<T>(tree_, boxes_, p_.n_bodies, p_.fix_phantom, s_);
   boxes_stale_ = false;
@@ -487,10 +487,18 @@ void Engine<T>::solve() {
     CS_HIP(hipMemcpyAsync(n_ngb_, adj_nngb_.p + rec, (size_t)nd_ * 4, hipMemcpyDeviceToDevice, s_));
     return;
   }
-  ensure_boxes();
+  // With the boxes in every form from kSolveBoxesMinN on: the h-solve leaves no
+  // walk lengths, and the neighbours it sums over and their order are the
+  // reference's either way.  Plain steps without / with them, ms: Plummer
+  // spheres of 4 096 particles 0.705 / 0.518, 16 384: 0.714 / 0.611, 100 003: 12.06 /
+  // 11.98; uniform cubes of 16 384: 0.722 / 0.722, of 1 000 (two launches more)
+  // 0.258 / 0.270.
+  const bool boxes = walk_boxes_ || n_ >= kSolveBoxesMinN;
+  if (boxes) ensure_boxes();
   {
     TimerScope ts(timers_, "solve_range", s_);
     WalkParams wp = walk_params();
+    if (boxes) wp.boxes = boxes_.p;
     wp.solve_cache = solve_cache_ != 0;
     launch_solve_range<T>(pos_, n_ngb_, hash_, tree_, nd_, wp, s_);
   }
@@ -539,7 +547,7 @@ long Engine<T>::accept_total(int tot) {
 // 0.385 -> 0.358 ms, 16 384: 0.469 -> 0.440; plain 16 384: 0.907 -> 0.890).
 template <class T>
 void Engine<T>::find() {
-  ensure_boxes();
+  if (walk_boxes_) ensure_boxes();
   const WalkParams wp = walk_params();
   for (int attempt = 0; attempt < 2; ++attempt) {
     {
@@ -861,12 +869,10 @@ void Engine<T>::step() {
   // (sph_accelerations, then CUDA_gravity, step.cpp:65,94).  The spline
   // softening needs the new ranges and keeps that order.
   const bool grav_first = p_.grav_mode == 1;
-  // overlap < 0 (the default) is on: the mixed form's SPH passes take ~12 ms
-  // at N = 2^20 and slow its gravity by ~4 ms when they run beside it
-  // (288.5 -> 282.9 ms/step; with the far field 106.2 -> 101.6); FP64 827 ->
-  // 814 ms/step at 2^20, 58.2 -> 53.4 at 262 144; plain, with its checked
-  // device tree build, 3.63 -> 2.22 ms/step at 16 384, 12.8 -> 8.5 at 65 536,
-  // 81.5 -> 71.3 at 262 144, 1056 -> 1036 at 2^20
+  // overlap < 0 (the default) is on.  In order / beside, ms per step: mixed
+  // 16 384 particles 0.64 / 0.44, 65 536: 2.01 / 1.67, 2^20: 236.9 / 234.1 (far field
+  // 80.1 / 78.3); FP64 65 536: 2.95 / 2.46, 262 144: 32.8 / 31.1; plain 16 384: 1.23 /
+  // 0.70, 65 536: 5.39 / 4.53, 262 144: 63.2 / 61.3
   const bool overlap = overlap_ != 0;
   // on its own stream, gravity starts before the device tree build, which
   // then runs beside it (the build is on the SPH passes' path, not gravity's)

@@ -67,6 +67,7 @@ class Engine final : public EngineBase {
  private:
   static constexpr bool kF32 = sizeof(T) == 4;
   bool mixed() const { return form_ == SPH_FORM_MIXED; }
+  static constexpr int kSolveBoxesMinN = 4096;
   void ensure_boxes();
   WalkParams walk_params() const {
     return {p_.n_bodies, p_.fix_phantom, p_.rel_err, p_.desired_ngb, p_.max_iter,
@@ -227,7 +228,7 @@ class Engine final : public EngineBase {
   int tree_gpu_ = 0;            // 0 host build, 1 device build, 2 device build checked for ties (host on a tie)
   long tree_fallbacks_ = 0;     // steps whose verified device build fell back to the host build
   DBuf<int> ties_;
-  int walk_boxes_ = 0;   // walks prune subtrees by their bounding boxes (mixed and FP64 forms)
+  int walk_boxes_ = 0;   // walks prune subtrees by their bounding boxes (mixed and FP64 forms; the h-solve in every form)
   DBuf<int> tree_work_;   // allocated on first use of the device build
   long ngb_tot_ = 0;
   bool tot_stale_ = true;   // ngb_tot_ not yet read for the current offsets (a host round trip)

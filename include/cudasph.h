@@ -207,8 +207,9 @@ long   sph_engine_get(void* e, const char* name, void* host, long max_bytes);
  * walk_boxes (1, the mixed and FP64 forms' default: the tree walks also skip
  * a child whose subtree bounding box lies beyond the range -- the same
  * neighbours in the same order, so the same results, with fewer nodes
- * visited; 0, the plain form's default: the reference's walk, whose node
- * counts it leaves in bodies_hash.key).
+ * visited; 0, the plain form's default: the list walk is the reference's,
+ * whose node counts it leaves in bodies_hash.key, and the h-solve, which leaves
+ * none, uses the boxes from 4096 particles on).
  * Mixed-form gravity measurement switches, all results within the form's
  * tolerance: grav_split_only (1: split hi/lo differences for every pair),
  * grav_unit_mass (0: the general-mass body even when every mass is equal),
