@@ -348,7 +348,7 @@ def scale_leg(cs, n, steps, seed):
            "sph_hbm": {"mean_list_length": kbar,
                        "measured": "1 step after the timed region with gravity in order, so each pass runs alone",
                        "passes": sph_bandwidth(t_in_order, s_in_order, n, kbar, walks)},
-           "gravity": {"kernel": "k_gravity_mixed_plummer", "launch_ms": g_avg * 1e3, "achieved": achieved,
+           "gravity": {"kernel": "k_gravity_mixed_pairs", "launch_ms": g_avg * 1e3, "achieved": achieved,
                        "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_TFLOPS},
            "far_field": {"value": n * steps / wall_far, "ms_per_step": wall_far / steps * 1e3,
                          "gravity_ms": t_far["gravity"][0] / max(t_far["gravity"][1], 1),
@@ -503,7 +503,7 @@ def main():
                     "measured": "2 steps after the timed region with gravity in order, so each pass runs alone",
                     "passes": sph_bandwidth(mixed["timers_in_order"][0], mixed["timers_in_order"][1], n,
                                             mixed["kbar"], mixed["walks"])},
-        "roofline": {"bound": "valu", "kernel": "k_gravity_mixed_plummer",
+        "roofline": {"bound": "valu", "kernel": "k_gravity_mixed_pairs",
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic_from_profile("k_gravity") if CONFIG == 3 else None,
                      "frac_of_measured_fma": achieved / peaks["fp32_fma_TFLOPs"],
