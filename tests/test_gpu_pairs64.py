@@ -1,6 +1,7 @@
 """FP64 gravity and its reverse pass where each pair of particles is evaluated
 once for both (csrc/pairs64.h): odd and even tile counts, a last tile with one
-particle, every part count, masses over a factor of 100."""
+particle, every part count; equal masses,
+masses over a factor of 100, and one that differs."""
 import numpy as np
 import pytest
 
@@ -12,12 +13,16 @@ pytestmark = pytest.mark.gpu
 # 8 192 is the first size, 12 287 the last with more parts; 16, 17, 18, 19, 24, 25
 # and 129 tiles
 @pytest.mark.parametrize("n", [8191, 8192, 8193, 8449, 8704, 9217, 12287, 12289, 65537])
-def test_pairs_give_the_direct_sum(cs, n):
-    print(f"fp64 pairs n={n}", flush=True)
+@pytest.mark.parametrize("masses", ["equal", "unequal", "one differs"])
+def test_pairs_give_the_direct_sum(cs, n, masses):
+    print(f"fp64 pairs n={n} {masses}", flush=True)
     p = cs.preset_params(2, n)
     pos, vel, hyd = cs.generate_ic(2, n, 3)
     rng = np.random.default_rng(n)
-    vel[:n, 3] *= 10.0 ** rng.uniform(-1, 1, n).astype(vel.dtype)
+    if masses == "unequal":
+        vel[:n, 3] *= 10.0 ** rng.uniform(-1, 1, n).astype(vel.dtype)
+    elif masses == "one differs":
+        vel[n // 3, 3] *= 3
     e = cs.Engine("fp64", p)
     e.load_ic(pos, vel, hyd)
     x, m = pos[:n, :3].astype(np.float64), vel[:n, 3].astype(np.float64)
