@@ -6,7 +6,9 @@
 // one LDS read per j per wave.  (Reading j through scalar loads instead was
 // measured ~4% slower at N = 2^20: the scalar cache misses once the j array
 // outgrows L2.)  j runs in ascending order over all records, the reference's
-// summation order.
+// summation order.  The mixed and FP64 forms have no such order to keep and take
+// each pair of particles once for both where that pays (k_gravity_mixed_pairs,
+// pairs64.h).
 //
 // Variants (template parameters):
 //   SOFT  0: M4 spline at the SPH range, half from each side (reference)
@@ -970,8 +972,8 @@ __device__ __forceinline__ void far_field(const float* __restrict__ M, float yx,
 // VGPRs next to the pairwise state: left alone the compiler takes 127
 // registers (4 wavefronts per SIMD); capped at 5 wavefronts it fits 96
 // registers without spilling (at 6 it spills 15 registers and runs 4-8 %
-// slower).  The pairwise instantiation is left unbounded (63 registers, 8
-// wavefronts).
+// slower).  The pairwise instantiation is held to 8 wavefronts (60 registers;
+// left alone it took 125, and 65 536 particles 2.2 in place of 1.9 ms).
 template <int JT, bool FAR>
 __global__ __launch_bounds__(kGravBlock) __attribute__((amdgpu_waves_per_eu(FAR ? 5 : 8)))
 void k_gravity_mixed_plummer(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ part_hi,
