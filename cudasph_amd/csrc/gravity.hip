@@ -1324,9 +1324,11 @@ __device__ __forceinline__ void rsq_spaced(float (&v)[2]) {
   v[1] = b;
 }
 
-// 4 wavefronts per SIMD (128 VGPRs; the folded sums wait in scratch between
-// sub-tiles): 5 reload in the loop (steps of 65 536 particles 1.72 against 1.68
-// ms, 80 000: 2.66 / 2.35), 3 issue worse (2^20: 235 against 229 ms).
+// 4 wavefronts per SIMD (120 VGPRs, nothing in scratch).  The two forms of r for
+// unequal masses stand in loops of their own: with the choice inside one loop
+// the kernel kept 596 bytes per lane in scratch, which this body reloaded in every
+// step (65 536 particles of unequal masses, the pass alone: 8.4 ms, 1.58 with loops
+// of their own; every ordered pair 2.24; equal masses 1.47 -> 1.42).
 constexpr int kMixTile = 512, kMixHalf = 256;
 __global__ __launch_bounds__(kMixHalf) __attribute__((amdgpu_waves_per_eu(4)))
 void k_gravity_mixed_pairs(const F4* __restrict__ hi, const F4* __restrict__ lo, F4* __restrict__ own_hi,
@@ -1478,23 +1480,8 @@ void k_gravity_mixed_pairs(const F4* __restrict__ hi, const F4* __restrict__ lo,
               }
             });
           } else {
-            sweep([&](int grp, int s) {
-              float rx[2], ry[2], rz[2], inv[2];
-              float mj;
-              if (tile_form) {
-                const F4 pj = s_rel[grp][c16 + s];
-                for (int p = 0; p < 2; ++p) {
-                  rx[p] = dx[p] - pj.x;
-                  ry[p] = dy[p] - pj.y;
-                  rz[p] = dz[p] - pj.z;
-                  inv[p] =
-                      __builtin_fmaf(rx[p], rx[p], __builtin_fmaf(ry[p], ry[p], __builtin_fmaf(rz[p], rz[p], eps2)));
-                }
-                rsq_spaced(inv);
-                mj = pj.w;
-              } else {
-                mj = split(grp * 16 + ((c16 + s) & 15), rx, ry, rz, inv);
-              }
+            const auto both = [&](const float (&rx)[2], const float (&ry)[2], const float (&rz)[2],
+                                  const float (&inv)[2], float mj) {
               for (int p = 0; p < 2; ++p) {
                 const float i2 = inv[p] * inv[p], wj = mj * inv[p], wi = pi[p].w * inv[p], sj = wj * i2, si = wi * i2;
                 a[p][0].fsub(rx[p], sj);
@@ -1506,7 +1493,27 @@ void k_gravity_mixed_pairs(const F4* __restrict__ hi, const F4* __restrict__ lo,
                 R.z = __builtin_fmaf(rz[p], si, R.z);
                 R.w -= wi;
               }
-            });
+            };
+            if (tile_form)
+              sweep([&](int grp, int s) {
+                const F4 pj = s_rel[grp][c16 + s];
+                float rx[2], ry[2], rz[2], inv[2];
+                for (int p = 0; p < 2; ++p) {
+                  rx[p] = dx[p] - pj.x;
+                  ry[p] = dy[p] - pj.y;
+                  rz[p] = dz[p] - pj.z;
+                  inv[p] =
+                      __builtin_fmaf(rx[p], rx[p], __builtin_fmaf(ry[p], ry[p], __builtin_fmaf(rz[p], rz[p], eps2)));
+                }
+                rsq_spaced(inv);
+                both(rx, ry, rz, inv, pj.w);
+              });
+            else
+              sweep([&](int grp, int s) {
+                float rx[2], ry[2], rz[2], inv[2];
+                const float mj = split(grp * 16 + ((c16 + s) & 15), rx, ry, rz, inv);
+                both(rx, ry, rz, inv, mj);
+              });
           }
         }
         if (sub & 1)
