@@ -1384,7 +1384,7 @@ void k_gravity_mixed_pairs(const F4* __restrict__ hi, const F4* __restrict__ lo,
       for (int sub = 0; sub < 4; ++sub) {
         Reaction R, total;   // of 16 records' steps, of all
         const F4 c = s_rel[4 * sub][31];
-        if (c.w >= 0.f) {
+        if (!(c.w < 0.f)) {   // (a NaN place gives a NaN radius, and its NaN must reach the sums)
           float dx[2], dy[2], dz[2], di2[2];
           for (int p = 0; p < 2; ++p) {
             dx[p] = (pi[p].x - c.x) + li[p].x;

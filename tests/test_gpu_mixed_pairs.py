@@ -37,3 +37,25 @@ def test_unequal_masses_cost_about_as_much_as_equal_ones(cs, n):
     e.close()
     print(f"  equal {equal:.3f} ms, unequal {other:.3f} ms", flush=True)
     assert other <= 2 * equal
+
+
+@pytest.mark.parametrize("masses", ["equal", "unequal"])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+# records of the 8193: the origin record of a sub-tile of 64, another one, the
+# last tile's only real record, which is its sub-tile's origin too
+@pytest.mark.parametrize("at", [32, 4128, 100, 8192])
+def test_a_lost_place_reaches_every_sum(cs, at, value, masses):
+    """One particle at NaN or infinity: no particle's acceleration stays finite,
+    as in a sum over all pairs."""
+    n = 8193
+    print(f"lost place at={at} {value} {masses}", flush=True)
+    e = cs.make_engine("mixed", 2, n, 7, ph_sort=True)
+    if masses == "unequal":
+        unequal(e, n)
+    x = e.get("pos64")
+    x[at, 0] = value
+    e.set("pos64", x)
+    e.run_pass(cs.GRAVITY)
+    a = e.get("grav")[:n, :3]
+    e.close()
+    assert not np.isfinite(a[:, 0]).any(), np.isfinite(a[:, 0]).sum()
