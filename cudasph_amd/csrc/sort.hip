@@ -104,7 +104,8 @@ void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scrat
 // counts in a table and look back over it (decoupled look-back, Merrill and
 // Garland): an entry says whether it holds the tile's own count or already
 // the sum over all tiles up to it, and a tile adds earlier ones' counts until
-// it meets a sum.  Tiles take their number from a counter as they start, so a
+// it meets a sum.  An entry is 0 until it is published, then the count + 1 (at
+// most 4097) or the sum + 4098: 32 bits hold sums up to 2^31 - 1.  Tiles take their number from a counter as they start, so a
 // tile waits only for ones that are running, and those publish before they
 // wait.  A pass uses one of two tables and clears its part of the other for
 // the next.
@@ -116,7 +117,7 @@ constexpr int kRadixBlock = 1024;
 constexpr int kRadixItems = 4;
 constexpr int kRadixTile = kRadixBlock * kRadixItems;   // records per block
 constexpr int kRadixMaxPasses = 8;
-constexpr unsigned kCountFlag = 1u << 30, kSumFlag = 2u << 30, kCountMask = kCountFlag - 1;
+constexpr unsigned kCountBase = 1, kSumBase = kRadixTile + 2;   // what an entry's count, or sum, is above
 // polls of a table entry before a tile gives up (seconds; an earlier tile
 // that never publishes can only mean that another sort uses the same scratch)
 constexpr int kRadixMaxPolls = 1 << 22;
@@ -208,7 +209,7 @@ __device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __rest
       s_cnt[w][tid] = total;
       total += c;
     }
-    __hip_atomic_store(&table[tile * 256 + tid], (tile == 0 ? kSumFlag : kCountFlag) | (unsigned)total,
+    __hip_atomic_store(&table[tile * 256 + tid], (tile == 0 ? kSumBase : kCountBase) + (unsigned)total,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     other[tile * 256 + tid] = 0;
     // exclusive sums over the digits: of the tile's counts, of all records'
@@ -243,19 +244,20 @@ __device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __rest
 #pragma unroll
       for (int k = 0; k < kAhead; ++k)
         v[k] = t - k >= 0 ? __hip_atomic_load(&table[(t - k) * 256 + tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                          : kSumFlag;
+                          : kSumBase;
       bool done = false;
 #pragma unroll
       for (int k = 0; k < kAhead; ++k) {
-        if (done || v[k] < kCountFlag) break;   // not published: read again from here
-        earlier += v[k] & kCountMask;
-        done = v[k] >= kSumFlag;
+        if (done || v[k] < kCountBase) break;   // not published: read again from here
+        earlier += v[k] - kCountBase;
+        done = v[k] >= kSumBase;
         --t;
       }
+      if (done) earlier -= kSumBase - kCountBase;
       if (done || ++polls > kRadixMaxPolls) break;
     }
     if (tile > 0)
-      __hip_atomic_store(&table[tile * 256 + tid], kSumFlag | (earlier + (unsigned)total), __ATOMIC_RELAXED,
+      __hip_atomic_store(&table[tile * 256 + tid], kSumBase + earlier + (unsigned)total, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
     s_out[tid] = smaller + (int)earlier - excl;
   }

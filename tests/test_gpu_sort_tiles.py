@@ -29,3 +29,27 @@ def test_sort_around_tiles(cs, n, bits, kind):
                                         torch.cuda.current_stream().cuda_stream) == 0
         got = data.cpu().numpy().view(np.uint32)
         assert np.array_equal(got, kv[np.argsort(keys, kind="stable")])
+
+
+def test_more_records_of_one_digit_than_2_to_the_30(cs):
+    """RadixSort takes any count up to 2^31 - 1: 2^30 + 2^20 + 3 records, all but
+    the last 1000 with the same digit."""
+    import torch
+    n, few = (1 << 30) + (1 << 20) + 3, 1000
+    print(f"sort n={n}", flush=True)
+    data = torch.empty((n, 2), dtype=torch.int32, device="cuda")
+    data[:, 0] = 5
+    data[n - few:, 0] = 3
+    torch.arange(n, dtype=torch.int32, out=data[:, 1])
+    alt = torch.zeros_like(data)
+    torch.cuda.synchronize()
+    L = cs.lib()
+    L.RadixSort.argtypes = [C.c_void_p, C.c_void_p, C.c_uint, C.c_uint]
+    L.RadixSort.restype = None
+    L.RadixSort(data.data_ptr(), alt.data_ptr(), n, 8)
+    del alt
+    torch.cuda.synchronize()
+    first = data[:few].cpu().numpy()
+    assert (first[:, 0] == 3).all() and np.array_equal(first[:, 1], np.arange(n - few, n))
+    assert bool((data[few:, 0] == 5).all())
+    assert torch.equal(data[few:, 1], torch.arange(n - few, dtype=torch.int32, device="cuda"))
