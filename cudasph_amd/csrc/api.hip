@@ -293,6 +293,18 @@ int sph_adjoint_replay(void* e, const double* x0, const double* v0, const double
   }, -1);
 }
 
+int sph_radix_sort_polls(sph_kv* pData0, sph_kv* pData1, unsigned int elements, unsigned int bits, int max_polls) {
+  return guard([&] {
+    if (max_polls < 0) throw std::invalid_argument("sph_radix_sort_polls: max_polls must not be negative");
+    DBuf<int> scratch;
+    scratch.alloc(radix_scratch_ints(elements));
+    launch_radix_sort(reinterpret_cast<KV*>(pData0), reinterpret_cast<KV*>(pData1), (long)elements, (int)bits, scratch,
+                      nullptr, max_polls);
+    CS_HIP(hipDeviceSynchronize());
+    return 0;
+  }, -1);
+}
+
 double sph_copy_calibration(long bytes) {
   return guard([&] {
     const long n = bytes / 16;

@@ -145,9 +145,11 @@ long scan_scratch_ints(long n);
 void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scratch, hipStream_t s);
 // stable LSD radix sort of KV records by key bits [0, bits); the result is
 // left in `data` (alt is scratch of the same length).  scratch holds
-// radix_scratch_ints(n) ints.
+// radix_scratch_ints(n) ints.  max_polls: a tile's looks at the table of the
+// earlier ones' counts before it counts their records itself (negative: some
+// seconds of them)
 long radix_scratch_ints(long n);
-void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s);
+void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s, int max_polls = -1);
 constexpr long radix_header_ints = 8 * 257 + 8;
 // ints of a sort's scratch to be zero before launch_axis_sorts
 long radix_clear_ints(long n);

@@ -108,7 +108,8 @@ void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scrat
 // most 4097) or the sum + 4098: 32 bits hold sums up to 2^31 - 1.  Tiles take their number from a counter as they start, so a
 // tile waits only for ones that are running, and those publish before they
 // wait.  A pass uses one of two tables and clears its part of the other for
-// the next.
+// the next.  The wait is bounded all the same: a thread that has looked often
+// enough counts the digits of the missing tile in its records.
 //
 // Bound: the records in and out (16 B a pass and record) for many records,
 // the chain of launches for few.  1 000 003 records, 4 passes: 137 us with a
@@ -118,8 +119,9 @@ constexpr int kRadixItems = 4;
 constexpr int kRadixTile = kRadixBlock * kRadixItems;   // records per block
 constexpr int kRadixMaxPasses = 8;
 constexpr unsigned kCountBase = 1, kSumBase = kRadixTile + 2;   // what an entry's count, or sum, is above
-// polls of a table entry before a tile gives up (seconds; an earlier tile
-// that never publishes can only mean that another sort uses the same scratch)
+// looks at the table before a thread counts an earlier tile's records itself
+// (seconds; an earlier tile that never publishes can only mean that another
+// sort uses the same scratch)
 constexpr int kRadixMaxPolls = 1 << 22;
 
 // scratch of one sort: digit counts of each pass, the tile counter of each
@@ -154,11 +156,30 @@ __global__ __launch_bounds__(kRadixBlock) void k_radix_count(const KV* __restric
   if (c && (int)threadIdx.x < passes * 256) atomicAdd(&scratch[threadIdx.x], c);
 }
 
+// records of digit d in the tiles 0 .. t, those of an unpublished tile counted
+// one by one (an earlier tile is full)
+template <class Rekey>
+__device__ __forceinline__ unsigned count_earlier(const KV* in, long t, int shift, int d, const unsigned* table,
+                                               Rekey rekey) {
+  unsigned sum = 0;
+  for (; t >= 0; --t) {
+    const unsigned v = __hip_atomic_load(&table[t * 256 + d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v >= kSumBase) return sum + v - kSumBase;
+    if (v >= kCountBase) {
+      sum += v - kCountBase;
+      continue;
+    }
+    for (long q = t * kRadixTile; q < (t + 1) * kRadixTile; ++q) sum += (int)((rekey(in[q]).key >> shift) & 255) == d;
+  }
+  return sum;
+}
+
 // rekey(record) may replace a record's key as it is read; out_ids, if given,
 // receives the values alone
 template <class Rekey>
 __device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __restrict__ out, int* __restrict__ out_ids,
-                                           long n, int shift, int pass, int* __restrict__ scratch, Rekey&& rekey) {
+                                           long n, int shift, int pass, int* __restrict__ scratch, int max_polls,
+                                           Rekey&& rekey) {
   __shared__ int s_cnt[kRadixBlock / 64][256];   // per wavefront and digit: count, then first place
   __shared__ KV s_rec[kRadixTile];
   __shared__ int s_local[256], s_out[256];       // a digit's first place in the tile; its run's place in `out`, less that
@@ -238,7 +259,8 @@ __device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __rest
     s_local[tid] = excl;
     unsigned earlier = 0;
     int polls = 0;
-    for (long t = tile - 1; t >= 0;) {
+    long t = tile - 1;
+    while (t >= 0) {
       constexpr int kAhead = 4;   // entries read together
       unsigned v[kAhead];
 #pragma unroll
@@ -254,8 +276,9 @@ __device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __rest
         --t;
       }
       if (done) earlier -= kSumBase - kCountBase;
-      if (done || ++polls > kRadixMaxPolls) break;
+      if (done || ++polls > max_polls) break;
     }
+    if (polls > max_polls) earlier += count_earlier(in, t, shift, tid, table, rekey);
     if (tile > 0)
       __hip_atomic_store(&table[tile * 256 + tid], kSumBase + earlier + (unsigned)total, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
@@ -278,11 +301,13 @@ __device__ __forceinline__ void radix_pass(const KV* __restrict__ in, KV* __rest
 }
 
 __global__ __launch_bounds__(kRadixBlock) void k_radix_pass(const KV* __restrict__ in, KV* __restrict__ out, long n,
-                                                             int shift, int pass, int* __restrict__ scratch) {
-  radix_pass(in, out, nullptr, n, shift, pass, scratch, [](const KV& e) { return e; });
+                                                             int shift, int pass, int* __restrict__ scratch,
+                                                             int max_polls) {
+  radix_pass(in, out, nullptr, n, shift, pass, scratch, max_polls, [](const KV& e) { return e; });
 }
 
-void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s) {
+void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStream_t s, int max_polls) {
+  if (max_polls < 0) max_polls = kRadixMaxPolls;
   if (n <= 1 || bits <= 0) return;
   const int passes = std::min(4, (bits + 7) / 8), nb = (int)radix_tiles(n);
   const long clear = radix_clear_ints(n);
@@ -293,7 +318,7 @@ void launch_radix_sort(KV* data, KV* alt, long n, int bits, int* scratch, hipStr
   KV* src = data;
   KV* dst = alt;
   for (int p = 0; p < passes; ++p) {
-    hipLaunchKernelGGL(k_radix_pass, dim3(nb), dim3(kRadixBlock), 0, s, src, dst, n, 8 * p, p, scratch);
+    hipLaunchKernelGGL(k_radix_pass, dim3(nb), dim3(kRadixBlock), 0, s, src, dst, n, 8 * p, p, scratch, max_polls);
     CS_CHECK_LAUNCH();
     std::swap(src, dst);
   }
@@ -354,7 +379,7 @@ __global__ __launch_bounds__(kRadixBlock) void k_axis_pass(const KV* __restrict_
   const int axis = blockIdx.y;
   radix_pass(in + (size_t)axis * n, out + (size_t)axis * n,
              pass == (int)sizeof(T) - 1 ? lists + axis * list_stride : nullptr, n, 8 * (pass & 3), pass,
-             scratch + axis * stride, [&](const KV& e) {
+             scratch + axis * stride, kRadixMaxPolls, [&](const KV& e) {
                if (sizeof(T) == 8 && pass == 4)
                  return KV{(uint32_t)((uint64_t)ordered_bits(coordinate(pos[e.value], axis)) >> (sizeof(T) * 4)),
                            e.value};

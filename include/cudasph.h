@@ -95,7 +95,8 @@ void RadixSort(sph_kv* pData0, sph_kv* pData1, unsigned int elements, unsigned i
  * per GPU, held until the process ends) instead of a hipMalloc per call, so
  * at most SPH_NOALLOC_SORT_MAX elements.  Enqueued on `stream` (a
  * hipStream_t; NULL is the null stream) and not waited for.  Every call on a
- * GPU uses that GPU's one array: calls that overlap on one GPU race.
+ * GPU uses that GPU's one array: calls that overlap on one GPU race, and
+ * their records then come out in no order, some of them missing, unreported.
  * Returns 0, or -1 with sph_last_error() (more than SPH_NOALLOC_SORT_MAX
  * elements, bits above 32, a null pointer, a HIP error). */
 #define SPH_NOALLOC_SORT_MAX (1 << 24)
@@ -337,6 +338,11 @@ double sph_fma_peak_form(int form);
  * wavefronts per SIMD of every CU, the second of two launches timed; variant 1
  * replaces the rsq by a multiply.  No counterpart in the reference. */
 double sph_pair_body_probe(int variant);
+/* RadixSort with the wait of a tile for the earlier ones' digit counts cut to
+ * max_polls looks at them, after which it counts their records itself (what a
+ * sort does after some seconds): the same result.  Returns 0, or -1 with
+ * sph_last_error().  No counterpart in the reference. */
+int sph_radix_sort_polls(sph_kv* pData0, sph_kv* pData1, unsigned int elements, unsigned int bits, int max_polls);
 
 #ifdef __cplusplus
 }

@@ -53,3 +53,20 @@ def test_more_records_of_one_digit_than_2_to_the_30(cs):
     assert (first[:, 0] == 3).all() and np.array_equal(first[:, 1], np.arange(n - few, n))
     assert bool((data[few:, 0] == 5).all())
     assert torch.equal(data[few:, 1], torch.arange(n - few, dtype=torch.int32, device="cuda"))
+
+
+@pytest.mark.parametrize("polls", [0, 3])
+@pytest.mark.parametrize("n,bits,distinct", [(4097, 8, 256), (100001, 32, 1 << 32), (130000, 16, 5)])
+def test_a_wait_cut_short_changes_nothing(cs, n, bits, distinct, polls):
+    """A tile that stops waiting for an earlier one counts that one's records."""
+    print(f"short waits n={n} bits={bits} polls={polls}", flush=True)
+    import torch
+    rng = np.random.default_rng(n)
+    kv = np.stack([rng.integers(0, distinct, n, dtype=np.uint64).astype(np.uint32), np.arange(n, dtype=np.uint32)], 1)
+    data = torch.from_numpy(kv.view(np.int32).copy()).cuda()
+    alt = torch.zeros_like(data)
+    torch.cuda.synchronize()
+    L = cs.lib()
+    L.sph_radix_sort_polls.argtypes = [C.c_void_p, C.c_void_p, C.c_uint, C.c_uint, C.c_int]
+    assert L.sph_radix_sort_polls(data.data_ptr(), alt.data_ptr(), n, bits, polls) == 0
+    assert np.array_equal(data.cpu().numpy().view(np.uint32), kv[np.argsort(kv[:, 0], kind="stable")])
