@@ -206,7 +206,7 @@ struct Visit {
   bool left, right, in;   // push a child; accept the node's particle
   T ds2;
   int particle;
-  float margin_l, margin_r;   // (REACH) squared distance to the split plane a push to that child crosses
+  float margin_l, margin_r;   // (REACH) distance to the split plane a push to that child crosses
 };
 
 // the tests of one node at range q.w
@@ -239,9 +239,8 @@ __device__ __forceinline__ Visit<T> visit_node(const V4<T>& q, const Tree<T>& tr
     v.left = qc - q.w < nc && bl <= r2m;
     v.right = qc + q.w > nc && (!tr.fix_phantom || c < tr.n) && br <= r2m;
     if constexpr (REACH) {
-      const T ml = fmax(qc - nc, T(0)), mr = fmax(nc - qc, T(0));
-      v.margin_l = (float)(ml * ml);
-      v.margin_r = (float)(mr * mr);
+      v.margin_l = (float)fmax(qc - nc, T(0));
+      v.margin_r = (float)fmax(nc - qc, T(0));
     }
   }
   const T dx = q.x - node.x, dy = q.y - node.y, dz = q.z - node.z;
@@ -257,10 +256,13 @@ __device__ __forceinline__ Visit<T> visit_node(const V4<T>& q, const Tree<T>& tr
 // group's LDS (nothing counted then).  n_walk grows by the nodes visited;
 // phantom gets bit 0 when the walk reads node n+1 and bit 1 when it takes it.
 // With REACH, reach_ok is cleared when some accepted record's path bound (the
-// largest squared distance to a split plane that the path's pushes crossed)
-// is not below its distance: the phantom, whose place is not its particle's;
-// a tree whose nodes do not respect its own split planes.  (A box holds its
+// largest distance to a split plane that the path's pushes crossed) is not
+// below its distance: the phantom, whose place is not its particle's; a tree
+// whose nodes do not respect its own split planes.  (A box holds its
 // subtree's particles, so the box distances on the path are below it too.)
+// The bound is squared in T, where the distance is: squares of FP64 distances
+// have no place in a float.  Squares so small that they lose digits decide
+// nothing.
 template <bool REACH, class T, class S, class Make>
 __device__ __forceinline__ int walk_pass(const Lane& g, const V4<T>& q, const Tree<T>& tr, int root, S& s,
                                          int& n_walk, int& phantom, bool& reach_ok, Make&& make) {
@@ -285,7 +287,9 @@ __device__ __forceinline__ int walk_pass(const Lane& g, const V4<T>& q, const Tr
       v = visit_node<REACH, T>(q, tr, id);
       if (id == tr.n + 1) phantom |= v.in ? 3 : 1;
       // rounding of the margins and of ds2: below 2^-18
-      if (REACH) odd = v.in && !(path <= (float)v.ds2 * 1.00001f);
+      constexpr T kTiny = sizeof(T) == 4 ? T(1e-30) : T(1e-60);
+      if (REACH)
+        odd = v.in && path > 0.f && !((T)path * (T)path <= v.ds2 * T(1.00001) && v.ds2 >= kTiny);
     }
     if (REACH && g.ballot(odd)) reach_ok = false;
     const unsigned bl = g.ballot(v.left), br = g.ballot(v.right), ba = g.ballot(v.in);

@@ -119,3 +119,34 @@ def test_whole_evaluation_refuses_lists_beyond_the_allocation(cs, form):
     with pytest.raises(RuntimeError, match="overflow"):
         e.run_pass(cs.OFFSETS)
     e.close()
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e21, 1e-21, 1e40])
+@pytest.mark.parametrize("n,off,seed", [(256, 1.0, 1), (2048, 0.5, 1), (2048, 1.0, 3), (8192, 1.0, 1)])
+def test_kept_distances_at_any_scale(cs, n, off, seed, scale):
+    """FP64 lengths whose squares are no floats.  The reference's out-of-range
+    record n+1 (at the origin) is placed beside its parent node, where some walks
+    reach it at 17/16 of their range and not at the range itself."""
+    print(f"kept distances n={n} off={off} seed={seed} scale={scale}", flush=True)
+    p = cs.preset_params(1, n)
+    assert p.fix_phantom == 0 and p.n_dev == n
+    pos, vel, hyd = cs.generate_ic(1, n, seed)
+    e = cs.Engine("fp64", p)
+    e.load_ic(pos, vel, hyd)
+    for pid in (cs.TREE, cs.SOLVE):
+        e.run_pass(pid)
+    r = e.get("pos")[:n, 3].copy()
+    d = np.random.default_rng(seed).normal(size=3)
+    pos[:n, :3] -= e.get("tree")[n // 2, :3] + off * r.mean() * d / np.linalg.norm(d)
+    pos[:n, 3] = 1.1 * r
+    pos[:n] *= scale
+    out = []
+    for cache in (0, 1):
+        e.set_scalar("solve_cache", cache)
+        e.load_ic(pos, vel, hyd)
+        for pid in (cs.TREE, cs.SOLVE):
+            e.run_pass(pid)
+        out.append((e.get("pos")[:n, 3].copy(), e.get("n_ngb")[:n].copy()))
+    e.close()
+    assert_bits(out[1][0], out[0][0], "range")
+    assert np.array_equal(out[1][1], out[0][1])
