@@ -726,11 +726,31 @@ __global__ __launch_bounds__(kBlock) void k_find_ngb_lane(const V4<T>* __restric
   count_out[i] = c;
 }
 
-// A lane walks alone from 2^19 particles on: there the walks run in many
-// rounds.  Solve / lists of the mixed form, 16 lanes against one: 262 144
-// particles 0.59 / 0.42 against 0.96 / 0.64 ms, 2^20 (turbulent sphere)
-// 3.2 / 1.56 against 2.1 / 1.2 ms.
-static bool walk_alone(int n_dev) { return n_dev >= 1 << 19; }
+// A lane walks alone where its longer chain is hidden by many rounds of
+// others: from 2^19 particles on, and for long lists earlier.  A walk of more
+// than kWalkCap records takes several passes, parts of which are walked twice:
+// the first walk of an h-solve takes 1.2 times the list, so from a target of 42
+// (lists of 59) on a growing part of them do.  Solve + lists, ms, 16 lanes / one lane:
+//   target, particles        turbulent sphere   polytropes FP64   Plummer sphere
+//   45.2 (64)   131 072       0.80 / 1.13        1.30 / 1.74       1.00 / 2.80
+//               262 144       1.51 / 1.61        2.46 / 2.66       1.80 / 4.15
+//               327 680       1.88 / 1.88        2.93 / 2.95       2.14 / 4.25
+//   50 (72)      98 304       0.81 / 1.16        1.35 / 1.83       1.10 / 2.81
+//               131 072       1.15 / 1.21        2.02 / 1.88       1.38 / 2.99
+//               262 144       2.35 / 1.68        3.73 / 2.69       2.66 / 4.11
+//   57 (82)      65 536       1.11 / 1.27        1.47 / 1.50       1.31 / 2.64
+//                98 304       1.50 / 1.25        2.14 / 1.90       1.72 / 2.81
+//   62 (89)      65 536       1.49 / 1.30        2.29 / 1.60       1.86 / 2.66
+//               262 144       6.48 / 1.91       10.5  / 2.86       7.17 / 4.37
+// so the two are even where particles * (target - 42) is about 2^20, but for the
+// Plummer sphere, whose halo keeps single lanes long.  (A solve started far
+// from its range, with some thousand records in its first walks, is not
+// foreseen by this: 3 times off at 262 144 particles, 97 / 21 ms in the sphere,
+// 168 / 277 in the Plummer sphere, once in a run.)
+static bool walk_alone(int n_dev, const WalkParams& wp) {
+  constexpr int kMin = 1 << 16, kAlways = 1 << 19;
+  return n_dev >= kAlways || (n_dev >= kMin && n_dev * ((double)wp.desired_ngb - 42.0) >= 1 << 20);
+}
 
 // threads per block of the walks: one wavefront while there are few
 // particles, so that they spread over every CU
@@ -740,7 +760,7 @@ template <class T>
 void launch_solve_range(V4<T>* pos, int* n_ngb, const KV* hash, const V4<T>* tree, int n_dev,
                         const WalkParams& wp, hipStream_t s) {
   const int bs = walk_block(n_dev);
-  if (walk_alone(n_dev)) {
+  if (walk_alone(n_dev, wp)) {
     const size_t lds = (size_t)walk_stack_depth(wp.n_nodes) * bs * sizeof(int);
     hipLaunchKernelGGL(k_solve_range_lane<T>, dim3(ceil_div(n_dev, bs)), dim3(bs), lds, s, pos, n_ngb, hash, tree,
                        n_dev, wp);
@@ -757,7 +777,7 @@ void launch_find_ngb(const V4<T>* pos, const V4<T>* tree, KV* hash, const int* o
                      int* count_out, int* list, int* flags, int n_dev, const WalkParams& wp, int clamp, int list_cap,
                      hipStream_t s) {
   const int bs = walk_block(n_dev);
-  if (walk_alone(n_dev)) {
+  if (walk_alone(n_dev, wp)) {
     const size_t lds = (size_t)walk_stack_depth(wp.n_nodes) * bs * sizeof(int);
     hipLaunchKernelGGL(k_find_ngb_lane<T>, dim3(ceil_div(n_dev, bs)), dim3(bs), lds, s, pos, tree, hash, offset,
                        cap_count, count_out, list, flags, n_dev, wp, clamp, list_cap);
