@@ -62,8 +62,9 @@ struct DBuf {
   void alloc(size_t count) {
     if (p) CS_HIP(hipFree(p));
     p = nullptr;
-    n = count;
+    n = 0;
     if (count) CS_HIP(hipMalloc(&p, count * sizeof(X)));
+    n = count;
   }
   size_t bytes() const { return n * sizeof(X); }
   operator X*() const { return p; }

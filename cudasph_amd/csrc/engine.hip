@@ -100,7 +100,7 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
   tree_.alloc(nd_ + 2);
   ties_.alloc(1);
   boxes_.alloc(2 * ((size_t)nd_ + 2));
-  if (!kF32) reserve_gpart64(gravity64_parts(nd_));
+  if (!kF32 && p.grav_mode == 1) reserve_gpart64(gravity64_parts(nd_));
   hash_.alloc(nd_);
   perm_.alloc(nd_);
   n_ngb_.alloc(nd_);
@@ -132,7 +132,7 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
     ghi_.alloc(nd_);
     glo_.alloc(nd_);
     gvel32_.alloc(nd_);
-    gpart_.alloc(mixed_part_words(nd_));
+    size_gpart();
     gmass_.alloc(2 + 2 * (size_t)ceil_div(n_, kBlock));
     // far-field records: 64-record sub-tiles, then cells of 16384, 4096, 1024, 256,
     // then the sub-tiles' 32-record halves
@@ -322,6 +322,8 @@ void Engine<T>::set_scalar(const std::string& name, double v) {
     adj_implicit_h_ = (int)v;
   } else if (name == "grav_far") {
     grav_far_ = (int)v;
+    sync();
+    size_gpart();
   } else if (name == "grav_far_ratio") {
     if (!(v >= 4)) throw std::invalid_argument("grav_far_ratio must be at least 4");
     grav_far_ratio_ = v;
@@ -712,11 +714,22 @@ void Engine<T>::reserve_gpart64(int parts) {
   if (gpart64_.n < need) gpart64_.alloc(need);
 }
 
+// The partial sums of mixed gravity: none under the spline softening, without
+// the pairs' reactions (up to 2 GiB) with the far field.  Sized before a step
+// needs it, when the engine is made and when the far field is switched.
+template <class T>
+void Engine<T>::size_gpart() {
+  if (!mixed() || p_.grav_mode != 1) return;
+  const size_t need = mixed_part_words(nd_, !grav_far_);
+  if (gpart_.n != need) gpart_.alloc(need);
+}
+
 template <class T>
 void Engine<T>::gravity_kernels(hipStream_t gs) {
   TimerScope ts(timers_, "gravity", gs);
   if constexpr (kF32) {
     if (mixed()) {
+      size_gpart();   // (in place already, unless memory ran out)
       launch_gravity_mixed(ghi_, glo_, gvel32_, (F4*)grav_.p, gpart_, gmass_, gmom_, (float)grav_far_ratio_, (float)grav_far_grade_, nd_, nd_,
                            n_, p_.grav_mode,
                            p_.grav_eps,

@@ -111,6 +111,7 @@ class Engine final : public EngineBase {
   void gravity(bool async = false);
   void gravity_join();
   void gravity_pack();
+  void size_gpart();
   void reserve_gpart64(int parts);
   void gravity_kernels(hipStream_t gs);
   void step_end(int what, double* dt_out);

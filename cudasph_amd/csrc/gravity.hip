@@ -1869,9 +1869,9 @@ int mixed_pairs_chunk(int n) {
   const size_t slot = sizeof(F4) * kMixTile * (size_t)tiles;
   return (int)std::min<size_t>(tiles / 2 + 1, std::max<size_t>(1, ((size_t)2 << 30) / slot));
 }
-size_t mixed_part_words(int n) {
+size_t mixed_part_words(int n, bool pairs) {
   const size_t items = 2 * kGravMixedParts * (size_t)n;
-  if (!mixed_pairs_fit(n)) return items;
+  if (!pairs || !mixed_pairs_fit(n)) return items;
   const size_t np = (size_t)ceil_div(n, kMixTile) * kMixTile;
   return std::max(items, (2 * kGravMixedParts + 2 + mixed_pairs_chunk(n)) * np);
 }

@@ -114,9 +114,9 @@ void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, i
 int gravity64_parts(int n_i);
 void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_j, double eps, hipStream_t s,
                               int parts = 0);
-// part: scratch of mixed_part_words(n_j) records (Plummer only): the parts' sums,
-// and where pairs are taken once running sums and a chunk of reactions (at
-// most 2 GiB); mass_range: scratch of 2 + 2 * ceil(n_real / 256) floats ({min, max}
+// part: scratch of mixed_part_words(n_j, pairs) records (Plummer only): the
+// parts' sums, and where pairs are taken once (never with the far field) running
+// sums and a chunk of reactions (at most 2 GiB); mass_range: scratch of 2 + 2 * ceil(n_real / 256) floats ({min, max}
 // of the real particles' masses, then per-block partials)
 // moments: scratch of 52 floats per 64-record j sub-tile followed by 52 per
 // cell of 16384, 4096, 1024 and 256 records and, with split_only bit 6, 52
@@ -132,7 +132,7 @@ constexpr int kGravMixedParts = 8;   // one per XCD
 constexpr int kMixedPairsMinN = 8192;   // (from 2 048 to here both are as fast)
 inline bool mixed_pairs_fit(int n) { return n >= kMixedPairsMinN; }
 int mixed_pairs_chunk(int n);
-size_t mixed_part_words(int n);   // F4s of `part`
+size_t mixed_part_words(int n, bool pairs);   // F4s of `part`
 void launch_gravity_mixed(const F4* hi, const F4* lo, const F4* gvel, F4* out, F4* part, float* mass_range,
                           float* moments, float far_ratio, float far_grade, int n_i, int n_j, int n_real,
                           int soft, float eps, int split_only, hipStream_t s, int parts = 0);
