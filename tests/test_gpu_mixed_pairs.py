@@ -59,3 +59,33 @@ def test_a_lost_place_reaches_every_sum(cs, at, value, masses):
     a = e.get("grav")[:n, :3]
     e.close()
     assert not np.isfinite(a[:, 0]).any(), np.isfinite(a[:, 0]).sum()
+
+
+# 733 and 734 tiles have 367 and 368 offsets, of which 2 GiB of reactions hold
+# 357 (from 724 tiles on there are two chunks); the even count's opposite tiles
+# meet in the second
+@pytest.mark.parametrize("masses", ["equal", "unequal"])
+@pytest.mark.parametrize("n", [733 * 512 - 100, 734 * 512 - 511])
+def test_offsets_in_two_chunks(cs, n, masses):
+    """Odd and even counts of tiles whose reactions do not fit at once: sampled
+    sums against FP64, as in test_gpu_mixed_items.py."""
+    print(f"two chunks n={n} {masses}", flush=True)
+    e = cs.make_engine("mixed", 2, n, 7, ph_sort=True)
+    tiles = -(-e.nd // 512)
+    chunk = (2 << 30) // (16 * 512 * tiles)
+    assert chunk < tiles // 2 + 1
+    if masses == "unequal":
+        unequal(e, n)
+    e.run_pass(cs.GRAVITY)
+    got = e.get("grav")[:n].astype(np.float64)
+    x = e.get("pos64")[:n, :3]
+    m = e.get("vel64")[:n, 3].astype(np.float32).astype(np.float64)
+    eps2 = float(e.params.grav_eps) ** 2
+    e.close()
+    half = tiles // 2 * 512   # (a tile at most half way round: particles on both sides of it)
+    for i in np.unique(np.r_[0, 511, 512, half - 1, half, half + 512, n - 1, np.linspace(0, n - 1, 40).astype(int)]):
+        r = x[i] - x
+        inv = 1.0 / np.sqrt((r * r).sum(1) + eps2)
+        a = -(m * inv ** 3)[:, None] * r
+        assert np.linalg.norm(got[i, :3] - a.sum(0)) <= 2.0 ** -20 * np.linalg.norm(a, axis=1).sum(), i
+        assert abs(got[i, 3] + (m * inv).sum()) <= 2.0 ** -20 * (m * inv).sum(), i

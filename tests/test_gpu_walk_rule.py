@@ -29,6 +29,30 @@ def test_ranges_and_lists_on_both_sides(cs, orc, n, target):
     e.close()
 
 
+# lists of 50 stay with 16 lanes up to 2^19 records
+@pytest.mark.parametrize("n,alone", [(524032, False), (524288, True)])
+def test_lists_on_both_sides_of_2_to_the_19(cs, n, alone):
+    """The mixed form's lists are the particles within the range, by brute force
+    over a sample."""
+    print(f"sampled lists n={n}", flush=True)
+    p = cs.preset_params(5, n)
+    p.desired_ngb = 35.3
+    p.eos_newton = 1
+    e = cs.make_engine("mixed", 5, n, 3, params=p, ph_sort=True)
+    assert (e.nd >= 1 << 19) == alone
+    for pid in (cs.TREE, cs.SOLVE, cs.OFFSETS, cs.FIND):
+        e.run_pass(pid)
+    q = e.get("pos")[:n]
+    off, cnt = e.get("ngb_offset"), e.get("ngb_count")
+    lst = e.get("ngb_list", int(off[-1]))
+    e.close()
+    for i in range(0, n, n // 37):
+        d = q[i, :3] - q[:, :3]
+        d2 = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+        want = np.nonzero(d2 < q[i, 3] * q[i, 3])[0]
+        assert np.array_equal(np.sort(lst[off[i]:off[i] + cnt[i]]), want), i
+
+
 @pytest.mark.parametrize("form", ["mixed", "fp64"])
 def test_long_lists_cost_what_they_are_longer(cs, form):
     """h-solve and lists of 262 144 particles: lists 1.37 times as long take at
