@@ -104,7 +104,6 @@ void launch_hydro(const V4<T>* pos, const V4<T>* vel, const V4<T>* hydro, const 
 constexpr int kChainsMaxN = 94208;
 constexpr int kChainsMaxNSpline = 81920;
 constexpr int kFastLaneMinN = 1 << 19;
-bool gravity_by_chains(int n_i, int soft, int sums);
 template <class T>
 void launch_gravity(const V4<T>* gpos, const V4<T>* gvel, V4<T>* out, int n_i, int n_j, int soft, T eps,
                     int exact, hipStream_t s, int sums = -1);
@@ -126,10 +125,14 @@ void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_
 // (C / 16384)^far_grade; may be null otherwise)
 // parts: the number of j-parts, 1 .. kGravMixedParts; 0 for the most.
 constexpr int kGravMixedParts = 8;   // one per XCD
-// Pairs taken once (k_gravity_mixed_pairs).  Steps, ms, every ordered pair / once:
-// 8 192 particles 0.449 / 0.407, 16 384: 0.483 / 0.469, 32 768: 0.669 / 0.630, 65 536:
-// 1.81 / 1.68, 131 072: 6.05 / 4.95, 250 007: 18.9 / 16.1, 2^20: 274 / 236.
-constexpr int kMixedPairsMinN = 8192;   // (from 2 048 to here both are as fast)
+// Pairs taken once (k_gravity_mixed_pairs).  Steps / the pass alone, ms, every
+// ordered pair against once: 8 192 particles 0.378 / 0.103 against 0.377 / 0.143,
+// 12 288: 0.425 / 0.152, 0.421 / 0.159, 14 336: 0.432 / 0.176, 0.427 / 0.161, 18 432:
+// 0.478 / 0.244, 0.468 / 0.271, 24 576: 0.522 / 0.327, 0.521 / 0.299, 32 768: 0.671,
+// 0.595, 65 536: 2.00, 1.64, 131 072: 6.17, 4.78, 250 007: 19.0, 15.7, 2^20: 272.7,
+// 231.6; unequal masses 65 536: 2.01, 1.75, 2^20: 300, 254.  (Few tiles: 16 at 8 192,
+// whose 128 blocks leave half of the CUs to the SPH passes, and idle without them.)
+constexpr int kMixedPairsMinN = 12288;
 inline bool mixed_pairs_fit(int n) { return n >= kMixedPairsMinN; }
 int mixed_pairs_chunk(int n);
 size_t mixed_part_words(int n, bool pairs);   // F4s of `part`
