@@ -446,9 +446,10 @@ def main():
              "what": "k_copy16 over 1 GiB (read + written bytes / time); k_fma_peak, 8 wavefronts per SIMD "
                      "on every CU, 2 flops per single-lane FMA: 16 chains of the accumulate form v_fmac_f32 "
                      "with vector operands (fp32_fma_TFLOPs) and 8 chains of v_fma_f32 with scalar "
-                     "coefficients; k_pair_body: the gravity kernel's expanded equal-mass pair body alone "
-                     "(11 VALU + rsq) on register-held records, 8 wavefronts per SIMD, in the 20-flop "
-                     "convention: the ceiling of that pair body"}
+                     "coefficients; k_pair_body: the expanded equal-mass body of every ordered pair alone (11 VALU "
+                     "+ rsq per interaction) on register-held records, 8 wavefronts per SIMD, in the 20-flop "
+                     "convention: what k_gravity_mixed_plummer could reach, no bound for k_gravity_mixed_pairs, "
+                     "whose body has 16 VALU + rsq for two interactions"}
     value = n * K / mixed["wall_s"]
     g_ms, g_calls = mixed["timers"].get("gravity", (float("nan"), 0))
     g_avg = g_ms / max(g_calls, 1) / 1e3
@@ -507,7 +508,6 @@ def main():
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic_from_profile("k_gravity") if CONFIG == 3 else None,
                      "frac_of_measured_fma": achieved / peaks["fp32_fma_TFLOPs"],
-                     "frac_of_pair_body": achieved / peaks["gravity_pair_body_TFLOPs"],
                      "per_launch": f"{FLOP_PER_PAIR} flop x {nd}^2 pairs",
                      "launch_ms": g_avg * 1e3},
         "far_field": None if far is None else {

@@ -102,7 +102,6 @@ Engine<T>::Engine(int form, const sph_params& p, int device) : form_(form), p_(p
   boxes_.alloc(2 * ((size_t)nd_ + 2));
   if (!kF32 && p.grav_mode == 1) reserve_gpart64(gravity64_parts(nd_));
   hash_.alloc(nd_);
-  perm_.alloc(nd_);
   n_ngb_.alloc(nd_);
   ngb_count_.alloc(nd_);
   ngb_offset_.alloc(nd_ + 1);

@@ -23,12 +23,6 @@ struct TimerScope {
   ~TimerScope() { t.end(s); }
 };
 
-inline int bits_for(long v) {
-  int b = 0;
-  while ((1L << b) <= v) ++b;
-  return b;
-}
-
 // ---------------------------------------------------------------------------
 template <class T>
 class Engine final : public EngineBase {
@@ -186,7 +180,7 @@ class Engine final : public EngineBase {
   Timers timers_;
 
   DBuf<V4<T>> pos_, vel_, hydro_, dots_, bdots_, hydro2_, grav_, tree_, gpos_, gvel_, old_vu_, tmp4_;
-  DBuf<KV> hash_, pairs_, pairs_alt_, perm_;
+  DBuf<KV> hash_, pairs_, pairs_alt_;
   DBuf<int> n_ngb_, ngb_count_, ngb_offset_, list_, owner_, tr_start_, flags_, scan_tmp_, sort_tmp_;
   DBuf<T> acc_;
   DBuf<double> dt_cur_, dt_next_, partials_, force6_, stats6_;

@@ -878,7 +878,9 @@ __global__ __launch_bounds__(kGravBlock) void k_cell_moments(const F4* __restric
 //   B_0 = M0, B_1 = tr M2 / 2, B_2 = y.M2.y / 2 - t3.y / 2 + tr Q / 8,
 //   B_3 = y.Q.y / 4 - M3.yyy / 6, B_4 = M4.yyyy / 24,
 // that is B_3 = y.(V_3 + Q.y / 4) / 3 and B_4 = y.V_4 / 4.  The kernel with the far
-// field is bound by the operations here, about two thirds of its VALU work.
+// field is bound by VALU issue, these operations about half of it: counted at
+// 2^20 particles, a wavefront takes 6 500 expansions and 84 000 pairs (polytropes:
+// 1.0e6 and 1.1e6 operations), 8 300 and 68 000 (turbulent sphere: 1.3e6, 0.9e6).
 // The moments are stored with the factors (2 k - 1)!! of g_k, so that the G_k are
 // plain powers, and every line is a chain of multiply-adds: 141 operations
 // and a v_rsq_f32 (196 term by term).
@@ -1745,10 +1747,11 @@ static int gpu_cus() {
 
 // Parts for the passes of the FP64 form: of 2 .. 8 (1 from 2^19 particles on)
 // the count whose blocks fill the CUs most evenly, the larger of equals.
-// Every block is resident at once and takes the same time, so a pass lasts as
-// long as its fullest CU.  Pairs taken once, gravity alone, 8 / 5 parts, ms:
-// 50 021 particles (98 tiles on 256 CUs) 1.59 / 1.34, 65 536 (128): 2.06 / 2.36,
-// 100 003 (196): 5.42 / 5.09, 131 072 (256): 7.9 / 8.2.
+// Where every block is resident at once (pairs: 4 blocks a CU, so tiles * parts up
+// to 1 024 on 256 CUs) and takes the same time, a pass lasts as long as its fullest
+// CU; with more blocks it is a guide only, and matters less.  Pairs taken once,
+// gravity alone, 8 / 5 parts, ms: 50 021 particles (98 tiles on 256 CUs) 1.59 / 1.34,
+// 65 536 (128): 2.06 / 2.36, 100 003 (196): 5.42 / 5.09, 131 072 (256): 7.9 / 8.2.
 int gravity64_parts(int n_i) {
   const bool pairs = pairs64_fits(n_i);
   const int blocks = pairs ? pairs64_tiles(n_i) : ceil_div(n_i, kGravBlock);
@@ -1828,7 +1831,7 @@ void launch_gravity64_plummer(const D4* gpos, D4* out, D4* part, int n_i, int n_
   }
 }
 
-bool gravity_by_chains(int n_i, int soft, int sums) {
+static bool gravity_by_chains(int n_i, int soft, int sums) {
   if (sums >= 0) return sums != 0;
   return n_i <= (soft == 1 ? kChainsMaxN : kChainsMaxNSpline);
 }

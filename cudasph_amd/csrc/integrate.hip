@@ -526,7 +526,7 @@ __global__ __launch_bounds__(kBlock) void k_fma_peak(float* __restrict__ out, in
   for (int k = 0; k < kChains; ++k) sum += x[k];
   out[(long)blockIdx.x * kBlock + threadIdx.x] = sum;
 }
-// The gravity kernel's expanded equal-mass pair body alone (11 VALU + rsq
+// k_gravity_mixed_plummer's expanded equal-mass pair body alone (11 VALU + rsq
 // per pair) on 8 records held in registers, 16 pairs per round: no LDS, no
 // memory in the loop, 8 wavefronts per SIMD.
 // The records are wave-uniform, as in the kernel; d_i moves a little each

@@ -113,7 +113,9 @@ void launch_exclusive_scan(const int* in, int* out, long n, int mode, int* scrat
 //
 // Bound: the records in and out (16 B a pass and record) for many records,
 // the chain of launches for few.  1 000 003 records, 4 passes: 137 us with a
-// histogram, a scan of 3 launches and a scatter per pass -> 51 us.
+// histogram, a scan of 3 launches and a scatter per pass -> 79 us, of which the
+// four passes take about 17 each: 245 tiles on 256 CUs are one chain of loads,
+// ranks, look-back and stores.
 constexpr int kRadixBlock = 1024;
 constexpr int kRadixItems = 4;
 constexpr int kRadixTile = kRadixBlock * kRadixItems;   // records per block

@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kLdsThreads) void k_tree_lds(const int* __restrict_
         const V4<T> q = pos[id];
         tree[t] = {q.x, q.y, q.z, node_word(T(0), id | (a << 24))};
         if (heap_order) hash[t - 1] = {(uint32_t)(t - 1), (uint32_t)id};
-        if (ties) {   // as in k_tree_split
+        if (ties) {   // as in k_tree_move
           const T cq = coord(q, a);
           if ((p > 0 && coord(pos[gl[0][s_list[a][cur[a]][i - 1]]], a) == cq) ||
               (p + 1 < subtree_size(t, n) && coord(pos[gl[0][s_list[a][cur[a]][i + 1]]], a) == cq))

@@ -415,7 +415,7 @@ struct NgbSum {
   }
 };
 
-// The evaluations of one particle's solve.  The first walks at 9/8 of its
+// The evaluations of one particle's solve.  The first walks at 17/16 of its
 // range and keeps the distances accepted there, in walk order; a later one at
 // r <= that range takes the kept distances below r.  That is the walk at r
 // if every one of them is reached by it.  A record's path bound (the
@@ -424,6 +424,7 @@ struct NgbSum {
 // when r exceeds its distance by more than the rounding of the push tests,
 // fl(qc -+ r) against nc: at most 2^-24 (|qc| + r) (2^-53 in FP64), taken 32 times over.  If
 // a distance lies closer to r than that, the evaluation walks at r instead.
+constexpr double kWide = 1.0625;
 template <class T>
 struct Solver {
   const Lane g;
@@ -433,7 +434,7 @@ struct Solver {
   T pad;               // the rounding allowance at r = 0
   int n = -1;          // records kept, -1: none
   T radius = T(0);     // ... of a walk at this range
-  bool full = false;   // the records of a walk at 9/8 of full_at outgrew the group's share
+  bool full = false;   // the records of a walk at kWide full_at outgrew the group's share
   T full_at = T(0);
   __device__ Solver(const V4<T>& q, const V4<T>* tree, const WalkParams& w, WalkLds<T, true>& lds)
       : tr(tree, w), wp(w), s(lds) {
@@ -447,7 +448,7 @@ struct Solver {
     const auto make = [](const Visit<T>& v) { return v.ds2; };
     if (wp.solve_cache && (n < 0 || r > radius) && !(full && r >= full_at)) {
       V4<T> wide = q;
-      wide.w = r * T(1.0625);
+      wide.w = r * T(kWide);
       bool ok = true;
       n = walk_pass<true, T>(g, wide, tr, 1, s, nw, ph, ok, make);
       radius = wide.w;
