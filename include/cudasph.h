@@ -219,9 +219,10 @@ long   sph_engine_get(void* e, const char* name, void* host, long max_bytes);
  * sums' grouping follows it; also the FP64 form's, by default the count of up
  * to 8 whose blocks fill the GPU most evenly;
  * read-only grav_parts_auto: the count the default takes at this size).
- * solve_cache (below 2^19 particles the h-solve keeps the distances of its
- * first walk for its later ranges: 1 and -1, the default, on, 0 off; the same
- * bits either way).
+ * solve_cache (where 16 lanes share a particle's walk -- below 2^19 particles,
+ * with long lists below 2^16 -- the h-solve keeps the distances of its first
+ * walk for its later ranges: 1 and -1, the default, on, 0 off; the same bits
+ * either way).
  * Plain-form gravity, the same bits either way: grav_sums (1 or 2: each
  * particle's four sums in four wavefronts, 0: in one lane; -1, the default:
  * four wavefronts up to 94 208 particles, 81 920 with the spline softening).
